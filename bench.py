@@ -31,7 +31,7 @@ configurations.
 
 `--workload flash_c3` measures the exact causal softmax baseline (triton_flash_causal_attention) on the
 default workload's inputs (1 x 32 heads, N = 65536, d = dv = 64, scale 1/8, fp32): value =
-head-tokens/s, roofline of the flash kernel against the fp32 MFMA peak (algorithmic (d + dv) N (N + 1)
+head-tokens/s, roofline of the flash kernel against a sixth of the bf16 MFMA peak (algorithmic (d + dv) N (N + 1)
 flop per head); CPU baseline = torch's fp32 softmax attention on the host over a bounded row sample.
 """
 
@@ -520,7 +520,8 @@ def run_flash(args) -> int:
     flops = float(d + dv) * n * (n + 1) * bh  # QK^T and PV over the n (n + 1) / 2 causal pairs
     achieved = flops / (k_ms * 1e-3) / 1e12
     value = bh * n / (ms_step * 1e-3)
-    peak = MFMA_FP32_PEAK_TFLOPS if args.flash_dtype == "fp32" else MFMA_BF16_PEAK_TFLOPS
+    # fp32 operands: six bf16 products per product
+    peak = MFMA_BF16_PEAK_TFLOPS / 6 if args.flash_dtype == "fp32" else MFMA_BF16_PEAK_TFLOPS
     line = {
         "metric": "head-tokens/sec, exact causal softmax attention, N=64K d=64; % of MFMA roofline",
         "value": value,
@@ -536,8 +537,9 @@ def run_flash(args) -> int:
         "data": "synthetic",
         "config": w,
         "roofline": {
-            "kernel": ("flash_attn_kernel (online-softmax exact attention, fp32 matrix cores)" if args.flash_dtype == "fp32"
-                       else "flash_attn16_kernel (online-softmax exact attention, 16-bit matrix cores: one product "
+            "kernel": ("flash_attn_kernel (online-softmax exact attention, fp32 operands as three bf16 planes: six "
+                       "products)" if args.flash_dtype == "fp32"
+                       else "flash_attn_kernel (online-softmax exact attention, 16-bit matrix cores: one product "
                             "for QK^T, two (P as hi + lo) for PV)"),
             "bound": "mfma",
             "achieved": achieved,

@@ -400,10 +400,20 @@ int sta_block_attention(const void* q, const void* k, const void* v, int dtype, 
  * :580-637):  out_i = sum_{j<=i} exp(s q_i.k_j - m_i) v_j / max(sum_{j<=i} exp(s q_i.k_j - m_i), 1e-20).
  *   q, k rows are ld_qk elements apart (a multiple of 4, >= d; columns [d, ld_qk) are ignored), v rows
  *   ld_v (a multiple of 4, >= dv); q, k, v 16-byte aligned.  out [BH][N][Dv] dense, dtype out_dtype.
- *   d <= 128, dv <= 256.  fp32 accumulation; products of the inputs are exact (fp32 matrix cores).
+ *   d <= 128, dv <= 256.  fp32 accumulation; 16-bit inputs' products are exact, fp32 operands are carried
+ *   as three bf16 planes (each product within 2^-23 of its exact value).
  */
 int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, void* stream);
+
+/*
+ * Exact causal attention with the article's unnormalised weights (compressor "none",
+ * fast_article_attention.py:437-464, :596-598: the Taylor part and the residual over every earlier key add up
+ * to exp):  out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum_{j<=i} exp(s q_i.k_j), eps).
+ * Arguments as sta_flash_attention; the weights keep fp32 accuracy for every input type.
+ */
+int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                        int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream);
 
 /* Rows per block-attention tile and the moment chunk the library uses for a head dimension D (the
  * chunk argument of sta_block_attention is that chunk for sta_moments' partials, the query block for

@@ -154,6 +154,7 @@ def _unit_width(width: int, element_size: int) -> int:
     return -(-width // per_unit) * per_unit
 
 
+FLASH_D = 128  # key dimensions of the pair kernel (sta_flash_attention, sta_exact_attention)
 STAGED_D = 128  # key dimensions the moment kernels stage whole; wider keys go through dimension windows
 MAX_D_HIGH_DEGREE = 64  # degree 5 .. 8
 
@@ -318,6 +319,14 @@ def prefill(
     if plan.call_sizes and max(plan.call_sizes) > lim["max_compress_in"]:
         raise ValueError(f"block_size {block} needs compress calls on {max(plan.call_sizes)} items; "
                          f"the HIP compressor handles at most {lim['max_compress_in']}")
+
+    # no coreset item takes part (compressor "none", or a sequence inside its first block): the Taylor part
+    # and the residual add up to exp, summed over the pairs in one launch.  Keys wider than the pair
+    # kernel's rows, and callers that choose a moment kernel or its products, keep the moment scan.
+    no_items = semantics == "exact" or (semantics == "flat" and n <= block) or (semantics == "levels" and n < block)
+    if no_items and d <= FLASH_D and products is None and residual_products is None and moment_kernel is None:
+        return PrefillResult(_pairs(q3, k3, v3, scale, eps, out_dtype, timer), None, None, plan,
+                             _plan.num_features(d, degree), 0)
 
     # the moment kernel reads rows in 16-byte units: q/k padded with zero dimensions to a whole unit
     # (zero dimensions only add zero-valued features), v to whole 32-column groups; keys wider than the
@@ -560,21 +569,31 @@ def flash(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, *, scale: float,
         _native.require_device(t)
     if not (q3.dtype == k3.dtype == v3.dtype) or q3.dtype not in _native.DTYPE_CODES:
         raise ValueError("q, k, v must share one of the dtypes float32, bfloat16, float16")
+    odt = out_dtype if out_dtype in _native.DTYPE_CODES else torch.float32
+    if q3.shape[0] == 0 or q3.shape[1] == 0:
+        return torch.empty((*q3.shape[:2], v3.shape[-1]), device=q3.device, dtype=out_dtype)
+    out = _pairs(q3, k3, v3, scale, None, odt, timer)
+    return out if odt == out_dtype else out.to(out_dtype)
+
+
+def _pairs(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, scale: float, eps: Optional[float],
+           out_dtype: torch.dtype, timer: Optional[KernelTimer]) -> torch.Tensor:
+    """Launch of the pair kernel: sta_flash_attention (eps None), or sta_exact_attention with its smallest
+    denominator eps."""
     bh, n, d = q3.shape
     dv = v3.shape[-1]
-    odt = out_dtype if out_dtype in _native.DTYPE_CODES else torch.float32
-    out = torch.empty((bh, n, dv), device=q3.device, dtype=odt)
-    if bh == 0 or n == 0:
-        return out.to(out_dtype)
+    out = torch.empty((bh, n, dv), device=q3.device, dtype=out_dtype)
     dq, dvp = -(-d // 4) * 4, -(-dv // 4) * 4
     mq, mk, mv = _padded_rows(q3, dq), _padded_rows(k3, dq), _padded_rows(v3, dvp)
     lib = _native.lib()
+    name = "flash" if eps is None else "exact_attention"
+    fn = lib.sta_flash_attention if eps is None else lib.sta_exact_attention
+    args = (float(scale),) if eps is None else (float(scale), float(eps))
 
     def launch():
-        st = lib.sta_flash_attention(mq.data_ptr(), mk.data_ptr(), mv.data_ptr(), _native.DTYPE_CODES[q3.dtype],
-                                     bh, n, d, dv, dq, dvp, float(scale), out.data_ptr(), _native.DTYPE_CODES[odt],
-                                     _native.stream_handle(q3.device))
-        _native.check(st, "sta_flash_attention")
+        st = fn(mq.data_ptr(), mk.data_ptr(), mv.data_ptr(), _native.DTYPE_CODES[q3.dtype], bh, n, d, dv, dq, dvp,
+                *args, out.data_ptr(), _native.DTYPE_CODES[out_dtype], _native.stream_handle(q3.device))
+        _native.check(st, "sta_" + ("flash_attention" if eps is None else name))
 
-    _run(timer, "flash", launch)
-    return out if odt == out_dtype else out.to(out_dtype)
+    _run(timer, name, launch)
+    return out

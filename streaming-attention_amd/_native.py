@@ -91,6 +91,9 @@ _SIGNATURES = {
     "sta_flash_attention": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _c_p, _i32, _c_p],
     ),
+    "sta_exact_attention": (
+        _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _c_p, _i32, _c_p],
+    ),
     "sta_moment_accumulate_block": (
         _i32,
         [_c_p, _c_p, _i32, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _c_p, _c_p, _c_p, _i32, _c_p,

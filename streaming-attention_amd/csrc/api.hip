@@ -92,13 +92,39 @@ int dispatch_dvt(const sta::BlockArgs& a, int64_t bh, hipStream_t s) {
 }
 
 template <int DP, int ES>
-int dispatch_flash_dvt(const sta::FlashArgs& a, int64_t bh, hipStream_t s) {
-  if (a.dv <= 16) return launch_flash<DP, 1, ES>(a, bh, s);
-  if (a.dv <= 32) return launch_flash<DP, 2, ES>(a, bh, s);
-  if (a.dv <= 64) return launch_flash<DP, 4, ES>(a, bh, s);
-  if (a.dv <= 128) return launch_flash<DP, 8, ES>(a, bh, s);
-  if (a.dv <= 256) return launch_flash<DP, 16, ES>(a, bh, s);
+int dispatch_flash_dvt(const sta::FlashArgs& a, int weight, int64_t bh, hipStream_t s) {
+  if (a.dv <= 16) return launch_flash<DP, 1, ES>(a, weight, bh, s);
+  if (a.dv <= 32) return launch_flash<DP, 2, ES>(a, weight, bh, s);
+  if (a.dv <= 64) return launch_flash<DP, 4, ES>(a, weight, bh, s);
+  if (a.dv <= 128) return launch_flash<DP, 8, ES>(a, weight, bh, s);
+  if (a.dv <= 256) return launch_flash<DP, 16, ES>(a, weight, bh, s);
   return STA_ERR_UNSUPPORTED;
+}
+
+// Argument checks and launch shared by sta_flash_attention and sta_exact_attention.
+int flash_launch(int weight, const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                 int dv, int ld_qk, int ld_v, float scale, float floor, void* out, int out_dtype, void* stream) {
+  if (!q || !k || !v || !out) return STA_ERR_ARG;
+  if (!dtype_ok(dtype) || !dtype_ok(out_dtype)) return STA_ERR_DTYPE;
+  if (bh <= 0 || n <= 0 || d <= 0 || dv <= 0) return STA_ERR_SHAPE;
+  if (d > kMaxFlashD || dv > kMaxDv) return STA_ERR_UNSUPPORTED;
+  if (ld_qk < d || ld_qk % 4 != 0 || ld_v < dv || ld_v % 4 != 0) return STA_ERR_ARG;
+  if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u) != 0)
+    return STA_ERR_ARG;
+  if (n >= (int64_t(1) << 31) - 128) return STA_ERR_UNSUPPORTED;
+  sta::FlashArgs a;
+  a.q = q; a.k = k; a.v = v; a.dtype = dtype; a.n = n; a.d = d; a.dv = dv; a.ldqk = ld_qk; a.ldv = ld_v;
+  a.scale2 = scale * 1.4426950408889634f;
+  a.n_tiles = static_cast<int>((n + sta::FLASH_ROWS - 1) / sta::FLASH_ROWS);
+  a.bh = bh; a.floor = floor;
+  a.out = out; a.out_dtype = out_dtype;
+  a.vec_out = (out_dtype == STA_F32 && dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) ? 1 : 0;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool f32 = dtype == STA_F32;
+  if (d <= 16) return f32 ? dispatch_flash_dvt<16, 4>(a, weight, bh, s) : dispatch_flash_dvt<16, 2>(a, weight, bh, s);
+  if (d <= 32) return f32 ? dispatch_flash_dvt<32, 4>(a, weight, bh, s) : dispatch_flash_dvt<32, 2>(a, weight, bh, s);
+  if (d <= 64) return f32 ? dispatch_flash_dvt<64, 4>(a, weight, bh, s) : dispatch_flash_dvt<64, 2>(a, weight, bh, s);
+  return f32 ? dispatch_flash_dvt<128, 4>(a, weight, bh, s) : dispatch_flash_dvt<128, 2>(a, weight, bh, s);
 }
 
 // Exclusive scan over the segments of each (head, feature split, column group): seg_state[p] <- sum of
@@ -150,27 +176,13 @@ int sta_limits(int* max_d, int* max_dv, int* max_degree, int* max_compress_in) {
 
 int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, void* stream) {
-  if (!q || !k || !v || !out) return STA_ERR_ARG;
-  if (!dtype_ok(dtype) || !dtype_ok(out_dtype)) return STA_ERR_DTYPE;
-  if (bh <= 0 || n <= 0 || d <= 0 || dv <= 0) return STA_ERR_SHAPE;
-  if (d > kMaxFlashD || dv > kMaxDv) return STA_ERR_UNSUPPORTED;
-  if (ld_qk < d || ld_qk % 4 != 0 || ld_v < dv || ld_v % 4 != 0) return STA_ERR_ARG;
-  if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u) != 0)
-    return STA_ERR_ARG;
-  if (n >= (int64_t(1) << 31) - 128) return STA_ERR_UNSUPPORTED;
-  constexpr int kFlashRows = 128;  // 64 RS query rows per workgroup, RS = 2
-  sta::FlashArgs a;
-  a.q = q; a.k = k; a.v = v; a.dtype = dtype; a.n = n; a.d = d; a.dv = dv; a.ldqk = ld_qk; a.ldv = ld_v;
-  a.scale2 = scale * 1.4426950408889634f;
-  a.n_tiles = static_cast<int>((n + kFlashRows - 1) / kFlashRows);
-  a.out = out; a.out_dtype = out_dtype;
-  a.vec_out = (out_dtype == STA_F32 && dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) ? 1 : 0;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool f32 = dtype == STA_F32;
-  if (d <= 16) return f32 ? dispatch_flash_dvt<16, 4>(a, bh, s) : dispatch_flash_dvt<16, 2>(a, bh, s);
-  if (d <= 32) return f32 ? dispatch_flash_dvt<32, 4>(a, bh, s) : dispatch_flash_dvt<32, 2>(a, bh, s);
-  if (d <= 64) return f32 ? dispatch_flash_dvt<64, 4>(a, bh, s) : dispatch_flash_dvt<64, 2>(a, bh, s);
-  return f32 ? dispatch_flash_dvt<128, 4>(a, bh, s) : dispatch_flash_dvt<128, 2>(a, bh, s);
+  return flash_launch(sta::FLASH_SOFTMAX, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, 1e-20f, out, out_dtype,
+                      stream);
+}
+
+int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                        int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream) {
+  return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, stream);
 }
 
 int sta_tile_rows(void) { return kTileRows; }

@@ -130,8 +130,9 @@ inline bool accumulate_block_ok(int nt, int nx, int ct) {
 // padded key width DP, value-column tile count DVT and element size ES.
 template <int DP, int DVT, int ES>
 int launch_block(const sta::BlockArgs& a, int64_t bh, hipStream_t s);
-// launch_flash.hip, one object per (DP, DVT, ES): exact causal softmax attention (flash_attn_kernel).
+// launch_flash.hip, one object per (DP, DVT, ES): causal attention over pairs (flash_attn_kernel); weight: a
+// sta::FlashWeight.
 template <int DP, int DVT, int ES>
-int launch_flash(const sta::FlashArgs& a, int64_t bh, hipStream_t s);
+int launch_flash(const sta::FlashArgs& a, int weight, int64_t bh, hipStream_t s);
 
 }  // namespace sta_api

@@ -1,24 +1,42 @@
-// Exact causal softmax attention, the FlashAttention-style baseline of the reference's GPU module
-// (_flash_causal_kernel, triton_article_attention.py:372-435; triton_flash_causal_attention :580-637):
-//   out_i = sum_{j<=i} exp(s q_i.k_j - m_i) v_j / max(sum_{j<=i} exp(s q_i.k_j - m_i), 1e-20)
-// with m_i the running row maximum (online softmax) and fp32 accumulation; no N x N score matrix.
+// Causal attention over pairs of contiguous rows, without coreset items: one kernel, three weights of a
+// pair (query row i, key j):
+//   FLASH_SOFTMAX  exact causal softmax attention, the FlashAttention-style baseline of the reference's GPU
+//                  module (_flash_causal_kernel, triton_article_attention.py:372-435;
+//                  triton_flash_causal_attention :580-637):
+//                  out_i = sum_{j<=i} exp(s q_i.k_j - m_i) v_j / max(sum_{j<=i} exp(s q_i.k_j - m_i), 1e-20),
+//                  m_i a running row maximum (online softmax)
+//   FLASH_EXP      compressor "none" (fast_article_attention.py:437-464, :596-598), where the Taylor part and the
+//                  residual add up to exp itself: out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum, eps)
+// fp32 accumulation, no N x N score matrix.
 //
-// Matrix-core layout (as in block_attn_kernel): X^T = K Q^T with A = key rows staged in LDS and B = the
-// wave's query rows in registers, pre-multiplied by s log2(e) so the logits come out in base 2; the
-// probabilities P^T stay in the accumulator layout and are the B operand of num^T += V^T P^T.  A lane
-// holds one query row (li) and, per 16-key subtile, four keys 4 lg + r; its accumulators hold value
-// columns 16 ct + 4 lg + r of the same row.  So the batch maximum of a row needs two cross-lane steps
-// (lanes li, li + 16, li + 32, li + 48) and the rescale exp2(m_old - m_new) applies to the lane's own
-// accumulators.
+// Matrix-core layout (v_mfma_f32_16x16x32): X^T = K Q^T with A = key rows staged in LDS and B = the wave's
+// query rows in registers; the weights P^T stay in the accumulator layout and are the B operand of
+// num^T += V^T P^T.  A lane holds one query row (li) and, per 16-key subtile, four keys 4 lg + r; its
+// accumulators hold value columns 16 ct + 4 lg + r of the same row.  k-step m of lane group lg covers
+// dimensions 32 m + 8 lg + j; the V^T rows hold each pair of 16-key subtiles in contraction order
+// (flash_key_pos), so every operand is one 16-byte LDS read.
 //
-// Products for fp32 inputs are fp32 matrix-core ops: exact products of the inputs (the reference's tf32
-// dots round fp32 operands to 10 mantissa bits); 16-bit inputs use the 16-bit matrix cores
-// (flash_attn16_kernel below).
+// Products.  gfx950's 16-bit matrix cores run 16x the fp32 rate, so fp32 operands are carried as three bf16
+// planes, x = h + m + l (8 bits each, together the 24 of fp32), and a product as the six largest plane
+// products (hh, hm, mh, mm, hl, lh): the three left out are at most 2^-23 |x x'| together, and in the sums
+// their signs are random (measured against 64 bits the results are closer than with fp32 matrix
+// instructions, 4.4e-7 against 5.1e-7 at 8191 keys).  2500 / 6 = 417 TF/s against their 157 TF/s.
+// 16-bit inputs are taken as they are (exact products, fp32 sums); their fp32 weights are carried as
+// 16-bit planes: hi + lo for the softmax (within 2^-16 P for bf16, 2^-20 P for fp16), three bf16 planes for
+// FLASH_EXP, whose fp16 values are two bf16 planes (exact: 11 bits).
+//
+// What bounds it: fp32 rows the six products (two thirds of the time at d = dv = 64), 16-bit rows the VALU
+// work of a pair (exponential, maximum, planes: 6 instructions).  1 x 8 heads x 8191 fp32, d = dv = 64: 397 us
+// = 174 TF/s (fp32 matrix instructions, unbalanced tiles: 857 us); 2 x 16 x 8192 bf16: 479 us = 579 TF/s
+// (710 us with a rescale and 12 more VALU instructions a pair); FLASH_EXP 4 x 8 x 2048 fp32: 102 us (513 us as
+// moment scan + residual kernel in fp32 products).
 #include <type_traits>
 
 #include "common.hpp"
 
 namespace sta {
+
+enum FlashWeight : int { FLASH_SOFTMAX = 0, FLASH_EXP = 1 };
 
 struct FlashArgs {
   const void* q;
@@ -31,263 +49,50 @@ struct FlashArgs {
   int ldqk;      // row stride (elements) of q and k: a multiple of 4, >= d (columns >= d are ignored)
   int ldv;       // row stride of v: a multiple of 4, >= dv
   float scale2;  // softmax scale times log2(e)
-  int n_tiles;   // ceil(n / (64 RS))
+  int n_tiles;   // ceil(n / FLASH_ROWS)
+  int64_t bh;
+  float floor;   // smallest denominator
   void* out;     // [BH][n][dv], dense
   int out_dtype;
   int vec_out;  // fp32 output, dv % 4 == 0 and 16-byte aligned: 16-byte stores
 };
 
-// keys per LDS stage, per-thread staging units of keys and values, and waves per SIMD (the per-wave
-// register arrays: queries RS DP/4, accumulators RS DVT 4, logits RS KB/16 4, staging 4 (KPT + VPT))
-__host__ __device__ constexpr int flash_kb(int dp, int dvt) { return (dp + dvt * 16 > 192) ? 32 : 64; }
-__host__ __device__ constexpr int flash_kpt(int dp, int dvt) { return (flash_kb(dp, dvt) * dp / 4 + 255) / 256; }
-__host__ __device__ constexpr int flash_vpt(int dp, int dvt) { return (flash_kb(dp, dvt) * dvt * 4 + 255) / 256; }
-__host__ __device__ constexpr int flash_occupancy(int dp, int dvt, int rs) {
-  return (rs * dp / 4 + rs * dvt * 4 + rs * (flash_kb(dp, dvt) / 16) * 4 +
-          4 * (flash_kpt(dp, dvt) + flash_vpt(dp, dvt))) <= 160
-             ? 2
-             : 1;
-}
+constexpr int FLASH_ROWS = 128;  // query rows of a workgroup: 4 waves x 2 strips of 16
 
-// Elements of a 4-element unit starting at column c that lie in [0, width), the rest zero (a select,
-// so padding that holds non-finite bits cannot leak in).
-__device__ __forceinline__ floatx4 unit_mask(floatx4 f, bool ok, int c, int width) {
-  floatx4 r;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = (ok && c + e < width) ? f[e] : 0.f;
-  return r;
-}
-
-// One workgroup per (head, tile of 64 RS query rows), longest tiles (highest rows) first; wave w owns
-// RS strips of 16 rows.  Keys [0, last row of the tile] are staged KB at a time (K row-major, V
-// transposed), the next batch's rows loaded into registers while the current one computes.  A wave
-// skips batches that lie wholly after its rows and applies the causal mask only on batches that
-// straddle them.
-template <int DP, int DVT, int RS, int ES>
-__global__ __launch_bounds__(256, flash_occupancy(DP, DVT, RS)) void flash_attn_kernel(const FlashArgs a) {
-  constexpr int KB = flash_kb(DP, DVT);
-  constexpr int NSUB = KB / 16;
-  constexpr int LDK = DP + 4;  // = 4 (mod 64) for the 16-byte key reads
-  constexpr int DV = DVT * 16;
-  constexpr int LDVT = KB + 4;
-  constexpr int DQ = DP / 4;  // k-steps of X = K Q^T, dimensions per lane group
-  constexpr int TM = 64 * RS;
-  __shared__ float Kst[KB * LDK];
-  __shared__ float Vt[DV * LDVT];
-
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t bh = wg / a.n_tiles;
-  const int t = a.n_tiles - 1 - (wg - static_cast<int>(bh) * a.n_tiles);
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, lg = lane >> 4;
-  const int n = static_cast<int>(a.n);
-  const int r0 = t * TM;
-  const int64_t qkbase = bh * a.n * a.ldqk;
-  const int64_t vbase = bh * a.n * a.ldv;
-
-  int myrow[RS];
-  bool rvalid[RS];
-  float qB[RS][DQ];
-#pragma unroll
-  for (int rs = 0; rs < RS; ++rs) {
-    myrow[rs] = r0 + (wave * RS + rs) * 16 + li;
-    rvalid[rs] = myrow[rs] < n;
-    const int64_t qoff = qkbase + static_cast<int64_t>(rvalid[rs] ? myrow[rs] : 0) * a.ldqk;
-#pragma unroll
-    for (int m = 0; m < DQ / 4; ++m) {
-      const int col = DQ * lg + 4 * m;
-      const floatx4 raw = unit_to_f4<ES>(load_unit<ES>(a.q, qoff + min(col, a.ldqk - 4)), a.dtype, a.scale2);
-      const floatx4 v4 = unit_mask(raw, rvalid[rs], col, a.d);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qB[rs][4 * m + e] = v4[e];
-    }
-  }
-  const int wrow_lo = r0 + wave * RS * 16, wrow_hi = wrow_lo + RS * 16 - 1;  // this wave's rows
-
-  floatx4 num[RS][DVT];
-  float den[RS], mrow[RS];
-#pragma unroll
-  for (int rs = 0; rs < RS; ++rs) {
-    den[rs] = 0.f;
-    mrow[rs] = -1e30f;  // finite: exp2(m_old - m_new) is then 0 or 1, never a NaN
-#pragma unroll
-    for (int ct = 0; ct < DVT; ++ct) num[rs][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // one staged batch of keys [off, off + KB); DIAG: some key of it follows some row of this wave
-  auto process = [&](auto diag_tag, int off) {
-    constexpr bool DIAG = decltype(diag_tag)::value;
-    floatx4 X[NSUB][RS];
-#pragma unroll
-    for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-      for (int rs = 0; rs < RS; ++rs) X[kt][rs] = floatx4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int m = 0; m < DQ / 4; ++m) {
-      floatx4 kv[NSUB];
-#pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt)
-        kv[kt] = *reinterpret_cast<const floatx4*>(Kst + (16 * kt + li) * LDK + DQ * lg + 4 * m);
-#pragma unroll
-      for (int e = 0; e < 4; ++e)
-#pragma unroll
-        for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-          for (int rs = 0; rs < RS; ++rs) X[kt][rs] = mfma4(kv[kt][e], qB[rs][4 * m + e], X[kt][rs]);
-    }
-#pragma unroll
-    for (int rs = 0; rs < RS; ++rs) {
-      float mx = -__builtin_huge_valf();
-#pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          if constexpr (DIAG) {
-            if (off + 16 * kt + 4 * lg + r > myrow[rs]) X[kt][rs][r] = -__builtin_huge_valf();
-          }
-          mx = fmaxf(mx, X[kt][rs][r]);
-        }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mnew = fmaxf(mrow[rs], mx);
-      const float alpha = __builtin_amdgcn_exp2f(mrow[rs] - mnew);
-      mrow[rs] = mnew;
-      den[rs] *= alpha;
-#pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) num[rs][ct] *= alpha;
-#pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(X[kt][rs][r] - mnew);
-          X[kt][rs][r] = p;
-          den[rs] += p;
-        }
-    }
-#pragma unroll
-    for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) {
-        const floatx4 va = *reinterpret_cast<const floatx4*>(Vt + (16 * ct + li) * LDVT + 16 * kt + 4 * lg);
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-          for (int rs = 0; rs < RS; ++rs) num[rs][ct] = mfma4(va[s], X[kt][rs][s], num[rs][ct]);
-      }
-  };
-
-  const int row_hi = (r0 + TM < n ? r0 + TM : n) - 1;  // r0 < n: t < ceil(n / TM)
-  const int kend = row_hi + 1;
-  const int nb = (kend + KB - 1) / KB;
-
-  // staging registers: this thread's 4-element units of the next batch's key and value rows, raw
-  constexpr int KU = DP / 4, VU = DV / 4;
-  constexpr int KPT = flash_kpt(DP, DVT), VPT = flash_vpt(DP, DVT);
-  uint4 pk[KPT], pv[VPT];
-  uint32_t pk_ok = 0, pv_ok = 0;
-  auto prefetch = [&](int off) {
-    pk_ok = pv_ok = 0;
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      const int r = e / KU, u = e - r * KU;
-      const bool ok = e < KB * KU && off + r < kend && 4 * u < a.d;
-      pk_ok |= ok ? (1u << i) : 0u;
-      const int src = ok ? off + r : 0;
-      pk[i] = load_unit<ES>(a.k, qkbase + static_cast<int64_t>(src) * a.ldqk + min(4 * u, a.ldqk - 4));
-    }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const int e = tid + 256 * i;
-      const int r = e % KB, u = e / KB;  // key-fast: conflict-light transposed writes
-      const bool ok = e < KB * VU && off + r < kend && 4 * u < a.dv;
-      pv_ok |= ok ? (1u << i) : 0u;
-      const int src = ok ? off + r : 0;
-      pv[i] = load_unit<ES>(a.v, vbase + static_cast<int64_t>(src) * a.ldv + min(4 * u, a.ldv - 4));
-    }
-  };
-  auto commit = [&]() {
-#pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * KU) {
-        const int r = e / KU, u = e - r * KU;
-        *reinterpret_cast<floatx4*>(Kst + r * LDK + 4 * u) =
-            unit_mask(unit_to_f4<ES>(pk[i], a.dtype, 1.f), (pk_ok >> i) & 1u, 4 * u, a.d);
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * VU) {
-        const int r = e % KB, u = e / KB;
-        const floatx4 f = unit_mask(unit_to_f4<ES>(pv[i], a.dtype, 1.f), (pv_ok >> i) & 1u, 4 * u, a.dv);
-#pragma unroll
-        for (int m = 0; m < 4; ++m) Vt[(4 * u + m) * LDVT + r] = f[m];
-      }
-    }
-  };
-
-  prefetch(0);
-  for (int b = 0; b < nb; ++b) {
-    __syncthreads();  // every wave is done with the staging buffers of the previous batch
-    commit();
-    __syncthreads();  // staged batch visible
-    if (b + 1 < nb) prefetch((b + 1) * KB);
-    const int off = b * KB;
-    if (off <= wrow_hi) {
-      if (off + KB - 1 > wrow_lo)
-        process(std::true_type{}, off);
-      else
-        process(std::false_type{}, off);
-    }
-  }
-
-  // ---- epilogue: row sums over the four lane groups, normalise, store ----
-#pragma unroll
-  for (int rs = 0; rs < RS; ++rs) {
-    float dsum = den[rs];
-    dsum += __shfl_xor(dsum, 16);
-    dsum += __shfl_xor(dsum, 32);
-    if (!rvalid[rs]) continue;
-    const float dn = fmaxf(dsum, 1e-20f);
-    const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
-#pragma unroll
-    for (int ct = 0; ct < DVT; ++ct) {
-      const int c0 = 16 * ct + 4 * lg;
-      if (c0 >= a.dv) continue;
-      floatx4 o;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = num[rs][ct][r] / dn;
-      if (a.vec_out) {
-        *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + obase + c0) = o;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (c0 + r < a.dv) store_elem(a.out, obase + c0 + r, a.out_dtype, o[r]);
-      }
-    }
-  }
-}
-
-// ------------------------------------------------------------------------------------------------
-// 16-bit inputs (bf16 / fp16): the matrix cores take the inputs as they are.  X^T = K Q^T with
-// v_mfma_f32_16x16x32_{bf16,f16} is exact (16-bit products, fp32 sums) and scaled to base-2 logits
-// afterwards; num^T += V^T P^T takes the fp32 probabilities as 16-bit hi + lo (P = hi + lo + e,
-// |e| <= 2^-17 P for bf16, 2^-21 P for fp16) against the exact values: two products.  Lane layout as
-// in the split-product residual kernel: k-step m of lane group lg covers dimensions 32 m + 8 lg + j;
-// the V^T rows hold each pair of 16-key subtiles in contraction order (flash_key_pos), so every
-// operand is one 16-byte LDS read.
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+
+// Planes of the key / query rows, of the weights and of the values, and keys per LDS stage.
+__host__ __device__ constexpr int flash_kp(int in, int) { return in == F32 ? 3 : 1; }
+__host__ __device__ constexpr int flash_pp(int in, int w) { return (in == F32 || w == FLASH_EXP) ? 3 : 2; }
+__host__ __device__ constexpr int flash_vp(int in, int w) { return in == F32 ? 3 : (in == F16 && w == FLASH_EXP ? 2 : 1); }
+__host__ __device__ constexpr int flash_dps(int dp) { return dp < 32 ? 32 : dp; }
+__host__ __device__ constexpr int flash_stage_bytes(int dp, int dvt, int in, int w, int kb) {
+  return 2 * (flash_kp(in, w) * kb * (flash_dps(dp) + 8) + flash_vp(in, w) * dvt * 16 * (kb + 8));
+}
+__host__ __device__ constexpr int flash_kb(int dp, int dvt, int in, int w) {
+  return flash_stage_bytes(dp, dvt, in, w, 64) > 120 * 1024 ? 32 : 64;
+}
+// Two stages (the next batch is written while this one is read, one barrier a batch) where four workgroups'
+// stages fit a compute unit's 160 KiB; one stage (two barriers) otherwise.
+__host__ __device__ constexpr int flash_stages(int dp, int dvt, int in, int w) {
+  return flash_stage_bytes(dp, dvt, in, w, flash_kb(dp, dvt, in, w)) <= 20 * 1024 ? 2 : 1;
+}
+// waves per SIMD by the per-wave register arrays (query planes, accumulators, logits, staged units)
+__host__ __device__ constexpr int flash_occupancy(int dp, int dvt, int in, int w) {
+  const int kb = flash_kb(dp, dvt, in, w);
+  const int unit = in == F32 ? 4 : 2;
+  const int regs = flash_kp(in, w) * 2 * flash_dps(dp) / 8 + 2 * dvt * 4 + 2 * (kb / 16) * 4 +
+                   unit * ((kb * dp / 4 + 255) / 256 + 4 * ((kb / 4 * dvt * 4 + 255) / 256));
+  return regs <= 100 && in != F32 ? 3 : (regs <= 176 ? 2 : 1);
+}
 
 __host__ __device__ constexpr int flash_key_pos(int r) {
   return 32 * (r >> 5) + 8 * ((r >> 2) & 3) + 4 * ((r >> 4) & 1) + (r & 3);
 }
 
-template <bool F16>
+template <bool F16M>
 __device__ __forceinline__ floatx4 mfma16(const uint4& a, const uint4& b, floatx4 c) {
-  if constexpr (F16)
+  if constexpr (F16M)
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(halfx8, a), __builtin_bit_cast(halfx8, b), c,
                                                   0, 0, 0);
   else
@@ -295,72 +100,138 @@ __device__ __forceinline__ floatx4 mfma16(const uint4& a, const uint4& b, floatx
                                                    0, 0, 0);
 }
 
-// two fp32 values as packed 16-bit (bf16: round to nearest even; fp16: round toward zero, so the low
-// part x - hi keeps the sign of x) and back
-template <bool F16>
-__device__ __forceinline__ uint32_t pack16(float a, float b) {
-  if constexpr (F16)
-    return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
-  else
-    return pk_bf16(a, b);
-}
-template <bool F16>
-__device__ __forceinline__ float lo16(uint32_t p) {
-  if constexpr (F16)
-    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(p & 0xffffu)));
-  else
-    return __uint_as_float(p << 16);
-}
-template <bool F16>
-__device__ __forceinline__ float hi16(uint32_t p) {
-  if constexpr (F16)
-    return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(p >> 16)));
-  else
-    return __uint_as_float(p & 0xffff0000u);
+// x - (the 16-bit value in half `hi` of p), exact where the half is the rounding of x
+template <bool F16M>
+__device__ __forceinline__ void sub_pair(uint32_t p, float& a, float& b) {
+  if constexpr (F16M) {
+    a -= static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(p & 0xffffu)));
+    b -= static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(p >> 16)));
+  } else {
+    uint32_t c0 = 0x0000BF80u, c1 = 0xBF800000u;  // bf16 pairs (-1, 0), (0, -1); see split_pair
+    asm("" : "+s"(c0));
+    asm("" : "+s"(c1));
+    const bf16x2 hp = __builtin_bit_cast(bf16x2, p);
+    a = __builtin_amdgcn_fdot2_f32_bf16(hp, __builtin_bit_cast(bf16x2, c0), a, false);
+    b = __builtin_amdgcn_fdot2_f32_bf16(hp, __builtin_bit_cast(bf16x2, c1), b, false);
+  }
 }
 
-// the first `valid` of the 4 16-bit elements of a raw unit (x: elements 0, 1; y: 2, 3), the rest zero
-__device__ __forceinline__ uint2 mask16(uint2 u, int valid) {
-  const uint32_t m0 = valid >= 2 ? 0xffffffffu : (valid == 1 ? 0x0000ffffu : 0u);
-  const uint32_t m1 = valid >= 4 ? 0xffffffffu : (valid == 3 ? 0x0000ffffu : 0u);
-  return uint2{u.x & m0, u.y & m1};
+// two fp32 values as NP packed 16-bit planes (bf16: each plane rounded to nearest even; fp16: toward zero)
+template <int NP, bool F16M>
+__device__ __forceinline__ void plane_pair(float a, float b, uint32_t (&p)[NP]) {
+#pragma unroll
+  for (int i = 0; i < NP; ++i) {
+    if constexpr (F16M)
+      p[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a, b));
+    else
+      p[i] = pk_bf16(a, b);
+    if (i + 1 < NP) sub_pair<F16M>(p[i], a, b);
+  }
 }
 
-// two workgroups per compute unit while the accumulators and staging registers fit in 256 VGPRs
-__host__ __device__ constexpr int flash16_occupancy(int dp, int dvt) { return dp + 16 * dvt <= 128 ? 2 : 1; }
+// Elements of a 4-element unit starting at column c that lie in [0, width), the rest zero (a select,
+// so padding that holds non-finite bits cannot leak in).
+template <int ES>
+__device__ __forceinline__ uint4 unit_clip(uint4 u, int valid) {
+  if constexpr (ES == 4)
+    return uint4{valid > 0 ? u.x : 0u, valid > 1 ? u.y : 0u, valid > 2 ? u.z : 0u, valid > 3 ? u.w : 0u};
+  else
+    return uint4{u.x & (valid > 1 ? 0xffffffffu : (valid > 0 ? 0xffffu : 0u)),
+                 u.y & (valid > 3 ? 0xffffffffu : (valid > 2 ? 0xffffu : 0u)), 0u, 0u};
+}
 
-template <int DP, int DVT, int RS, bool F16>
-__global__ __launch_bounds__(256, flash16_occupancy(DP, DVT)) void flash_attn16_kernel(const FlashArgs a) {
-  constexpr int KB = 64;  // keys per LDS stage
+// Buffer resource of `bytes` bytes at p: loads beyond it return zero (at most 1 GiB: a batch needs
+// a few tens of KiB, and the offset that marks absent units lies behind it).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t flash_rsrc(const void* p, int64_t bytes) {
+  const int64_t b = bytes < 0 ? 0 : (bytes > 0x40000000 ? 0x40000000 : bytes);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(b), 0x00020000);
+}
+template <int ES>
+__device__ __forceinline__ uint4 load_buf(__amdgpu_buffer_rsrc_t r, int off) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  if constexpr (ES == 4) {
+    const u4 x = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+    return uint4{x.x, x.y, x.z, x.w};
+  } else {
+    const u2 x = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    return uint4{x.x, x.y, 0u, 0u};
+  }
+}
+
+// Which tile a workgroup takes.  Long tiles first (the last rows have the most keys); the workgroups of one
+// XCD (w % 8) share heads when the heads divide by 8.  When about two workgroups fit a compute unit at a
+// time the first two rounds are all there is, and plain descending order would give compute unit c the
+// c-th longest of both rounds (1.5x the mean for the first): the second round therefore ascends.
+__device__ __forceinline__ void flash_tile(const FlashArgs& a, int64_t& bh, int& t) {
+  const int total = gridDim.x, nbh = static_cast<int>(a.bh);
+  const bool xcd = (nbh & 7) == 0;
+  const int hx = xcd ? nbh >> 3 : nbh;            // heads of this group of workgroups
+  const int j = xcd ? blockIdx.x >> 3 : blockIdx.x;
+  const int count = xcd ? total >> 3 : total, round = xcd ? 32 : 256;
+  int rank = j;
+  if (j >= round && j < 2 * round) {
+    const int m = (count < 2 * round ? count : 2 * round) - round;
+    if (j - round < m) rank = round + (m - 1 - (j - round));
+  }
+  const int step = rank / hx, h = rank - step * hx;
+  t = a.n_tiles - 1 - step;
+  bh = xcd ? (blockIdx.x & 7) * hx + h : h;
+}
+
+// One workgroup per (head, tile of FLASH_ROWS query rows); wave w owns 2 strips of 16 rows.  Keys [0, last row
+// of the tile] are staged KB at a time (K row-major, V transposed), the next batch's rows loaded into
+// registers while the current one computes.  A wave skips batches that lie wholly after its rows and
+// applies the causal mask only on batches that straddle them.
+template <int DP, int DVT, int IN, int W>
+__global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_attn_kernel(const FlashArgs a) {
+  constexpr int ES = IN == F32 ? 4 : 2;
+  constexpr int RS = 2;
+  constexpr int KB = flash_kb(DP, DVT, IN, W);
   constexpr int NSUB = KB / 16;
-  constexpr int DPS = DP < 32 ? 32 : DP;  // dimensions in whole 32-element steps
+  constexpr int DPS = flash_dps(DP);  // dimensions in whole 32-element steps
   constexpr int MS = DPS / 32;
-  constexpr int LDK = DPS + 8;  // 16-bit elements per key row: 16 (2 j + 1) bytes
+  constexpr int KP = flash_kp(IN, W), PP = flash_pp(IN, W), VP = flash_vp(IN, W);
+  constexpr int XORD = KP == 3 ? 2 : 0;  // plane products (i, j) with i + j <= order are taken
+  constexpr int PORD = (PP > VP ? PP : VP) - 1;
+  constexpr bool KF16 = IN == F16, PF16 = IN == F16 && W == FLASH_SOFTMAX;
+  // denominators: a column of ones on the matrix cores where the weights' planes keep fp32 accuracy and the
+  // matrix cores have room (16-bit inputs), else fp32 VALU sums
+  constexpr bool DENM = IN != F32 && PP == 3;
+  // how far (log2) a row may exceed its running maximum before the sums are rescaled; two-plane weights keep
+  // the latest maximum, whose own weight 1 is then exact (bf16, 32 heads x 8192: error against 64 bits 1.9e-6
+  // and 479 us, with 8 here 2.1e-6 and 450 us)
+  constexpr float GROW = PP == 3 ? 8.f : 0.f;
+  constexpr int LDK = DPS + 8;      // 16-bit elements per key row: 16 (2 j + 1) bytes
   constexpr int DV = DVT * 16;
   constexpr int LDV = KB + 8;
-  constexpr int TM = 64 * RS;
-  constexpr int KU = DP / 4, VU = DV / 4;
-  constexpr int KPT = (KB * KU + 255) / 256, VPT = (KB * VU + 255) / 256;
-  __shared__ uint4 kst4[(KB * LDK + 7) / 8];
-  __shared__ uint4 vst4[(DV * LDV + 7) / 8];
-  uint16_t* const Kst = reinterpret_cast<uint16_t*>(kst4);
-  uint16_t* const Vst = reinterpret_cast<uint16_t*>(vst4);
+  constexpr int KPL = KB * LDK, VPL = DV * LDV;  // elements of a plane
+  constexpr int STAGE = KP * KPL + VP * VPL;
+  constexpr int NST = flash_stages(DP, DVT, IN, W);
+  constexpr int KU = DP / 4, VU = DV / 4, KG = KB / 4;
+  constexpr int KPT = (KB * KU + 255) / 256, VPT = (KG * VU + 255) / 256;
+  __shared__ uint4 stage4[(NST * STAGE + 7) / 8];
+  uint16_t* const stage = reinterpret_cast<uint16_t*>(stage4);
 
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
-  const int64_t bh = wg / a.n_tiles;
-  const int t = a.n_tiles - 1 - (wg - static_cast<int>(bh) * a.n_tiles);
+  int64_t bh;
+  int t;
+  flash_tile(a, bh, t);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int n = static_cast<int>(a.n);
-  const int r0 = t * TM;
+  const int r0 = t * FLASH_ROWS;
   const int64_t qkbase = bh * a.n * a.ldqk;
   const int64_t vbase = bh * a.n * a.ldv;
 
-  // the wave's query rows as B operands (8 dimensions per lane and k-step), columns >= d zero
+  // the wave's query rows as B operands (8 dimensions per lane and k-step), columns >= d zero.  fp32 rows
+  // are scaled before they are split; 16-bit rows keep their exact values and the logits are scaled
+  // instead, by |scale| (its sign moves to the queries, so that the largest product is the largest logit).
   int myrow[RS];
   bool rvalid[RS];
-  uint4 qB[RS][MS];
+  uint4 qB[RS][MS][KP];
+  const uint32_t flip = (IN != F32 && a.scale2 < 0.f) ? 0x80008000u : 0u;
+  const float sc = IN == F32 ? 1.f : (a.scale2 < 0.f ? -a.scale2 : a.scale2);
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
     myrow[rs] = r0 + (wave * RS + rs) * 16 + li;
@@ -368,180 +239,308 @@ __global__ __launch_bounds__(256, flash16_occupancy(DP, DVT)) void flash_attn16_
     const int64_t qoff = qkbase + static_cast<int64_t>(rvalid[rs] ? myrow[rs] : 0) * a.ldqk;
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
-      uint2 h[2];
+      uint32_t w[KP][4];
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         const int col = 32 * m + 8 * lg + 4 * hh;
-        const uint4 raw = load_unit<2>(a.q, qoff + min(col, a.ldqk - 4));
-        h[hh] = mask16(uint2{raw.x, raw.y}, rvalid[rs] ? a.d - col : 0);
+        const uint4 raw = unit_clip<ES>(load_unit<ES>(a.q, qoff + min(col, a.ldqk - 4)), rvalid[rs] ? a.d - col : 0);
+        if constexpr (IN == F32) {
+          const floatx4 f = unit_to_f4<4>(raw, F32, a.scale2);
+          uint32_t p[KP];
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            plane_pair<KP, false>(f[2 * e], f[2 * e + 1], p);
+#pragma unroll
+            for (int i = 0; i < KP; ++i) w[i][2 * hh + e] = p[i];
+          }
+        } else {
+          w[0][2 * hh] = raw.x ^ flip;
+          w[0][2 * hh + 1] = raw.y ^ flip;
+        }
       }
-      qB[rs][m] = uint4{h[0].x, h[0].y, h[1].x, h[1].y};
+#pragma unroll
+      for (int i = 0; i < KP; ++i) qB[rs][m][i] = uint4{w[i][0], w[i][1], w[i][2], w[i][3]};
     }
   }
   const int wrow_lo = r0 + wave * RS * 16, wrow_hi = wrow_lo + RS * 16 - 1;
 
-  floatx4 num[RS][DVT];
+  floatx4 num[RS][DVT], dacc[RS];
   float den[RS], mrow[RS];
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
     den[rs] = 0.f;
-    mrow[rs] = -1e30f;
+    dacc[rs] = floatx4{0.f, 0.f, 0.f, 0.f};
+    mrow[rs] = -1e30f;  // finite: exp2(m_old - m_new) is then 0 or 1, never a NaN
 #pragma unroll
     for (int ct = 0; ct < DVT; ++ct) num[rs][ct] = floatx4{0.f, 0.f, 0.f, 0.f};
   }
+  const uint32_t one2 = PF16 ? 0x3c003c00u : 0x3f803f80u;
+  const uint4 ones = uint4{one2, one2, one2, one2};
 
-  auto process = [&](auto diag_tag, int off) {
+  auto process = [&](auto diag_tag, int off, const uint16_t* Kst, const uint16_t* Vst) {
     constexpr bool DIAG = decltype(diag_tag)::value;
     floatx4 X[NSUB][RS];
 #pragma unroll
     for (int kt = 0; kt < NSUB; ++kt)
 #pragma unroll
       for (int rs = 0; rs < RS; ++rs) X[kt][rs] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // two key subtiles at a time: 2 RS independent chains of products cover the matrix-core latency
 #pragma unroll
-    for (int m = 0; m < MS; ++m)
+    for (int kp = 0; kp < NSUB; kp += 2)
 #pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt) {
-        const uint4 kv = *reinterpret_cast<const uint4*>(Kst + (16 * kt + li) * LDK + 32 * m + 8 * lg);
+      for (int m = 0; m < MS; ++m) {
+        uint4 kv[2][KP];
 #pragma unroll
-        for (int rs = 0; rs < RS; ++rs) X[kt][rs] = mfma16<F16>(kv, qB[rs][m], X[kt][rs]);
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < KP; ++i)
+            kv[h][i] = *reinterpret_cast<const uint4*>(Kst + i * KPL + (16 * (kp + h) + li) * LDK + 32 * m + 8 * lg);
+#pragma unroll
+        for (int o = XORD; o >= 0; --o)  // smallest products first
+#pragma unroll
+          for (int i = 0; i <= o; ++i)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+              for (int rs = 0; rs < RS; ++rs)
+                if (i < KP && o - i < KP) X[kp + h][rs] = mfma16<KF16>(kv[h][i], qB[rs][m][o - i], X[kp + h][rs]);
       }
+    if constexpr (W == FLASH_SOFTMAX) {
+      // The weights are relative to a row maximum that is replaced (and the sums rescaled) only when some
+      // row of the wave exceeds its own by more than GROW.  Lanes compare their own keys, so a batch that
+      // changes no maximum has no cross-lane step.
+      bool grow = false;
+      float mx[RS];
 #pragma unroll
-    for (int rs = 0; rs < RS; ++rs) {
-      float mx = -__builtin_huge_valf();
+      for (int rs = 0; rs < RS; ++rs) {
+        float m0 = -__builtin_huge_valf(), m1 = -__builtin_huge_valf();
 #pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt)
+        for (int kt = 0; kt < NSUB; ++kt)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          float y = X[kt][rs][r] * a.scale2;
-          if constexpr (DIAG) {
-            if (off + 16 * kt + 4 * lg + r > myrow[rs]) y = -__builtin_huge_valf();
+          for (int r = 0; r < 4; ++r) {
+            float x = X[kt][rs][r];
+            if constexpr (DIAG) {
+              if (off + 16 * kt + 4 * lg + r > myrow[rs]) x = -__builtin_huge_valf();
+            }
+            float& mm = (r & 1) ? m1 : m0;
+            mm = __builtin_amdgcn_fmed3f(mm, x, __builtin_huge_valf());  // max, without quieting its inputs
           }
-          X[kt][rs][r] = y;
-          mx = fmaxf(mx, y);
+        mx[rs] = __builtin_amdgcn_fmed3f(m0, m1, __builtin_huge_valf()) * sc;
+        grow = grow || mx[rs] > mrow[rs] + GROW;
+      }
+      if (__any(grow)) {
+#pragma unroll
+        for (int rs = 0; rs < RS; ++rs) {
+          float m0 = fmaxf(mrow[rs], mx[rs]);
+          m0 = fmaxf(m0, __shfl_xor(m0, 16));
+          m0 = fmaxf(m0, __shfl_xor(m0, 32));
+          const float alpha = __builtin_amdgcn_exp2f(mrow[rs] - m0);
+          mrow[rs] = m0;
+          if constexpr (DENM) dacc[rs] *= alpha;
+          den[rs] *= alpha;
+#pragma unroll
+          for (int ct = 0; ct < DVT; ++ct) num[rs][ct] *= alpha;
         }
-      mx = fmaxf(mx, __shfl_xor(mx, 16));
-      mx = fmaxf(mx, __shfl_xor(mx, 32));
-      const float mnew = fmaxf(mrow[rs], mx);
-      const float alpha = __builtin_amdgcn_exp2f(mrow[rs] - mnew);
-      mrow[rs] = mnew;
-      den[rs] *= alpha;
-#pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) num[rs][ct] *= alpha;
-#pragma unroll
-      for (int kt = 0; kt < NSUB; ++kt)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const float p = __builtin_amdgcn_exp2f(X[kt][rs][r] - mnew);
-          X[kt][rs][r] = p;
-          den[rs] += p;
-        }
+      }
     }
 #pragma unroll
     for (int sp = 0; sp < NSUB / 2; ++sp) {
-      uint4 ph[RS], pl[RS];
+      uint4 pB[RS][PP];
 #pragma unroll
       for (int rs = 0; rs < RS; ++rs) {
-        uint32_t h[4], l[4];
+        uint32_t w[PP][4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const floatx4& P = X[2 * sp + (e >> 1)][rs];
-          const float p0 = P[2 * (e & 1)], p1 = P[2 * (e & 1) + 1];
-          h[e] = pack16<F16>(p0, p1);
-          l[e] = pack16<F16>(p0 - lo16<F16>(h[e]), p1 - hi16<F16>(h[e]));
+          float p[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int kt = 2 * sp + (e >> 1), r = 2 * (e & 1) + h;
+            const float x = X[kt][rs][r];
+            float y;
+            if constexpr (W == FLASH_SOFTMAX)
+              y = IN == F32 ? x - mrow[rs] : fmaf(x, sc, -mrow[rs]);
+            else
+              y = IN == F32 ? x : x * sc;
+            p[h] = __builtin_amdgcn_exp2f(y);
+            if constexpr (DIAG) {
+              if (off + 16 * kt + 4 * lg + r > myrow[rs]) p[h] = 0.f;
+            }
+            if constexpr (!DENM) den[rs] += p[h];
+          }
+          uint32_t pl[PP];
+          plane_pair<PP, PF16>(p[0], p[1], pl);
+#pragma unroll
+          for (int i = 0; i < PP; ++i) w[i][e] = pl[i];
         }
-        ph[rs] = uint4{h[0], h[1], h[2], h[3]};
-        pl[rs] = uint4{l[0], l[1], l[2], l[3]};
+#pragma unroll
+        for (int i = 0; i < PP; ++i) pB[rs][i] = uint4{w[i][0], w[i][1], w[i][2], w[i][3]};
       }
+      if constexpr (DENM) {
 #pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) {
-        const uint4 vv = *reinterpret_cast<const uint4*>(Vst + (16 * ct + li) * LDV + 32 * sp + 8 * lg);
+        for (int i = PP - 1; i >= 0; --i)
 #pragma unroll
-        for (int rs = 0; rs < RS; ++rs) num[rs][ct] = mfma16<F16>(vv, pl[rs], num[rs][ct]);
+          for (int rs = 0; rs < RS; ++rs) dacc[rs] = mfma16<PF16>(ones, pB[rs][i], dacc[rs]);
+      }
+      constexpr int CG = DVT % 2 == 0 ? 2 : 1;  // value columns in pairs, as the key subtiles above
 #pragma unroll
-        for (int rs = 0; rs < RS; ++rs) num[rs][ct] = mfma16<F16>(vv, ph[rs], num[rs][ct]);
+      for (int cp = 0; cp < DVT; cp += CG) {
+        uint4 vv[CG][VP];
+#pragma unroll
+        for (int h = 0; h < CG; ++h)
+#pragma unroll
+          for (int i = 0; i < VP; ++i)
+            vv[h][i] = *reinterpret_cast<const uint4*>(Vst + i * VPL + (16 * (cp + h) + li) * LDV + 32 * sp + 8 * lg);
+#pragma unroll
+        for (int o = PORD; o >= 0; --o)
+#pragma unroll
+          for (int i = 0; i <= o; ++i)
+#pragma unroll
+            for (int h = 0; h < CG; ++h)
+#pragma unroll
+              for (int rs = 0; rs < RS; ++rs)
+                if (i < VP && o - i < PP)
+                  num[rs][cp + h] = mfma16<PF16>(vv[h][i], pB[rs][o - i], num[rs][cp + h]);
       }
     }
   };
 
-  const int row_hi = (r0 + TM < n ? r0 + TM : n) - 1;
+  const int row_hi = (r0 + FLASH_ROWS < n ? r0 + FLASH_ROWS : n) - 1;  // r0 < n: t < ceil(n / FLASH_ROWS)
   const int kend = row_hi + 1;
   const int nb = (kend + KB - 1) / KB;
 
-  uint2 pk[KPT], pv[VPT];
-  uint32_t pk_ok = 0, pv_ok = 0;
+  // Staging registers: this thread's 4-element units of the next batch's rows, raw: key rows unit by unit,
+  // value rows as blocks of 4 keys x 4 columns (the transposed write is then 8 bytes).  Offsets inside
+  // a batch are fixed per thread; the batch moves the buffer's base, whose size is the rows the tile
+  // needs, so rows behind them (and units behind the columns) read as zero.
+  int koff[KPT], voff[VPT];
+#pragma unroll
+  for (int i = 0; i < KPT; ++i) {
+    const int e = tid + 256 * i, r = e / KU, u = e - r * KU;
+    koff[i] = (e < KB * KU && 4 * u < a.d) ? (r * a.ldqk + 4 * u) * ES : 0x7ffffff0;
+  }
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int e = tid + 256 * i, g = e % KG, u = e / KG;  // key-fast: conflict-light transposed writes
+    voff[i] = (e < KG * VU && 4 * u < a.dv) ? (4 * g * a.ldv + 4 * u) * ES : 0x7ffffff0;
+  }
+  const bool kclip = (a.d & 3) != 0, vclip = (a.dv & 3) != 0;
+  const char* const kp0 = static_cast<const char*>(a.k) + qkbase * ES;
+  const char* const vp0 = static_cast<const char*>(a.v) + vbase * ES;
+  uint4 pk[KPT], pv[VPT][4];
   auto prefetch = [&](int off) {
-    pk_ok = pv_ok = 0;
+    const __amdgpu_buffer_rsrc_t kr = flash_rsrc(kp0 + static_cast<int64_t>(off) * a.ldqk * ES,
+                                                 static_cast<int64_t>(kend - off) * a.ldqk * ES);
+    const __amdgpu_buffer_rsrc_t vr = flash_rsrc(vp0 + static_cast<int64_t>(off) * a.ldv * ES,
+                                                 static_cast<int64_t>(kend - off) * a.ldv * ES);
 #pragma unroll
-    for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      const int r = e / KU, u = e - r * KU;
-      const bool ok = e < KB * KU && off + r < kend && 4 * u < a.d;
-      pk_ok |= ok ? (1u << i) : 0u;
-      const int src = ok ? off + r : 0;
-      const uint4 raw = load_unit<2>(a.k, qkbase + static_cast<int64_t>(src) * a.ldqk + min(4 * u, a.ldqk - 4));
-      pk[i] = uint2{raw.x, raw.y};
-    }
+    for (int i = 0; i < KPT; ++i) pk[i] = load_buf<ES>(kr, koff[i]);
 #pragma unroll
-    for (int i = 0; i < VPT; ++i) {
-      const int e = tid + 256 * i;
-      const int r = e % KB, u = e / KB;
-      const bool ok = e < KB * VU && off + r < kend && 4 * u < a.dv;
-      pv_ok |= ok ? (1u << i) : 0u;
-      const int src = ok ? off + r : 0;
-      const uint4 raw = load_unit<2>(a.v, vbase + static_cast<int64_t>(src) * a.ldv + min(4 * u, a.ldv - 4));
-      pv[i] = uint2{raw.x, raw.y};
-    }
+    for (int i = 0; i < VPT; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        pv[i][c] = load_buf<ES>(vr, voff[i] == 0x7ffffff0 ? voff[i] : voff[i] + c * a.ldv * ES);
   };
-  auto commit = [&]() {
+  auto commit = [&](uint16_t* Kst, uint16_t* Vst) {
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * KU) {
-        const int r = e / KU, u = e - r * KU;
-        const int valid = ((pk_ok >> i) & 1u) ? a.d - 4 * u : 0;
-        *reinterpret_cast<uint2*>(Kst + r * LDK + 4 * u) = mask16(pk[i], valid);
+      const int e = tid + 256 * i, r = e / KU, u = e - r * KU;
+      if (KB * KU % 256 != 0 && e >= KB * KU) continue;
+      uint4 x = pk[i];
+      if (kclip) x = unit_clip<ES>(x, a.d - 4 * u);
+      if constexpr (IN == F32) {
+        const floatx4 f = unit_to_f4<4>(x, F32, 1.f);
+        uint32_t p0[KP], p1[KP];
+        plane_pair<KP, false>(f[0], f[1], p0);
+        plane_pair<KP, false>(f[2], f[3], p1);
+#pragma unroll
+        for (int j = 0; j < KP; ++j) *reinterpret_cast<uint2*>(Kst + j * KPL + r * LDK + 4 * u) = uint2{p0[j], p1[j]};
+      } else {
+        *reinterpret_cast<uint2*>(Kst + r * LDK + 4 * u) = uint2{x.x, x.y};
       }
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * VU) {
-        const int r = e % KB, u = e / KB;
-        const uint2 w = mask16(pv[i], ((pv_ok >> i) & 1u) ? a.dv - 4 * u : 0);
-        const int pos = flash_key_pos(r);
-        Vst[(4 * u + 0) * LDV + pos] = static_cast<uint16_t>(w.x & 0xffffu);
-        Vst[(4 * u + 1) * LDV + pos] = static_cast<uint16_t>(w.x >> 16);
-        Vst[(4 * u + 2) * LDV + pos] = static_cast<uint16_t>(w.y & 0xffffu);
-        Vst[(4 * u + 3) * LDV + pos] = static_cast<uint16_t>(w.y >> 16);
+      const int e = tid + 256 * i, g = e % KG, u = e / KG;
+      if (KG * VU % 256 != 0 && e >= KG * VU) continue;
+      uint4 x[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[c] = vclip ? unit_clip<ES>(pv[i][c], a.dv - 4 * u) : pv[i][c];
+      uint16_t* const dst = Vst + 4 * u * LDV + flash_key_pos(4 * g);
+      if constexpr (VP == 1) {
+        // 16-bit 4 x 4 transpose: column m of the 4 keys
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
+          const uint32_t k0 = m < 2 ? x[0].x : x[0].y, k1 = m < 2 ? x[1].x : x[1].y;
+          const uint32_t k2 = m < 2 ? x[2].x : x[2].y, k3 = m < 2 ? x[3].x : x[3].y;
+          *reinterpret_cast<uint2*>(dst + m * LDV) =
+              uint2{__builtin_amdgcn_perm(k1, k0, sel), __builtin_amdgcn_perm(k3, k2, sel)};
+        }
+      } else {
+        floatx4 f[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) f[c] = unit_to_f4<ES>(x[c], IN, 1.f);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          uint32_t p0[VP], p1[VP];
+          plane_pair<VP, false>(f[0][m], f[1][m], p0);
+          plane_pair<VP, false>(f[2][m], f[3][m], p1);
+#pragma unroll
+          for (int j = 0; j < VP; ++j) *reinterpret_cast<uint2*>(dst + j * VPL + m * LDV) = uint2{p0[j], p1[j]};
+        }
       }
     }
   };
 
   if constexpr (DPS != DP) {  // dimensions [DP, DPS) of the key rows are never written: zero them
-    for (int e = tid; e < KB * LDK; e += 256) Kst[e] = 0;
+    for (int s = 0; s < NST; ++s)
+      for (int e = tid; e < KP * KPL; e += 256) stage[s * STAGE + e] = 0;
+    __syncthreads();
   }
-  prefetch(0);
-  for (int b = 0; b < nb; ++b) {
-    __syncthreads();
-    commit();
-    __syncthreads();
-    if (b + 1 < nb) prefetch((b + 1) * KB);
+  auto compute = [&](int b, const uint16_t* st) {
     const int off = b * KB;
     if (off <= wrow_hi) {
       if (off + KB - 1 > wrow_lo)
-        process(std::true_type{}, off);
+        process(std::true_type{}, off, st, st + KP * KPL);
       else
-        process(std::false_type{}, off);
+        process(std::false_type{}, off, st, st + KP * KPL);
+    }
+  };
+  prefetch(0);
+  if constexpr (NST == 2) {
+    commit(stage, stage + KP * KPL);
+    if (nb > 1) prefetch(KB);
+    __syncthreads();
+    for (int b = 0; b < nb; ++b) {
+      compute(b, stage + (b & 1) * STAGE);
+      // the other stage was read by batch b - 1, which every wave finished before the last barrier
+      if (b + 1 < nb) commit(stage + ((b + 1) & 1) * STAGE, stage + ((b + 1) & 1) * STAGE + KP * KPL);
+      if (b + 2 < nb) prefetch((b + 2) * KB);
+      __syncthreads();
+    }
+  } else {
+    for (int b = 0; b < nb; ++b) {
+      __syncthreads();  // every wave is done with the stage of the previous batch
+      commit(stage, stage + KP * KPL);
+      __syncthreads();  // staged batch visible
+      if (b + 1 < nb) prefetch((b + 1) * KB);
+      compute(b, stage);
     }
   }
 
+  // ---- epilogue: row sums (over the four lane groups), normalise, store ----
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
-    float dsum = den[rs];
-    dsum += __shfl_xor(dsum, 16);
-    dsum += __shfl_xor(dsum, 32);
+    float dsum;
+    if constexpr (DENM) {
+      dsum = dacc[rs][0];  // every element of the column is the row's sum
+    } else {
+      dsum = den[rs];
+      dsum += __shfl_xor(dsum, 16);
+      dsum += __shfl_xor(dsum, 32);
+    }
     if (!rvalid[rs]) continue;
-    const float dn = fmaxf(dsum, 1e-20f);
+    const float dn = fmaxf(dsum, a.floor);
     const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
 #pragma unroll
     for (int ct = 0; ct < DVT; ++ct) {

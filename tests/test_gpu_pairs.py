@@ -1,0 +1,74 @@
+"""The pair kernel (sta_flash_attention, sta_exact_attention) at the edges of its tiles, key batches and tile
+orders, against float64 attention.  fp32 operands as three bf16 planes keep each product within 2^-23 of its
+value and the sums are fp32: a few 2^-23 in the 2-norm (1e-6).  bf16 weights as hi + lo planes of 8 bits are
+within 2^-16 each, uniform and of random sign (4e-6 at most in the 2-norm).  16-bit outputs add their rounding:
+half a unit in the last of 8 (bf16) or 11 (fp16) bits at most, uniform, so 2^-8 / sqrt(3) or 2^-11 / sqrt(3)."""
+
+import pytest
+import torch
+
+import fast_article_attention as faa
+import triton_article_attention as taa
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+TOL = {torch.float32: 0.0, torch.bfloat16: 2 ** -8 / 3 ** 0.5, torch.float16: 2 ** -11 / 3 ** 0.5}
+
+
+def exact(q, k, v, scale, eps=None):
+    x = q.double() @ k.double().transpose(-1, -2).contiguous() * scale
+    x = x.masked_fill(torch.ones(x.shape[-2:], dtype=torch.bool).triu_(1), float("-inf"))
+    w = torch.softmax(x, -1) if eps is None else torch.exp(x)
+    den = 1.0 if eps is None else w.sum(-1, keepdim=True).clamp_min(eps)
+    return w @ v.double() / den
+
+
+def rel(a, b):
+    return (a.cpu().double() - b).norm().item() / b.norm().item()
+
+
+# heads x tiles: one workgroup, a full first round, a part of the second, more than two rounds, heads that
+# divide by the XCDs and heads that do not; n around the 64- and 32-key batches and the 128-row tiles
+@pytest.mark.parametrize("heads,n,d,dv", [
+    (1, 1, 4, 4), (1, 63, 64, 64), (2, 64, 16, 16), (3, 65, 40, 72), (1, 129, 128, 128), (2, 257, 33, 30),
+    (8, 1025, 64, 64), (8, 4225, 16, 32), (24, 300, 80, 96), (5, 7300, 32, 16), (3, 200, 128, 256), (700, 130, 8, 8),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("scale", [0.3, -0.2])
+def test_pairs_match_float64(heads, n, d, dv, dtype, scale):
+    g = torch.Generator().manual_seed(n * 7 + d)
+    q, k, v = (torch.randn(1, heads, n, w, generator=g).mul_(0.7 if w == d else 1.0).to(dtype) for w in (d, d, dv))
+    h = torch.tensor(sorted({0, heads // 2, heads - 1}))
+    print(heads, n, d, dv, dtype, scale, flush=True)
+    out = taa.triton_flash_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=scale)
+    ref = exact(q[:, h], k[:, h], v[:, h], scale)
+    assert rel(out[:, h.to(DEV)], ref) < (4e-6 if dtype == torch.bfloat16 else 1e-6)
+    out = faa.fast_article_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=scale, compressor="none")
+    ref = exact(q[:, h], k[:, h], v[:, h], scale, 1e-12)
+    assert rel(out[:, h.to(DEV)], ref) < TOL[dtype] + 1e-6
+
+
+@pytest.mark.parametrize("n,block", [(128, 128), (100, 128), (129, 128)])
+def test_sequence_inside_its_first_block(n, block):
+    """No coreset item up to n = block: exact attention; past it the block is compressed."""
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(2, 3, n, 32, generator=g) for _ in range(3))
+    out = faa.fast_article_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=0.1, block_size=block)
+    ref = exact(q, k, v, 0.1, 1e-12)
+    assert rel(out[:, :, :block], ref[:, :, :block]) < (1e-6 if n <= block else 2e-5)  # 2-plane products beyond
+
+
+def test_pair_weights_and_the_smallest_denominator():
+    """Raw weights far below 1 meet the smallest denominator as in num / max(den, eps); scale 0 is the mean."""
+    g = torch.Generator().manual_seed(6)
+    q = torch.full((1, 2, 70, 16), 2.0)
+    k = torch.full((1, 2, 70, 16), -1.5)
+    v = torch.randn(1, 2, 70, 16, generator=g)
+    out = faa.fast_article_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=1.0, compressor="none",
+                                            denominator_eps=1e-3)
+    ref = exact(q, k, v, 1.0, 1e-3)
+    assert rel(out, ref) < 2 * 48 * 2 ** -24  # the rounding of a logit of -48 is the weight's relative error
+    for dtype in (torch.float32, torch.bfloat16):
+        out = taa.triton_flash_causal_attention(q.to(DEV, dtype), k.to(DEV, dtype), v.to(DEV, dtype), scale=0.0)
+        mean = v.to(dtype).double().cumsum(2) / torch.arange(1, 71).reshape(-1, 1)
+        assert rel(out, mean) < 4e-6
