@@ -415,6 +415,17 @@ int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, 
 int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream);
 
+/*
+ * The Taylor part over pairs, for short sequences: low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i,
+ * c(i) = floor((i + shift) / chunk) chunk - shift, in sta_moments' partials layout with nsplit partials (a tile's
+ * keys are dealt out to nsplit workgroups), for sta_block_attention with the same chunk and shift.
+ * degree <= 3, 0 <= shift < chunk, low_num 16-byte aligned; the other arguments as sta_flash_attention.  fp32
+ * operands are carried as bf16 hi + lo.
+ */
+int sta_pair_moments(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d, int dv,
+                     int ld_qk, int ld_v, int degree, float scale, int chunk, int shift, int nsplit, float* low_num,
+                     float* low_den, void* stream);
+
 /* Rows per block-attention tile and the moment chunk the library uses for a head dimension D (the
  * chunk argument of sta_block_attention is that chunk for sta_moments' partials, the query block for
  * sta_moments_ws' partials). */

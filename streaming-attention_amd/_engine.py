@@ -109,6 +109,30 @@ def ws_query_block(semantics: str, block: int) -> Optional[int]:
     return None  # raw Taylor sums: the residual kernel adds the polynomial over the query block's keys
 
 
+# Longest sequence whose Taylor part runs over the pairs (sta_pair_moments) instead of the moment scan: the
+# pairs take n^2 / 2 (d + dv) products of a head, the moments n F dv for F features, both with the widths the
+# kernels pad to (and the scan no less than that of 512 features x 64 columns: its cost per chunk), so the
+# crossing is at n = R F dv / (d + dv), R from the rates measured on both sides (64 heads, d = dv = 64, degree 2,
+# scan / pairs): fp32 4096: 564 / 427 us, 6144: 881 / 968; fp16 6144: 943 / 746, 8192: 1372 / 1339; bf16 (two products
+# a value less) 6144: 775 / 561, 8192: 1071 / 1001.  d = dv = 128 (32 heads), fp32 8192: 5459 / 2385, bf16 5739 / 1026;
+# d = 16, dv = 64, degree 3, fp32 2048: 169 / 95, 4096: 317 / 342; degree 1, d = 64, fp32 1024: 61 / 49, 2048: 111 / 141.
+PAIRS_RATIO = {torch.float32: 4.7, torch.bfloat16: 7.5, torch.float16: 6.5}
+
+
+def use_pairs(n: int, d: int, dv: int, degree: int, dtype: torch.dtype) -> bool:
+    pad_d = max(16, 1 << (d - 1).bit_length())
+    pad_dv = max(16, 1 << (dv - 1).bit_length())
+    scan = max(_plan.num_features(d, degree) * 64 * -(-dv // 64), 512 * 64)
+    return n * (pad_d + pad_dv) <= PAIRS_RATIO[dtype] * scan
+
+
+def pair_splits(bh: int, n: int, compute_units: int) -> int:
+    """Workgroups that share a tile's keys in sta_pair_moments: two workgroups a compute unit where the tiles
+    alone are fewer, at most one per 256 keys of the longest tile and 8 (each adds a partial sum to read)."""
+    tiles = bh * -(-n // _plan.TILE_ROWS)
+    return max(1, min(2 * compute_units // tiles, n // 256, 8))
+
+
 # Offer the planner the 64-column moment workgroups (split products, 32 < dv <= 64).  Off: on 32 heads x
 # 65536 tokens (d = dv = 64) they take 9.6 ms against 8.4 ms for two 32-column workgroups per compute
 # unit; the feature work they save (17 % of the VALU) is less than one wave per SIMD loses in latency.
@@ -254,7 +278,8 @@ def prefill(
     reference_keys: Optional[torch.Tensor] = None,
 ) -> PrefillResult:
     """Run the whole prefill for contiguous [BH, N, D] device tensors of one dtype.  moment_kernel:
-    "ws" (sta_moments_ws where it applies), "chunked" (sta_moments) or None (use_moments_ws).
+    "ws" (sta_moments_ws where it applies), "chunked" (sta_moments), "pairs" (sta_pair_moments where it
+    applies) or None (use_pairs, then use_moments_ws).
     score_keys: the float64 keys of a float64 caller ([BH, N, D], contiguous, on the device; k3 is
     their float32 rounding): the compressor then draws its directions and uniforms as float64 and
     scores these keys in fp64, as the reference's float64 run does.
@@ -297,6 +322,7 @@ def prefill(
         first = parts[0]
         return PrefillResult(torch.cat([r.out for r in parts], dim=-1), first.node_src, first.node_w, first.plan,
                              first.feature_count, first.fsplit, first.den, first.moment_kernel)
+    pq, pk, pv = q3, k3, v3  # the caller's element type, for the pair kernel
     if semantics == "segment" and q3.dtype != torch.float32:
         # segment means are fp32 and the residual kernel reads them with the inputs in one format
         q3, k3, v3 = q3.float(), k3.float(), v3.float()
@@ -328,45 +354,55 @@ def prefill(
         return PrefillResult(_pairs(q3, k3, v3, scale, eps, out_dtype, timer), None, None, plan,
                              _plan.num_features(d, degree), 0)
 
-    # the moment kernel reads rows in 16-byte units: q/k padded with zero dimensions to a whole unit
-    # (zero dimensions only add zero-valued features), v to whole 32-column groups; keys wider than the
-    # 128 staged dimensions to whole 32-dimension window blocks
-    windowed = d > STAGED_D
-    dm = -(-d // _plan.WINDOW_BLOCK) * _plan.WINDOW_BLOCK if windowed else _unit_width(d, q3.element_size())
-    wt = _plan.window_tiles(dm, degree) if windowed else None
-    ft = _plan.window_feature_tiles(wt) if windowed else _plan.feature_tiles(dm, degree)
-    k1_products = MOMENT_PRODUCTS if products is None else int(products)
-    if degree >= 5:
-        k1_products = _native.PRODUCTS_FP32  # the degree 5 .. 8 scan runs fp32 products
-    qblock = ws_query_block(semantics, block) if (k1_products == _native.PRODUCTS_SPLIT_BF16 and degree <= 3 and
-                                                  not windowed and
-                                                  (use_moments_ws(q3.element_size(), degree) if moment_kernel is None
-                                                   else moment_kernel == "ws")) else None
-    ws_ct = 4 if (-(-dv // 32)) % 2 == 0 else 2
-    ws_opts = _native.moment_ws_slot_tiles(dm, degree, ws_ct, dv) if qblock else ()
-    nseg, seg_blocks = 1, 0
-    if ws_opts:
-        # few heads: cut each head's scan into segments of whole query blocks (sta_moments_ws_seg)
-        nseg, seg_blocks = _plan.ws_segments(n, shift, qblock, bh, ft, dv, ws_opts, ws_ct) if WS_SEGMENTS else (1, 0)
-        ms = _plan.moment_split_ws(ft, bh * nseg, dv, ws_opts, ws_ct)
-        chunk = qblock
-    elif windowed:
-        qblock = None
-        ms = _plan.moment_split_windows(wt, bh, dv, _native.moment_wave_tile_options(STAGED_D, degree))
+    # short sequences: the Taylor part over the pairs (sta_pair_moments)
+    pairs = (semantics in ("flat", "levels", "segment") and degree <= 3 and d <= FLASH_D and products is None and
+             (moment_kernel == "pairs" or (moment_kernel is None and use_pairs(n, d, dv, degree, pq.dtype))))
+    qblock = None
+    if pairs:
+        chunk = block if block % chunk == 0 else chunk
+        fsplit = pair_splits(bh, n, _compute_units(dev))
+        count, dm, dvm = _plan.num_features(d, degree), -(-d // 4) * 4, -(-dv // 4) * 4
     else:
-        qblock = None
-        ms = _plan.moment_split(ft, bh, dv, _native.moment_wave_tile_options(dm, degree),
-                                mixed_nts=_native.moment_mixed_tiles(dm, degree),
-                                wide_nts=_native.moment_wide_tiles(dm, degree, dv, k1_products) if MOMENT_WIDE else ())
-    fsplit = ms.fsplit
-    # split products at degree <= 2 apply one coefficient per tile on the query side
-    tile_coef = k1_products == _native.PRODUCTS_SPLIT_BF16 and degree <= 2
-    fidx, fcoef, fwin = _on_device(
-        ("mtable", dm, degree, bh, dv, ms.mixed, ms.wave_tiles, ms.fsplit, tile_coef, ms.columns, qblock is not None),
-        dev,
-        lambda: (_i32(ms.quads, dev),
-                 _f32(_plan.tile_coefficients(ms.quads, ms.coef, ft.d) if tile_coef else ms.coef, dev),
-                 _i32(ms.win, dev) if ms.win is not None else None))
+        # the moment kernel reads rows in 16-byte units: q/k padded with zero dimensions to a whole unit
+        # (zero dimensions only add zero-valued features), v to whole 32-column groups; keys wider than the
+        # 128 staged dimensions to whole 32-dimension window blocks
+        windowed = d > STAGED_D
+        dm = -(-d // _plan.WINDOW_BLOCK) * _plan.WINDOW_BLOCK if windowed else _unit_width(d, q3.element_size())
+        wt = _plan.window_tiles(dm, degree) if windowed else None
+        ft = _plan.window_feature_tiles(wt) if windowed else _plan.feature_tiles(dm, degree)
+        k1_products = MOMENT_PRODUCTS if products is None else int(products)
+        if degree >= 5:
+            k1_products = _native.PRODUCTS_FP32  # the degree 5 .. 8 scan runs fp32 products
+        qblock = ws_query_block(semantics, block) if (k1_products == _native.PRODUCTS_SPLIT_BF16 and degree <= 3 and
+                                                      not windowed and
+                                                      (use_moments_ws(q3.element_size(), degree) if moment_kernel is None
+                                                       else moment_kernel == "ws")) else None
+        ws_ct = 4 if (-(-dv // 32)) % 2 == 0 else 2
+        ws_opts = _native.moment_ws_slot_tiles(dm, degree, ws_ct, dv) if qblock else ()
+        nseg, seg_blocks = 1, 0
+        if ws_opts:
+            # few heads: cut each head's scan into segments of whole query blocks (sta_moments_ws_seg)
+            nseg, seg_blocks = _plan.ws_segments(n, shift, qblock, bh, ft, dv, ws_opts, ws_ct) if WS_SEGMENTS else (1, 0)
+            ms = _plan.moment_split_ws(ft, bh * nseg, dv, ws_opts, ws_ct)
+            chunk = qblock
+        elif windowed:
+            qblock = None
+            ms = _plan.moment_split_windows(wt, bh, dv, _native.moment_wave_tile_options(STAGED_D, degree))
+        else:
+            qblock = None
+            ms = _plan.moment_split(ft, bh, dv, _native.moment_wave_tile_options(dm, degree),
+                                    mixed_nts=_native.moment_mixed_tiles(dm, degree),
+                                    wide_nts=_native.moment_wide_tiles(dm, degree, dv, k1_products) if MOMENT_WIDE else ())
+        fsplit = ms.fsplit
+        # split products at degree <= 2 apply one coefficient per tile on the query side
+        tile_coef = k1_products == _native.PRODUCTS_SPLIT_BF16 and degree <= 2
+        fidx, fcoef, fwin = _on_device(
+            ("mtable", dm, degree, bh, dv, ms.mixed, ms.wave_tiles, ms.fsplit, tile_coef, ms.columns, qblock is not None),
+            dev,
+            lambda: (_i32(ms.quads, dev),
+                     _f32(_plan.tile_coefficients(ms.quads, ms.coef, ft.d) if tile_coef else ms.coef, dev),
+                     _i32(ms.win, dev) if ms.win is not None else None))
+        count, dvm = ft.count, -(-dv // 32) * 32
 
     # ---- host side first: every validation error is raised before anything is launched ----
     pkey = (plan.mode, plan.n, plan.block, compressor if semantics != "segment" else stride)
@@ -429,9 +465,20 @@ def prefill(
     low_num = torch.empty((bh, fsplit, lrows, lld), device=dev, dtype=torch.float32)
     low_den = torch.empty((bh, fsplit, lrows), device=dev, dtype=torch.float32)
 
-    mq, mk, mv = _padded_rows(q3, dm), _padded_rows(k3, dm), _padded_rows(v3, -(-dv // 32) * 32)
+    mq, mk, mv = _padded_rows(q3, dm), _padded_rows(k3, dm), _padded_rows(v3, dvm)
 
-    if qblock is not None:
+    if pairs:
+        if pq.dtype == q3.dtype:
+            pq, pk, pv = mq, mk, mv
+        else:
+            pq, pk, pv = _padded_rows(pq, dm), _padded_rows(pk, dm), _padded_rows(pv, dvm)
+
+        def k1():
+            st = lib.sta_pair_moments(
+                pq.data_ptr(), pk.data_ptr(), pv.data_ptr(), _native.DTYPE_CODES[pq.dtype], bh, n, d, dv, dm, dvm,
+                degree, float(scale), chunk, shift, fsplit, low_num.data_ptr(), low_den.data_ptr(), stream)
+            _native.check(st, "sta_pair_moments")
+    elif qblock is not None:
         hbytes = lib.sta_moments_ws_handoff_bytes(bh * nseg, fsplit, ms.wave_tiles, ws_ct, dv)
         handoff = torch.empty((max(hbytes, 16) // 4,), device=dev, dtype=torch.float32)
         seg_state = (torch.empty((lib.sta_moments_ws_seg_bytes(bh, fsplit, ms.wave_tiles, ws_ct, dv, nseg) // 4,),
@@ -557,7 +604,8 @@ def prefill(
         _native.check(st, "sta_block_attention")
 
     _run(timer, "block_attention", k24)
-    return PrefillResult(out, node_src, node_w, plan, ft.count, fsplit, out_den,
+    return PrefillResult(out, node_src, node_w, plan, count, fsplit, out_den,
+                         "flash_attn_kernel" if pairs else
                          "moments_ws_kernel" if qblock is not None else "moments_kernel")
 
 

@@ -94,6 +94,10 @@ _SIGNATURES = {
     "sta_exact_attention": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _c_p, _i32, _c_p],
     ),
+    "sta_pair_moments": (
+        _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _c_p, _c_p,
+               _c_p],  # q k v dtype bh n d dv ld_qk ld_v degree scale chunk shift nsplit num den stream
+    ),
     "sta_moment_accumulate_block": (
         _i32,
         [_c_p, _c_p, _i32, _i64, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _c_p, _c_p, _c_p, _i32, _c_p,

@@ -101,30 +101,45 @@ int dispatch_flash_dvt(const sta::FlashArgs& a, int weight, int64_t bh, hipStrea
   return STA_ERR_UNSUPPORTED;
 }
 
-// Argument checks and launch shared by sta_flash_attention and sta_exact_attention.
-int flash_launch(int weight, const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
-                 int dv, int ld_qk, int ld_v, float scale, float floor, void* out, int out_dtype, void* stream) {
-  if (!q || !k || !v || !out) return STA_ERR_ARG;
-  if (!dtype_ok(dtype) || !dtype_ok(out_dtype)) return STA_ERR_DTYPE;
+// Argument checks and arguments shared by the entry points of the pair kernel.
+int flash_args(sta::FlashArgs& a, const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+               int dv, int ld_qk, int ld_v) {
+  if (!q || !k || !v) return STA_ERR_ARG;
+  if (!dtype_ok(dtype)) return STA_ERR_DTYPE;
   if (bh <= 0 || n <= 0 || d <= 0 || dv <= 0) return STA_ERR_SHAPE;
   if (d > kMaxFlashD || dv > kMaxDv) return STA_ERR_UNSUPPORTED;
   if (ld_qk < d || ld_qk % 4 != 0 || ld_v < dv || ld_v % 4 != 0) return STA_ERR_ARG;
   if (((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) | reinterpret_cast<uintptr_t>(v)) & 15u) != 0)
     return STA_ERR_ARG;
   if (n >= (int64_t(1) << 31) - 128) return STA_ERR_UNSUPPORTED;
-  sta::FlashArgs a;
+  a = sta::FlashArgs{};
   a.q = q; a.k = k; a.v = v; a.dtype = dtype; a.n = n; a.d = d; a.dv = dv; a.ldqk = ld_qk; a.ldv = ld_v;
+  a.bh = bh; a.nsplit = 1;
+  return STA_OK;
+}
+
+int flash_dispatch(const sta::FlashArgs& a, int weight, void* stream) {
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool f32 = a.dtype == STA_F32;
+  const int64_t bh = a.bh;
+  if (a.d <= 16) return f32 ? dispatch_flash_dvt<16, 4>(a, weight, bh, s) : dispatch_flash_dvt<16, 2>(a, weight, bh, s);
+  if (a.d <= 32) return f32 ? dispatch_flash_dvt<32, 4>(a, weight, bh, s) : dispatch_flash_dvt<32, 2>(a, weight, bh, s);
+  if (a.d <= 64) return f32 ? dispatch_flash_dvt<64, 4>(a, weight, bh, s) : dispatch_flash_dvt<64, 2>(a, weight, bh, s);
+  return f32 ? dispatch_flash_dvt<128, 4>(a, weight, bh, s) : dispatch_flash_dvt<128, 2>(a, weight, bh, s);
+}
+
+int flash_launch(int weight, const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                 int dv, int ld_qk, int ld_v, float scale, float floor, void* out, int out_dtype, void* stream) {
+  sta::FlashArgs a;
+  if (!out) return STA_ERR_ARG;
+  if (!dtype_ok(out_dtype)) return STA_ERR_DTYPE;
+  if (const int st = flash_args(a, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v); st != STA_OK) return st;
   a.scale2 = scale * 1.4426950408889634f;
   a.n_tiles = static_cast<int>((n + sta::FLASH_ROWS - 1) / sta::FLASH_ROWS);
-  a.bh = bh; a.floor = floor;
+  a.floor = floor;
   a.out = out; a.out_dtype = out_dtype;
   a.vec_out = (out_dtype == STA_F32 && dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) ? 1 : 0;
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool f32 = dtype == STA_F32;
-  if (d <= 16) return f32 ? dispatch_flash_dvt<16, 4>(a, weight, bh, s) : dispatch_flash_dvt<16, 2>(a, weight, bh, s);
-  if (d <= 32) return f32 ? dispatch_flash_dvt<32, 4>(a, weight, bh, s) : dispatch_flash_dvt<32, 2>(a, weight, bh, s);
-  if (d <= 64) return f32 ? dispatch_flash_dvt<64, 4>(a, weight, bh, s) : dispatch_flash_dvt<64, 2>(a, weight, bh, s);
-  return f32 ? dispatch_flash_dvt<128, 4>(a, weight, bh, s) : dispatch_flash_dvt<128, 2>(a, weight, bh, s);
+  return flash_dispatch(a, weight, stream);
 }
 
 // Exclusive scan over the segments of each (head, feature split, column group): seg_state[p] <- sum of
@@ -183,6 +198,27 @@ int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, 
 int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream) {
   return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, stream);
+}
+
+int sta_pair_moments(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d, int dv,
+                     int ld_qk, int ld_v, int degree, float scale, int chunk, int shift, int nsplit, float* low_num,
+                     float* low_den, void* stream) {
+  sta::FlashArgs a;
+  if (!low_num || !low_den) return STA_ERR_ARG;
+  if (const int st = flash_args(a, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v); st != STA_OK) return st;
+  if (degree < 0 || degree > 3) return STA_ERR_UNSUPPORTED;
+  if (chunk <= 0 || shift < 0 || shift >= chunk || (reinterpret_cast<uintptr_t>(low_num) & 15u) != 0) return STA_ERR_ARG;
+  if (nsplit <= 0) return STA_ERR_SHAPE;
+  a.scale2 = scale;
+  const float x = dtype == STA_F32 ? 1.f : scale;  // fp32 queries are scaled, 16-bit products are not
+  a.c1 = degree >= 1 ? x : 0.f;
+  a.c2 = degree >= 2 ? x * x / 2.f : 0.f;
+  a.c3 = degree >= 3 ? x * x * x / 6.f : 0.f;
+  a.chunk = chunk; a.shift = shift; a.nsplit = nsplit;
+  a.n_tiles = static_cast<int>((n + shift + sta::FLASH_ROWS - 1) / sta::FLASH_ROWS);
+  a.low_num = low_num; a.low_den = low_den;
+  a.low_rows = n + 2 * sta::MOM_GUARD; a.low_ld = 32 * ((dv + 31) / 32); a.low_off = sta::MOM_GUARD;
+  return flash_dispatch(a, sta::FLASH_TAYLOR, stream);
 }
 
 int sta_tile_rows(void) { return kTileRows; }

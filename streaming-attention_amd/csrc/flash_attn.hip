@@ -1,5 +1,5 @@
-// Causal attention over pairs of contiguous rows, without coreset items: one kernel, three weights of a
-// pair (query row i, key j):
+// Causal attention over pairs of contiguous rows, without coreset items: one kernel, three weights of
+// a pair (query row i, key j):
 //   FLASH_SOFTMAX  exact causal softmax attention, the FlashAttention-style baseline of the reference's GPU
 //                  module (_flash_causal_kernel, triton_article_attention.py:372-435;
 //                  triton_flash_causal_attention :580-637):
@@ -7,6 +7,11 @@
 //                  m_i a running row maximum (online softmax)
 //   FLASH_EXP      compressor "none" (fast_article_attention.py:437-464, :596-598), where the Taylor part and the
 //                  residual add up to exp itself: out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum, eps)
+//   FLASH_TAYLOR   the Taylor part of a short sequence (degree <= 3; fast_article_attention.py:184-285): the partial sums
+//                  low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i in sta_moments' layout, c(i) the
+//                  start of the row's chunk, for sta_block_attention.  A pair costs 2 d + 2 (dv + 1) flop and a
+//                  token's moments 4 F (dv + 1), so the pairs are the cheaper way up to a few thousand tokens.
+//                  A tile's key batches can be dealt out to several workgroups (FlashArgs::nsplit).
 // fp32 accumulation, no N x N score matrix.
 //
 // Matrix-core layout (v_mfma_f32_16x16x32): X^T = K Q^T with A = key rows staged in LDS and B = the wave's
@@ -29,14 +34,15 @@
 // work of a pair (exponential, maximum, planes: 6 instructions).  1 x 8 heads x 8191 fp32, d = dv = 64: 397 us
 // = 174 TF/s (fp32 matrix instructions, unbalanced tiles: 857 us); 2 x 16 x 8192 bf16: 479 us = 579 TF/s
 // (710 us with a rescale and 12 more VALU instructions a pair); FLASH_EXP 4 x 8 x 2048 fp32: 102 us (513 us as
-// moment scan + residual kernel in fp32 products).
+// moment scan + residual kernel in fp32 products);
+// FLASH_TAYLOR 8 x 16 x 4096 bf16: 0.5 ms in the place of the moment scan's 1.06.
 #include <type_traits>
 
 #include "common.hpp"
 
 namespace sta {
 
-enum FlashWeight : int { FLASH_SOFTMAX = 0, FLASH_EXP = 1 };
+enum FlashWeight : int { FLASH_SOFTMAX = 0, FLASH_EXP = 1, FLASH_TAYLOR = 2 };
 
 struct FlashArgs {
   const void* q;
@@ -48,13 +54,23 @@ struct FlashArgs {
   int dv;
   int ldqk;      // row stride (elements) of q and k: a multiple of 4, >= d (columns >= d are ignored)
   int ldv;       // row stride of v: a multiple of 4, >= dv
-  float scale2;  // softmax scale times log2(e)
-  int n_tiles;   // ceil(n / FLASH_ROWS)
+  float scale2;  // softmax scale times log2(e); FLASH_TAYLOR: the scale
+  int n_tiles;   // ceil((n + shift) / FLASH_ROWS)
   int64_t bh;
   float floor;   // smallest denominator
   void* out;     // [BH][n][dv], dense
   int out_dtype;
   int vec_out;  // fp32 output, dv % 4 == 0 and 16-byte aligned: 16-byte stores
+  // key batches of a tile are dealt out to nsplit workgroups, each with sums of its own (1 but for FLASH_TAYLOR)
+  int nsplit;
+  // FLASH_TAYLOR: coefficients of x, x^2, x^3 (the logit, or q.k of 16-bit rows), the row chunk and its offset
+  // (c(i) = floor((i + shift) / chunk) chunk - shift; row tiles start at -shift), the partials
+  float c1, c2, c3;
+  int chunk, shift;
+  float* low_num;  // [BH][nsplit][low_rows][low_ld], row i at low_off + i
+  float* low_den;  // [BH][nsplit][low_rows]
+  int64_t low_rows;
+  int low_ld, low_off;
 };
 
 constexpr int FLASH_ROWS = 128;  // query rows of a workgroup: 4 waves x 2 strips of 16
@@ -62,9 +78,16 @@ constexpr int FLASH_ROWS = 128;  // query rows of a workgroup: 4 waves x 2 strip
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
 
 // Planes of the key / query rows, of the weights and of the values, and keys per LDS stage.
-__host__ __device__ constexpr int flash_kp(int in, int) { return in == F32 ? 3 : 1; }
-__host__ __device__ constexpr int flash_pp(int in, int w) { return (in == F32 || w == FLASH_EXP) ? 3 : 2; }
-__host__ __device__ constexpr int flash_vp(int in, int w) { return in == F32 ? 3 : (in == F16 && w == FLASH_EXP ? 2 : 1); }
+// FLASH_TAYLOR carries fp32 operands as two planes, as the moment scan does, and the weights as three: they are
+// near 1, so that two planes' error is 2^-17 of every value (2 x 8 x 3000 fp16 segment means: 4.0e-6 from
+// 64 bits in the whole result, against 3.5e-6 with the scan).
+__host__ __device__ constexpr int flash_kp(int in, int w) { return in != F32 ? 1 : (w == FLASH_TAYLOR ? 2 : 3); }
+__host__ __device__ constexpr int flash_pp(int in, int w) {
+  return (in == F32 || w != FLASH_SOFTMAX) ? 3 : 2;
+}
+__host__ __device__ constexpr int flash_vp(int in, int w) {
+  return in == F32 ? flash_kp(in, w) : (in == F16 && w != FLASH_SOFTMAX ? 2 : 1);
+}
 __host__ __device__ constexpr int flash_dps(int dp) { return dp < 32 ? 32 : dp; }
 __host__ __device__ constexpr int flash_stage_bytes(int dp, int dvt, int in, int w, int kb) {
   return 2 * (flash_kp(in, w) * kb * (flash_dps(dp) + 8) + flash_vp(in, w) * dvt * 16 * (kb + 8));
@@ -163,10 +186,10 @@ __device__ __forceinline__ uint4 load_buf(__amdgpu_buffer_rsrc_t r, int off) {
 // XCD (w % 8) share heads when the heads divide by 8.  When about two workgroups fit a compute unit at a
 // time the first two rounds are all there is, and plain descending order would give compute unit c the
 // c-th longest of both rounds (1.5x the mean for the first): the second round therefore ascends.
-__device__ __forceinline__ void flash_tile(const FlashArgs& a, int64_t& bh, int& t) {
+__device__ __forceinline__ void flash_tile(const FlashArgs& a, int64_t& bh, int& t, int& split) {
   const int total = gridDim.x, nbh = static_cast<int>(a.bh);
   const bool xcd = (nbh & 7) == 0;
-  const int hx = xcd ? nbh >> 3 : nbh;            // heads of this group of workgroups
+  const int hx = (xcd ? nbh >> 3 : nbh) * a.nsplit;  // (head, split)s of this group of workgroups
   const int j = xcd ? blockIdx.x >> 3 : blockIdx.x;
   const int count = xcd ? total >> 3 : total, round = xcd ? 32 : 256;
   int rank = j;
@@ -174,9 +197,10 @@ __device__ __forceinline__ void flash_tile(const FlashArgs& a, int64_t& bh, int&
     const int m = (count < 2 * round ? count : 2 * round) - round;
     if (j - round < m) rank = round + (m - 1 - (j - round));
   }
-  const int step = rank / hx, h = rank - step * hx;
+  const int step = rank / hx, hs = rank - step * hx, h = hs / a.nsplit;
+  split = hs - h * a.nsplit;
   t = a.n_tiles - 1 - step;
-  bh = xcd ? (blockIdx.x & 7) * hx + h : h;
+  bh = xcd ? (blockIdx.x & 7) * (nbh >> 3) + h : h;
 }
 
 // One workgroup per (head, tile of FLASH_ROWS query rows); wave w owns 2 strips of 16 rows.  Keys [0, last row
@@ -192,7 +216,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   constexpr int DPS = flash_dps(DP);  // dimensions in whole 32-element steps
   constexpr int MS = DPS / 32;
   constexpr int KP = flash_kp(IN, W), PP = flash_pp(IN, W), VP = flash_vp(IN, W);
-  constexpr int XORD = KP == 3 ? 2 : 0;  // plane products (i, j) with i + j <= order are taken
+  constexpr int XORD = KP - 1;  // plane products (i, j) with i + j <= order are taken
   constexpr int PORD = (PP > VP ? PP : VP) - 1;
   constexpr bool KF16 = IN == F16, PF16 = IN == F16 && W == FLASH_SOFTMAX;
   // denominators: a column of ones on the matrix cores where the weights' planes keep fp32 accuracy and the
@@ -213,29 +237,39 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   __shared__ uint4 stage4[(NST * STAGE + 7) / 8];
   uint16_t* const stage = reinterpret_cast<uint16_t*>(stage4);
 
+  constexpr bool TAYLOR = W == FLASH_TAYLOR;
   int64_t bh;
-  int t;
-  flash_tile(a, bh, t);
+  int t, split;
+  flash_tile(a, bh, t, split);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int n = static_cast<int>(a.n);
-  const int r0 = t * FLASH_ROWS;
+  const int r0 = t * FLASH_ROWS - (TAYLOR ? a.shift : 0);
   const int64_t qkbase = bh * a.n * a.ldqk;
   const int64_t vbase = bh * a.n * a.ldv;
 
+  // keys of a row: all up to its own, or those before its chunk
+  auto limit = [&](int row) -> int {
+    if constexpr (!TAYLOR) return row + 1;
+    const int c = (row + a.shift) / a.chunk * a.chunk - a.shift;  // row + shift >= 0
+    return c > 0 ? c : 0;
+  };
+
   // the wave's query rows as B operands (8 dimensions per lane and k-step), columns >= d zero.  fp32 rows
   // are scaled before they are split; 16-bit rows keep their exact values and the logits are scaled
-  // instead, by |scale| (its sign moves to the queries, so that the largest product is the largest logit).
-  int myrow[RS];
+  // instead, by |scale| (its sign moves to the queries, so that the largest product is the largest logit;
+  // FLASH_TAYLOR's coefficients hold the scale).
+  int myrow[RS], lim[RS];  // the row's keys are [0, lim)
   bool rvalid[RS];
   uint4 qB[RS][MS][KP];
-  const uint32_t flip = (IN != F32 && a.scale2 < 0.f) ? 0x80008000u : 0u;
+  const uint32_t flip = (!TAYLOR && IN != F32 && a.scale2 < 0.f) ? 0x80008000u : 0u;
   const float sc = IN == F32 ? 1.f : (a.scale2 < 0.f ? -a.scale2 : a.scale2);
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
     myrow[rs] = r0 + (wave * RS + rs) * 16 + li;
-    rvalid[rs] = myrow[rs] < n;
+    lim[rs] = limit(myrow[rs]);
+    rvalid[rs] = (!TAYLOR || myrow[rs] >= 0) && myrow[rs] < n;
     const int64_t qoff = qkbase + static_cast<int64_t>(rvalid[rs] ? myrow[rs] : 0) * a.ldqk;
 #pragma unroll
     for (int m = 0; m < MS; ++m) {
@@ -262,7 +296,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
       for (int i = 0; i < KP; ++i) qB[rs][m][i] = uint4{w[i][0], w[i][1], w[i][2], w[i][3]};
     }
   }
-  const int wrow_lo = r0 + wave * RS * 16, wrow_hi = wrow_lo + RS * 16 - 1;
+  const int wlim_lo = limit(r0 + wave * RS * 16), wlim_hi = limit(r0 + wave * RS * 16 + RS * 16 - 1);
 
   floatx4 num[RS][DVT], dacc[RS];
   float den[RS], mrow[RS];
@@ -320,7 +354,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
           for (int r = 0; r < 4; ++r) {
             float x = X[kt][rs][r];
             if constexpr (DIAG) {
-              if (off + 16 * kt + 4 * lg + r > myrow[rs]) x = -__builtin_huge_valf();
+              if (off + 16 * kt + 4 * lg + r >= lim[rs]) x = -__builtin_huge_valf();
             }
             float& mm = (r & 1) ? m1 : m0;
             mm = __builtin_amdgcn_fmed3f(mm, x, __builtin_huge_valf());  // max, without quieting its inputs
@@ -361,9 +395,9 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
               y = IN == F32 ? x - mrow[rs] : fmaf(x, sc, -mrow[rs]);
             else
               y = IN == F32 ? x : x * sc;
-            p[h] = __builtin_amdgcn_exp2f(y);
+            p[h] = TAYLOR ? fmaf(x, fmaf(x, fmaf(x, a.c3, a.c2), a.c1), 1.f) : __builtin_amdgcn_exp2f(y);
             if constexpr (DIAG) {
-              if (off + 16 * kt + 4 * lg + r > myrow[rs]) p[h] = 0.f;
+              if (off + 16 * kt + 4 * lg + r >= lim[rs]) p[h] = 0.f;
             }
             if constexpr (!DENM) den[rs] += p[h];
           }
@@ -405,8 +439,11 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   };
 
   const int row_hi = (r0 + FLASH_ROWS < n ? r0 + FLASH_ROWS : n) - 1;  // r0 < n: t < ceil(n / FLASH_ROWS)
-  const int kend = row_hi + 1;
-  const int nb = (kend + KB - 1) / KB;
+  const int kend = limit(row_hi);
+  const int step = TAYLOR ? a.nsplit : 1;  // this workgroup's batches: split, split + step, ...
+  const int nb_all = (kend + KB - 1) / KB;
+  const int nb = TAYLOR ? (nb_all - split + step - 1) / step : nb_all;
+  auto offset = [&](int b) { return (TAYLOR ? split + b * step : b) * KB; };
 
   // Staging registers: this thread's 4-element units of the next batch's rows, raw: key rows unit by unit,
   // value rows as blocks of 4 keys x 4 columns (the transposed write is then 8 bytes).  Offsets inside
@@ -498,24 +535,24 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
     __syncthreads();
   }
   auto compute = [&](int b, const uint16_t* st) {
-    const int off = b * KB;
-    if (off <= wrow_hi) {
-      if (off + KB - 1 > wrow_lo)
+    const int off = offset(b);
+    if (off < wlim_hi) {
+      if (off + KB > wlim_lo)
         process(std::true_type{}, off, st, st + KP * KPL);
       else
         process(std::false_type{}, off, st, st + KP * KPL);
     }
   };
-  prefetch(0);
+  if (!TAYLOR || nb > 0) prefetch(offset(0));
   if constexpr (NST == 2) {
-    commit(stage, stage + KP * KPL);
-    if (nb > 1) prefetch(KB);
+    if (!TAYLOR || nb > 0) commit(stage, stage + KP * KPL);
+    if (nb > 1) prefetch(offset(1));
     __syncthreads();
     for (int b = 0; b < nb; ++b) {
       compute(b, stage + (b & 1) * STAGE);
       // the other stage was read by batch b - 1, which every wave finished before the last barrier
       if (b + 1 < nb) commit(stage + ((b + 1) & 1) * STAGE, stage + ((b + 1) & 1) * STAGE + KP * KPL);
-      if (b + 2 < nb) prefetch((b + 2) * KB);
+      if (b + 2 < nb) prefetch(offset(b + 2));
       __syncthreads();
     }
   } else {
@@ -523,7 +560,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
       __syncthreads();  // every wave is done with the stage of the previous batch
       commit(stage, stage + KP * KPL);
       __syncthreads();  // staged batch visible
-      if (b + 1 < nb) prefetch((b + 1) * KB);
+      if (b + 1 < nb) prefetch(offset(b + 1));
       compute(b, stage);
     }
   }
@@ -540,6 +577,16 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
       dsum += __shfl_xor(dsum, 32);
     }
     if (!rvalid[rs]) continue;
+    if constexpr (TAYLOR) {
+      const int64_t row = (bh * a.nsplit + split) * a.low_rows + a.low_off + myrow[rs];
+      if (lg == 0) a.low_den[row] = dsum;
+#pragma unroll
+      for (int ct = 0; ct < DVT; ++ct) {
+        const int c0 = 16 * ct + 4 * lg;  // low_ld is whole 32-column groups
+        if (c0 < a.dv) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
+      }
+      continue;
+    }
     const float dn = fmaxf(dsum, a.floor);
     const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
 #pragma unroll

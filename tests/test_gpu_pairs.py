@@ -7,6 +7,8 @@ half a unit in the last of 8 (bf16) or 11 (fp16) bits at most, uniform, so 2^-8 
 import pytest
 import torch
 
+import _engine
+import _native
 import fast_article_attention as faa
 import triton_article_attention as taa
 
@@ -72,3 +74,32 @@ def test_pair_weights_and_the_smallest_denominator():
         out = taa.triton_flash_causal_attention(q.to(DEV, dtype), k.to(DEV, dtype), v.to(DEV, dtype), scale=0.0)
         mean = v.to(dtype).double().cumsum(2) / torch.arange(1, 71).reshape(-1, 1)
         assert rel(out, mean) < 4e-6
+
+
+# the Taylor part over pairs: chunks of a block (a multiple of 32) and of 32 rows, the level offset of one row,
+# row tiles and key batches with remainders, one and several workgroups a tile
+@pytest.mark.parametrize("bh,n,d,dv,degree,block", [
+    (1, 300, 16, 16, 2, 64), (3, 700, 40, 72, 1, 100), (2, 1153, 64, 64, 2, 128), (64, 385, 32, 32, 3, 96),
+    (1, 2049, 128, 128, 2, 256), (2, 260, 20, 200, 0, 50), (9, 513, 7, 30, 3, 37),
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("semantics", ["flat", "levels"])
+def test_taylor_pairs_match_the_moment_scan(bh, n, d, dv, degree, block, dtype, semantics):
+    """Same coreset items and residual, the Taylor part over the pairs or from the moments: each within 5e-6 of
+    the sums in 64 bits (split products), plus the rounding of 16-bit outputs."""
+    g = torch.Generator().manual_seed(n + d)
+    q, k, v = (torch.randn(bh, n, w, generator=g).mul_(s / w ** 0.5).to(dtype).to(DEV)
+               for w, s in ((d, 1.0), (d, 1.0), (dv, dv ** 0.5)))
+    print(bh, n, d, dv, degree, block, dtype, semantics, flush=True)
+    outs = [_engine.prefill(q, k, v, degree=degree, block=block, scale=-0.8, semantics=semantics, moment_kernel=mk,
+                            products=pr, out_dtype=torch.float32)
+            for mk, pr in (("pairs", None), ("chunked", _native.PRODUCTS_FP32))]
+    assert outs[0].moment_kernel == "flash_attn_kernel"
+    assert rel(outs[0].out, outs[1].out.cpu().double()) < 5e-6
+
+
+def test_pair_rule_and_splits():
+    assert _engine.use_pairs(1024, 32, 32, 2, torch.float32)
+    assert not _engine.use_pairs(65536, 64, 64, 2, torch.bfloat16)
+    assert _engine.pair_splits(1, 200, 256) == 1 and _engine.pair_splits(1, 4096, 256) == 8
+    assert _engine.pair_splits(64, 4096, 256) == 1
