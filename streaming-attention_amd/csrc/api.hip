@@ -810,6 +810,12 @@ int sta_block_attention(const void* q, const void* k, const void* v, int dtype, 
   a.node_w = node_w; a.rep_k = rep_k; a.rep_v = rep_v; a.n_rep = n_rep; a.out = out; a.out_dtype = out_dtype; a.out_den = out_den;
   a.ldqk = ld_qk; a.ldvr = ld_v; a.ldrk = ld_rep_k; a.ldrv = ld_rep_v;
   a.split = products == STA_PRODUCTS_SPLIT_BF16 ? 1 : 0;
+  a.vec_out = dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0 ? 1 : 0;
+  // a head's rows are addressed with 32-bit byte offsets (as in the moment scans)
+  const int64_t esize = dtype == STA_F32 ? 4 : 2;
+  const int64_t widest = std::max<int64_t>(n * std::max(ld_qk, ld_v) * esize,
+                                           rep_k ? n_rep * std::max(ld_rep_k, ld_rep_v) * 4 : 0);
+  if (widest > static_cast<int64_t>(sta::BLOCK_ABSENT) || n >= (int64_t(1) << 31) - 256) return STA_ERR_UNSUPPORTED;
   if (a.split && degree > 3) return STA_ERR_UNSUPPORTED;  // the split-product kernel's Taylor stops at 3
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool f32 = dtype == STA_F32;

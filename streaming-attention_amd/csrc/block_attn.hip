@@ -66,23 +66,42 @@ struct BlockArgs {
   void* out;  // [BH][n][dv]
   int out_dtype;
   float* out_den;  // optional [BH][n]: when set, out (fp32) receives num and out_den receives den, unnormalised
+  int vec_out;     // dv a multiple of 4 and out aligned to 4 elements: whole-unit stores
   int split;       // 1: split-bf16 matrix-core products (block_attn_kernel<..., true>)
 };
 
-__device__ __forceinline__ int64_t floordiv(int64_t a, int64_t b) {
-  const int64_t q = a / b;
-  return (a % b != 0 && ((a < 0) != (b < 0))) ? q - 1 : q;
+// Starts of a row's chunk and of its residual keys; i + shift >= 0 and, for MODE_LEVELS, i + 1 >= 0 (row tiles
+// start at -shift).
+__device__ __forceinline__ int chunk_start(int i, int chunk, int shift) {
+  return static_cast<int>(static_cast<uint32_t>(i + shift) / static_cast<uint32_t>(chunk)) * chunk - shift;
 }
 
-__device__ __forceinline__ int64_t chunk_start(int64_t i, int chunk, int shift) {
-  return floordiv(i + shift, chunk) * chunk - shift;
-}
-
-__device__ __forceinline__ int64_t residual_start(int64_t i, int mode, int block) {
-  if (mode == MODE_FLAT) return floordiv(i, block) * block;
-  if (mode == MODE_LEVELS) return floordiv(i + 1, block) * block;
-  if (mode == MODE_TAYLOR) return INT64_MAX;
+__device__ __forceinline__ int residual_start(int i, int mode, int block) {
+  const uint32_t b = static_cast<uint32_t>(block);
+  if (mode == MODE_FLAT) return static_cast<int>(static_cast<uint32_t>(i < 0 ? 0 : i) / b) * block;
+  if (mode == MODE_LEVELS) return static_cast<int>(static_cast<uint32_t>(i + 1) / b) * block;
+  if (mode == MODE_TAYLOR) return INT32_MAX;
   return 0;
+}
+
+// Buffer resource of `bytes` bytes at p: loads beyond it return zero (BLOCK_ABSENT marks absent rows: the
+// host keeps a head's rows within it).
+constexpr uint32_t BLOCK_ABSENT = 0xfffffff0u;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t block_rsrc(const void* p, int64_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, static_cast<int>(static_cast<uint32_t>(bytes)),
+                                           0x00020000);
+}
+template <int ES>
+__device__ __forceinline__ uint4 load_row_unit(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
+  if constexpr (ES == 4) {
+    const u4 x = __builtin_bit_cast(u4, __builtin_amdgcn_raw_buffer_load_b128(r, static_cast<int>(off), 0, 0));
+    return uint4{x.x, x.y, x.z, x.w};
+  } else {
+    const u2 x = __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(r, static_cast<int>(off), 0, 0));
+    return uint4{x.x, x.y, 0u, 0u};
+  }
 }
 
 // The logits come out in base 2: the staged queries carry scale * log2(e), so y = x log2(e) for the
@@ -129,10 +148,11 @@ constexpr float LOG2E = 1.44269504f;
 constexpr int BA_LIST = 1024;
 __host__ __device__ constexpr int block_kb(int dp, int dvt) { return (dp + dvt * 16 > 192) ? 32 : 64; }
 __host__ __device__ constexpr int block_kpt(int dp, int dvt) { return (block_kb(dp, dvt) * dp / 4 + 255) / 256; }
-__host__ __device__ constexpr int block_vpt(int dp, int dvt) { return (block_kb(dp, dvt) * dvt * 4 + 255) / 256; }
+// value units: blocks of 4 keys x 4 columns
+__host__ __device__ constexpr int block_vpt(int dp, int dvt) { return (block_kb(dp, dvt) * dvt + 255) / 256; }
 __host__ __device__ constexpr int block_occupancy(int dp, int dvt, int rs) {
   return (rs * dp / 4 + rs * dvt * 4 + 2 * rs * (block_kb(dp, dvt) / 16) * 4 +
-          4 * (block_kpt(dp, dvt) + block_vpt(dp, dvt))) <= 160
+          4 * (block_kpt(dp, dvt) + 4 * block_vpt(dp, dvt))) <= 160
              ? 2
              : 1;
 }
@@ -170,19 +190,20 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   constexpr int LDVB = KB + 8;
   static_assert(!SPLIT || NSUB % 2 == 0, "split products pair the 16-key subtiles");
   constexpr int F32_WORDS = KB * LDK + DV * LDVT;
-  constexpr int SPLIT_WORDS = KB * LDKB + DV * LDVB;  // two bf16 planes each
+  constexpr int SPLIT_WORDS = (KB * LDKB + DV * LDVB) / (KVX ? 2 : 1);  // two bf16 planes each (KVX: one)
   constexpr int STAGE_WORDS = SPLIT ? SPLIT_WORDS : F32_WORDS;
   __shared__ floatx4 stage4[(STAGE_WORDS + 3) / 4];
   float* const Kst = reinterpret_cast<float*>(stage4);
   float* const Vt = Kst + KB * LDK;
   __bf16* const Kh = reinterpret_cast<__bf16*>(stage4);
-  __bf16* const Kl = Kh + KB * LDKB;
+  __bf16* const Kl = KVX ? Kh : Kh + KB * LDKB;
   __bf16* const Vh = Kl + KB * LDKB;
-  __bf16* const Vl = Vh + DV * LDVB;
+  __bf16* const Vl = KVX ? Vh : Vh + DV * LDVB;
   __shared__ float Wst[KB];
   __shared__ int Jst[KB];
   __shared__ int Lost[KB], Hist[KB];  // active rows of the staged items (node batches)
-  __shared__ int Lj[BA_LIST], Llo[BA_LIST], Lhi[BA_LIST];
+  __shared__ __align__(16) int Lj[BA_LIST];  // token (materialized row) of an item, -1: none
+  __shared__ int Llo[BA_LIST], Lhi[BA_LIST];
   __shared__ float Lw[BA_LIST];
 
   const int wg = xcd_remap(blockIdx.x, gridDim.x);
@@ -195,7 +216,6 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   const int r0 = t * TM - a.shift;
 
   const int64_t qkbase = bh * a.n * a.ldqk;
-  const int64_t vbase = bh * a.n * a.ldvr;
 
   int rbase[RS], myrow[RS], csr[RS], rsr[RS];
   bool rvalid[RS];
@@ -206,9 +226,8 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     rbase[rs] = r0 + (wave * RS + rs) * 16;
     myrow[rs] = rbase[rs] + li;
     rvalid[rs] = myrow[rs] >= 0 && myrow[rs] < n;
-    csr[rs] = static_cast<int>(chunk_start(myrow[rs], a.chunk, a.shift));
-    const int64_t rsv = residual_start(myrow[rs], a.mode, a.block);
-    rsr[rs] = rsv > INT32_MAX ? INT32_MAX : static_cast<int>(rsv);
+    csr[rs] = chunk_start(myrow[rs], a.chunk, a.shift);
+    rsr[rs] = residual_start(myrow[rs], a.mode, a.block);
     const int64_t qoff = qkbase + static_cast<int64_t>(rvalid[rs] ? myrow[rs] : 0) * a.ldqk;
     const float qs = rvalid[rs] ? a.scale * LOG2E : 0.f;  // the logits come out scaled, in base 2
     if constexpr (SPLIT) {
@@ -262,27 +281,33 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // on every row of the tile (the test is skipped), 3 as 2 for degree <= 2 without the exp clamp: the
   // Horner form stops at y^2 and the logit is not clamped (the same values for every finite logit:
   // with k3 = 0 the third fused multiply-add returns k2 exactly, and min(y, inf) = y), two VALU
-  // instructions fewer per (row, item) pair on the most frequent batch kind
-  auto process = [&](auto node_tag) {
-    constexpr bool NODE = decltype(node_tag)::value != 0;
-    constexpr bool FULL = decltype(node_tag)::value >= 2;
-    constexpr bool FAST = decltype(node_tag)::value == 3;
+  // instructions fewer per (row, item) pair on the most frequent batch kind, 4 and 5 own keys [off, off + KB)
+  // that lie in the chunk and in the residual of every row of the tile, where the two parts add up to
+  // exp (the usual in-block batch), with the causal test and, where no row precedes a key, without
+  auto process = [&](auto node_tag, int off) {
+    constexpr int KIND = decltype(node_tag)::value;
+    constexpr bool EXPO = KIND >= 4;
+    constexpr bool NODE = KIND >= 1 && KIND <= 3;
+    constexpr bool FULL = KIND == 2 || KIND == 3;
+    constexpr bool FAST = KIND == 3;
     // weights of subtile kt from its logits X (key 16 kt + 4 lg + r, row myrow[rs]), elementwise
     auto weights = [&](int kt, const floatx4 (&X)[RS], floatx4 (&P)[RS]) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int kidx = 16 * kt + 4 * lg + r;
-        const int j = Jst[kidx];
-        const float w = Wst[kidx];
+        const int j = EXPO ? off + kidx : (NODE ? 0 : Jst[kidx]);
+        const float w = NODE ? Wst[kidx] : 1.f;
         const int lo = NODE ? Lost[kidx] : 0, hi = NODE ? Hist[kidx] : 0;
 #pragma unroll
         for (int rs = 0; rs < RS; ++rs) {
           const int i = myrow[rs];
           const float yv = X[rs][r];
           const float ex = __builtin_amdgcn_exp2f(FAST ? yv : fminf(yv, ymax));
-          const float tp = FAST ? fmaf(yv, fmaf(yv, tc.k2, tc.k1), 1.0f) : taylor2<!SPLIT, HD>(yv, tc);
+          const float tp = EXPO ? 0.f : FAST ? fmaf(yv, fmaf(yv, tc.k2, tc.k1), 1.0f) : taylor2<!SPLIT, HD>(yv, tc);
           float p;
-          if constexpr (FULL) {
+          if constexpr (EXPO) {
+            p = KIND == 5 || j <= i ? ex : 0.f;
+          } else if constexpr (FULL) {
             p = (ex - tp) * w;  // rows outside the sequence have zero queries and are never stored
           } else if constexpr (NODE) {
             const bool on = rvalid[rs] && i >= lo && i <= hi;
@@ -427,12 +452,15 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   using node_batch = std::integral_constant<int, 1>;
   using node_batch_full = std::integral_constant<int, 2>;
   using node_batch_full_fast = std::integral_constant<int, 3>;
+  using exp_batch_causal = std::integral_constant<int, 4>;
+  using exp_batch = std::integral_constant<int, 5>;
   const bool fast = !a.exp_clamp && a.degree <= 2;
 
   // ---- batch sequence: phase A = contiguous keys [kstart, kend), phase B = the node item list ----
-  int kstart = static_cast<int>(chunk_start(row_lo, a.chunk, a.shift));
-  const int64_t rs_lo = residual_start(row_lo, a.mode, a.block);
-  if (rs_lo < kstart) kstart = static_cast<int>(rs_lo);
+  int kstart = chunk_start(row_lo, a.chunk, a.shift);
+  const int rs_lo = residual_start(row_lo, a.mode, a.block);
+  if (rs_lo < kstart) kstart = rs_lo;
+  const int exp_from = max(chunk_start(row_hi, a.chunk, a.shift), residual_start(row_hi, a.mode, a.block));
   if (kstart < 0) kstart = 0;
   const int kend = row_hi + 1;
   const int n_a = kend > kstart ? (kend - kstart + KB - 1) / KB : 0;
@@ -463,157 +491,121 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
         i_cur = 0;
       }
     }
+    for (int e = llen + tid; e < (llen + KB - 1) / KB * KB; e += 256) {  // the last batch's absent items
+      Lj[e] = -1;
+      Lw[e] = 0.f;
+      Llo[e] = 0;
+      Lhi[e] = -1;
+    }
   };
 
-  // prefetch registers: this thread's 4-element units of the next batch's key and value rows, raw (they
-  // are converted when written to LDS, so no instruction waits on the loads before the next commit),
-  // and which of them are real (row of the batch, column inside the row)
-  constexpr int KU = DP / 4, VU = DV / 4;
+  // prefetch registers: this thread's 4-element units of the next batch's rows, raw (they are converted
+  // when written to LDS, so no instruction waits on the loads before the next commit): key rows unit by unit,
+  // value rows as blocks of 4 keys x 4 columns, so that the transposed write is one word per column and
+  // plane.  Absent rows and columns load from beyond the buffer, which reads as zero.
+  constexpr int KU = DP / 4, VU = DV / 4, KG = KB / 4;
   constexpr int KPT = block_kpt(DP, DVT), VPT = block_vpt(DP, DVT);
-  // value units in key pairs (split products, an even count of units per thread covering the batch
-  // exactly): units 2 k and 2 k + 1 of a thread are keys 2 rp and 2 rp + 1 of one column unit, which sit
-  // next to each other in the value planes (split_key_pos), so the commit splits them as packed pairs
-  // and writes 32-bit words; otherwise key-fast single units
-  constexpr bool VPAIR = SPLIT && VPT % 2 == 0 && KB * VU == 256 * VPT;
-  auto vunit = [&](int i, int& r, int& u) -> bool {
-    if constexpr (VPAIR) {
-      const int pe = tid + 256 * (i >> 1);
-      r = 2 * (pe % (KB / 2)) + (i & 1);
-      u = pe / (KB / 2);
-      return true;
-    } else {
-      const int e = tid + 256 * i;
-      r = e % KB;  // key-fast: conflict-light transposed writes
-      u = e / KB;
-      return e < KB * VU;
-    }
-  };
-  uint4 pk[KPT], pv[VPT];
-  uint32_t pk_ok = 0, pv_ok = 0;
+  static_assert(256 % KU == 0, "a thread's key units share one column");
+  uint4 pk[KPT], pv[VPT][4];
   int pj = -1, plo = 0, phi = -1;
   float pw = 0.f;
-  auto src_of = [&](bool node, int off, int r) -> int {
-    if (!node) return off + r < kend ? off + r : -1;
-    return off + r < llen ? Lj[off + r] : -1;
-  };
+  const int ku = tid % KU, kr0 = tid / KU;
   auto prefetch = [&](bool node, int off) {
     // in-block keys come from k / v; node items from rep_k / rep_v in segment mode (fp32, ES == 4 there)
-    const bool from_rep = mat && node;
-    const void* kb = a.k;
-    const void* vb = a.v;
-    int64_t kbase = qkbase, vbase2 = vbase;
-    int ldk = a.ldqk, ldv = a.ldvr;
-    if constexpr (ES == 4) {
-      if (from_rep) {
-        kb = a.rep_k;
-        vb = a.rep_v;
-        kbase = bh * a.n_rep * a.ldrk;
-        vbase2 = bh * a.n_rep * a.ldrv;
-        ldk = a.ldrk;
-        ldv = a.ldrv;
-      }
-    }
-    pk_ok = pv_ok = 0;
+    const bool from_rep = ES == 4 && mat && node;
+    const int ldk = from_rep ? a.ldrk : a.ldqk, ldv = from_rep ? a.ldrv : a.ldvr;
+    const int64_t rows = from_rep ? a.n_rep : a.n;
+    const char* const kb = static_cast<const char*>(from_rep ? static_cast<const void*>(a.rep_k) : a.k);
+    const char* const vb = static_cast<const char*>(from_rep ? static_cast<const void*>(a.rep_v) : a.v);
+    const __amdgpu_buffer_rsrc_t kr = block_rsrc(kb + bh * rows * ldk * ES, rows * ldk * ES);
+    const __amdgpu_buffer_rsrc_t vr = block_rsrc(vb + bh * rows * ldv * ES, rows * ldv * ES);
+    const uint32_t kst = static_cast<uint32_t>(ldk * ES), vst = static_cast<uint32_t>(ldv * ES);
+    const bool kcol = 4 * ku < ldk;
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      const int r = e / KU, u = e - r * KU;
-      const int src = (e < KB * KU) ? src_of(node, off, r) : -1;
-      const bool ok = src >= 0 && 4 * u < ldk;
-      pk_ok |= ok ? (1u << i) : 0u;
-      pk[i] = load_unit<ES>(kb, kbase + static_cast<int64_t>(src >= 0 ? src : 0) * ldk + min(4 * u, ldk - 4));
+      const int r = kr0 + i * (256 / KU);
+      int src = -1;
+      if (KB * KU % 256 == 0 || r < KB) src = node ? Lj[off + r] : (off + r < kend ? off + r : -1);
+      pk[i] = load_row_unit<ES>(kr, src >= 0 && kcol ? static_cast<uint32_t>(src) * kst + 4 * ES * ku : BLOCK_ABSENT);
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      int r, u;
-      const bool in = vunit(i, r, u);
-      const int src = in ? src_of(node, off, r) : -1;
-      const bool ok = src >= 0 && 4 * u < ldv;
-      pv_ok |= ok ? (1u << i) : 0u;
-      pv[i] = load_unit<ES>(vb, vbase2 + static_cast<int64_t>(src >= 0 ? src : 0) * ldv + min(4 * u, ldv - 4));
+      const int e = tid + 256 * i, g = e % KG, u = e / KG;  // key-fast: conflict-light transposed writes
+      const bool in = (KG * VU % 256 == 0 || e < KG * VU) && 4 * u < ldv;
+      int4 src = int4{-1, -1, -1, -1};
+      if (in) {
+        if (node) {
+          src = *reinterpret_cast<const int4*>(Lj + off + 4 * g);
+        } else {
+          const int j = off + 4 * g;
+          src = int4{j < kend ? j : -1, j + 1 < kend ? j + 1 : -1, j + 2 < kend ? j + 2 : -1, j + 3 < kend ? j + 3 : -1};
+        }
+      }
+      const int sv[4] = {src.x, src.y, src.z, src.w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        pv[i][c] = load_row_unit<ES>(vr, sv[c] >= 0 ? static_cast<uint32_t>(sv[c]) * vst + 4 * ES * u : BLOCK_ABSENT);
     }
     if (tid < KB) {
-      pj = src_of(node, off, tid);
-      const bool in = node && off + tid < llen;
-      pw = in ? Lw[off + tid] : (node ? 0.f : 1.f);
-      plo = in ? Llo[off + tid] : 0;
-      phi = in ? Lhi[off + tid] : -1;
+      pj = node ? Lj[off + tid] : (off + tid < kend ? off + tid : -1);
+      pw = node ? Lw[off + tid] : 1.f;
+      plo = node ? Llo[off + tid] : 0;
+      phi = node ? Lhi[off + tid] : -1;
     }
   };
   bool item_full = true;
   auto commit = [&]() {
-    if constexpr (SPLIT) {
-      // bf16 hi / lo planes; keys row-major (dimension 4 u..4 u+3 of key r: 8 bytes per plane), values
-      // transposed with each subtile pair's keys in contraction order (split_key_pos)
-#pragma unroll
-      for (int i = 0; i < KPT; ++i) {
-        const int e = tid + 256 * i;
-        if (e < KB * KU) {
-          const int r = e / KU, u = e - r * KU;
-          const floatx4 f = unit_to_f4<ES>(pk[i], a.dtype, ((pk_ok >> i) & 1u) ? 1.f : 0.f);
-          uint32_t h0, h1, l0, l1;
-          split_pair(f[0], f[1], h0, l0);
-          split_pair(f[2], f[3], h1, l1);
-          *reinterpret_cast<uint2*>(Kh + r * LDKB + 4 * u) = uint2{h0, h1};
-          if constexpr (!KVX) *reinterpret_cast<uint2*>(Kl + r * LDKB + 4 * u) = uint2{l0, l1};
-        }
-      }
-      if constexpr (VPAIR) {
-#pragma unroll
-        for (int k = 0; k < VPT / 2; ++k) {
-          int r, u;
-          vunit(2 * k, r, u);
-          const floatx4 f0 = unit_to_f4<ES>(pv[2 * k], a.dtype, ((pv_ok >> (2 * k)) & 1u) ? 1.f : 0.f);
-          const floatx4 f1 = unit_to_f4<ES>(pv[2 * k + 1], a.dtype, ((pv_ok >> (2 * k + 1)) & 1u) ? 1.f : 0.f);
-          const int pos = split_key_pos(r);  // even: key r + 1 at pos + 1
-#pragma unroll
-          for (int m = 0; m < 4; ++m) {
-            uint32_t h, l;
-            if constexpr (KVX) {
-              h = pk_bf16(f0[m], f1[m]);  // exact bf16 values: the lo plane is zero and not kept
-            } else {
-              split_pair(f0[m], f1[m], h, l);
-              *reinterpret_cast<uint32_t*>(Vl + (4 * u + m) * LDVB + pos) = l;
-            }
-            *reinterpret_cast<uint32_t*>(Vh + (4 * u + m) * LDVB + pos) = h;
-          }
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < VPT; ++i) {
-          int r, u;
-          if (vunit(i, r, u)) {
-            const floatx4 f = unit_to_f4<ES>(pv[i], a.dtype, ((pv_ok >> i) & 1u) ? 1.f : 0.f);
-            const int pos = split_key_pos(r);
-#pragma unroll
-            for (int m = 0; m < 4; ++m) {
-              const __bf16 h = static_cast<__bf16>(f[m]);
-              Vh[(4 * u + m) * LDVB + pos] = h;
-              if constexpr (!KVX) Vl[(4 * u + m) * LDVB + pos] = static_cast<__bf16>(f[m] - static_cast<float>(h));
-            }
-          }
-        }
-      }
-    } else {
 #pragma unroll
     for (int i = 0; i < KPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * KU) {
-        const int r = e / KU, u = e - r * KU;
-        *reinterpret_cast<floatx4*>(Kst + r * LDK + 4 * u) =
-            unit_to_f4<ES>(pk[i], a.dtype, ((pk_ok >> i) & 1u) ? 1.f : 0.f);
+      const int r = kr0 + i * (256 / KU);
+      if (KB * KU % 256 != 0 && r >= KB) continue;
+      if constexpr (KVX) {  // bf16 rows as they are
+        *reinterpret_cast<uint2*>(Kh + r * LDKB + 4 * ku) = uint2{pk[i].x, pk[i].y};
+      } else if constexpr (SPLIT) {
+        const floatx4 f = unit_to_f4<ES>(pk[i], a.dtype, 1.f);
+        uint32_t h0, h1, l0, l1;
+        split_pair(f[0], f[1], h0, l0);
+        split_pair(f[2], f[3], h1, l1);
+        *reinterpret_cast<uint2*>(Kh + r * LDKB + 4 * ku) = uint2{h0, h1};
+        *reinterpret_cast<uint2*>(Kl + r * LDKB + 4 * ku) = uint2{l0, l1};
+      } else {
+        *reinterpret_cast<floatx4*>(Kst + r * LDK + 4 * ku) = unit_to_f4<ES>(pk[i], a.dtype, 1.f);
       }
     }
 #pragma unroll
     for (int i = 0; i < VPT; ++i) {
-      const int e = tid + 256 * i;
-      if (e < KB * VU) {
-        const int r = e % KB, u = e / KB;
-        const floatx4 f = unit_to_f4<ES>(pv[i], a.dtype, ((pv_ok >> i) & 1u) ? 1.f : 0.f);
+      const int e = tid + 256 * i, g = e % KG, u = e / KG;
+      if (KG * VU % 256 != 0 && e >= KG * VU) continue;
+      if constexpr (KVX) {
+        // 16-bit 4 x 4 transpose: column m of the 4 keys
+        __bf16* const dst = Vh + 4 * u * LDVB + split_key_pos(4 * g);
 #pragma unroll
-        for (int m = 0; m < 4; ++m) Vt[(4 * u + m) * LDVT + r] = f[m];
+        for (int m = 0; m < 4; ++m) {
+          const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
+          const uint32_t k0 = m < 2 ? pv[i][0].x : pv[i][0].y, k1 = m < 2 ? pv[i][1].x : pv[i][1].y;
+          const uint32_t k2 = m < 2 ? pv[i][2].x : pv[i][2].y, k3 = m < 2 ? pv[i][3].x : pv[i][3].y;
+          *reinterpret_cast<uint2*>(dst + m * LDVB) =
+              uint2{__builtin_amdgcn_perm(k1, k0, sel), __builtin_amdgcn_perm(k3, k2, sel)};
+        }
+      } else {
+        floatx4 f[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) f[c] = unit_to_f4<ES>(pv[i][c], a.dtype, 1.f);
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          if constexpr (SPLIT) {
+            // each subtile pair's keys in contraction order (split_key_pos)
+            const int dst = (4 * u + m) * LDVB + split_key_pos(4 * g);
+            uint32_t h0, h1, l0, l1;
+            split_pair(f[0][m], f[1][m], h0, l0);
+            split_pair(f[2][m], f[3][m], h1, l1);
+            *reinterpret_cast<uint2*>(Vh + dst) = uint2{h0, h1};
+            *reinterpret_cast<uint2*>(Vl + dst) = uint2{l0, l1};
+          } else {
+            *reinterpret_cast<floatx4*>(Vt + (4 * u + m) * LDVT + 4 * g) = floatx4{f[0][m], f[1][m], f[2][m], f[3][m]};
+          }
+        }
       }
-    }
     }
     if (tid < KB) {
       Jst[tid] = pj;
@@ -629,7 +621,7 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // list is read only by prefetch(); once a batch is committed its items live in Jst/Wst/Lost/Hist, so
   // the list can be refilled right after the commit of its last batch.
   if constexpr (SPLIT && DPS != DP) {  // dimensions [DP, DPS) of the key planes are never written: zero
-    for (int e = tid; e < KB * LDKB; e += 256) Kh[e] = Kl[e] = static_cast<__bf16>(0.f);
+    for (int e = tid; e < KB * LDKB; e += 256) Kh[e] = Kl[e] = static_cast<__bf16>(0.f);  // (KVX: one plane)
   }
   // Moment partials: a.fsplit partial sums per row (the feature splits of the moment scan), RS * fsplit
   // (strip, split) pairs per lane.  Pair p = RS f + rs is loaded during batch p (issued after the next
@@ -716,13 +708,19 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     const bool pair = PAIR_OVERLAP && pairs_done < n_pairs;
     if (pair) pair_load(pairs_done);
     if (cur_node && full && fast)
-      process(node_batch_full_fast{});
+      process(node_batch_full_fast{}, cur_off);
     else if (cur_node && full)
-      process(node_batch_full{});
+      process(node_batch_full{}, cur_off);
     else if (cur_node)
-      process(node_batch{});
-    else if (cur_off <= wrow_hi)
-      process(block_batch{});  // some key of the batch precedes some row of this wave
+      process(node_batch{}, cur_off);
+    else if (cur_off <= wrow_hi) {  // some key of the batch precedes some row of this wave
+      if (cur_off < exp_from)
+        process(block_batch{}, cur_off);
+      else if (cur_off + KB - 1 > wrow_lo)
+        process(exp_batch_causal{}, cur_off);
+      else
+        process(exp_batch{}, cur_off);
+    }
     if (pair) pair_add(pairs_done++);
     cur_node = nxt_node;
     cur_off = nxt_off;
@@ -771,16 +769,30 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     for (int ct = 0; ct < DVT; ++ct) {
       const int c0 = 16 * ct + 4 * lg;
       if (c0 >= a.dv) continue;
+      const int64_t o0 = (bh * a.n + i) * a.dv + c0;
+      floatx4 o = num[rs][ct];
+      if (!raw) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int col = c0 + r;
-        if (col < a.dv) {
-          const float numv = num[rs][ct][r];
-          if (raw)
-            static_cast<float*>(a.out)[(bh * a.n + i) * a.dv + col] = numv;
-          else
-            store_elem(a.out, (bh * a.n + i) * a.dv + col, a.out_dtype, numv / dn);
+        for (int r = 0; r < 4; ++r) o[r] = o[r] / dn;
+      }
+      if (a.vec_out) {  // whole units: dv a multiple of 4 and the output aligned
+        if (a.out_dtype == F32) {
+          *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + o0) = o;
+        } else {
+          uint2 h;
+          if (a.out_dtype == BF16) {
+            h = uint2{pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3])};
+          } else {
+            typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
+            h.x = __builtin_bit_cast(uint32_t, halfx2{static_cast<_Float16>(o[0]), static_cast<_Float16>(o[1])});
+            h.y = __builtin_bit_cast(uint32_t, halfx2{static_cast<_Float16>(o[2]), static_cast<_Float16>(o[3])});
+          }
+          *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + o0) = h;
         }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c0 + r < a.dv) store_elem(a.out, o0 + r, a.out_dtype, o[r]);
       }
     }
   }

@@ -220,8 +220,9 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   constexpr int PORD = (PP > VP ? PP : VP) - 1;
   constexpr bool KF16 = IN == F16, PF16 = IN == F16 && W == FLASH_SOFTMAX;
   // denominators: a column of ones on the matrix cores where the weights' planes keep fp32 accuracy and the
-  // matrix cores have room (16-bit inputs), else fp32 VALU sums
-  constexpr bool DENM = IN != F32 && PP == 3;
+  // matrix cores have room (16-bit inputs; FLASH_TAYLOR of every type, so that 16-bit rows and their fp32
+  // values give the same sums), else fp32 VALU sums
+  constexpr bool DENM = (IN != F32 || W == FLASH_TAYLOR) && PP == 3;
   // how far (log2) a row may exceed its running maximum before the sums are rescaled; two-plane weights keep
   // the latest maximum, whose own weight 1 is then exact (bf16, 32 heads x 8192: error against 64 bits 1.9e-6
   // and 479 us, with 8 here 2.1e-6 and 450 us)

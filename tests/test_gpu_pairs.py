@@ -103,3 +103,21 @@ def test_pair_rule_and_splits():
     assert not _engine.use_pairs(65536, 64, 64, 2, torch.bfloat16)
     assert _engine.pair_splits(1, 200, 256) == 1 and _engine.pair_splits(1, 4096, 256) == 8
     assert _engine.pair_splits(64, 4096, 256) == 1
+
+
+@pytest.mark.parametrize("n,d,dv,dtype", [(1, 64, 64, torch.float32), (127, 16, 30, torch.float16),
+                                          (193, 40, 72, torch.bfloat16), (320, 128, 128, torch.float32)])
+@pytest.mark.parametrize("products", ["fp32", "split"])
+@pytest.mark.parametrize("semantics", ["flat", "levels"])
+def test_residual_kernel_inside_one_block(n, d, dv, dtype, products, semantics):
+    """Own keys of the residual kernel only (the chunks of 32 rows of the moment scan make the batches in which
+    the Taylor part, the residual or both apply): exact attention, to 2e-6 in fp32 products, 1e-5 in split
+    products (2^-16 a product), plus the rounding of 16-bit outputs in whole and in partial units."""
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(2, n, w, generator=g).to(dtype) for w in (d, d, dv))
+    pr = _native.PRODUCTS_FP32 if products == "fp32" else _native.PRODUCTS_SPLIT_BF16
+    print(n, d, dv, dtype, products, semantics, flush=True)
+    out = _engine.prefill(q.to(DEV), k.to(DEV), v.to(DEV), degree=2, block=512, scale=0.2, semantics=semantics,
+                          products=pr, residual_products=pr, out_dtype=dtype).out
+    ref = exact(q, k, v, 0.2, 1e-12)
+    assert rel(out, ref) < TOL[dtype] + (2e-6 if products == "fp32" else 1e-5)
