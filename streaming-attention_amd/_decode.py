@@ -329,16 +329,39 @@ class DecodeState:
         self.buf_k, self.buf_v, self.cap = bk, bv, new_cap
 
     # ------------------------------------------------------------------ draws
-    def _draw_completion(self, blocks_before: int) -> _CompletionDraws:
-        sizes = _plan.completion_call_sizes(blocks_before, self.block, self.compressor)
-        n_calls = len(sizes)
+    def _draw_completions(self, first: int, count: int) -> List[_CompletionDraws]:
+        """The draws of the block completions first, ..., first + count - 1: one pass over the generators and
+        one upload for all of them."""
+        sizes = [_plan.completion_call_sizes(b, self.block, self.compressor) for b in range(first, first + count)]
         max_in = max(self.block, 2 * self.m)
-        methods = [_plan._call_method(n_in, self.compressor) for n_in in sizes]
-        dirs, unif, perms = self._gens.next(sizes, self.d, self.compressor, max_in, f64=self.score_f64)
-        dev = self.device
-        return _CompletionDraws(
-            blocks_before, n_calls, torch.tensor(methods, dtype=torch.int32).to(dev), torch.from_numpy(dirs).to(dev),
-            torch.from_numpy(unif).to(dev), torch.from_numpy(perms).to(dev))
+        methods = [[_plan._call_method(n_in, self.compressor) for n_in in sz] for sz in sizes]
+        dirs, unif, perms = self._gens.next([n for sz in sizes for n in sz], self.d, self.compressor, max_in,
+                                            f64=self.score_f64)
+        # tables are [S, calls of the completion, .]; permutations only where a call reads them
+        perm = any(m == _plan.METHOD_PERM for ms in methods for m in ms)
+        parts, at, spans, c0 = [], 0, [], 0
+        for ms in methods:
+            c1 = c0 + len(ms)
+            row = [np.asarray(ms, dtype=np.int32), dirs[:, c0:c1], unif[:, c0:c1]] + ([perms[:, c0:c1]] if perm else [])
+            for x in row:
+                raw = np.ascontiguousarray(x).reshape(-1).view(np.uint8)
+                pad = -raw.size % 16
+                parts.append(raw)
+                if pad:
+                    parts.append(np.zeros(pad, np.uint8))
+                spans.append((at, raw.size, x.shape))
+                at += raw.size + pad
+            c0 = c1
+        flat = torch.from_numpy(np.concatenate(parts)).to(self.device)
+        real = torch.float64 if self.score_f64 else torch.float32
+        views = [flat[o: o + n].view(t).view(shape) for (o, n, shape), t in
+                 zip(spans, ([torch.int32, real, real] + ([torch.int32] if perm else [])) * count)]
+        out, per = [], 4 if perm else 3
+        for i, ms in enumerate(methods):
+            v = views[per * i: per * i + per]
+            pm = v[3] if perm else torch.zeros((self.S, len(ms), max_in), device=self.device, dtype=torch.int32)
+            out.append(_CompletionDraws(first + i, len(ms), v[0], v[1], v[2], pm))
+        return out
 
     def reserve_draws(self, tokens: int) -> int:
         """Draw ahead, on the host, the compress calls of every block completion within the next
@@ -347,8 +370,11 @@ class DecodeState:
             return 0
         queued_to = self.blocks + len(self._draws)
         last = (self.length + tokens) // self.block
-        for c in range(queued_to, last):
-            self._draws.append(self._draw_completion(c))
+        # about 64 MiB of tables at a time
+        per = self.S * (2 * self.d + 3 * self.block) * 4 * (2 if self.score_f64 else 1)
+        group = max(1, (64 << 20) // per)
+        for c in range(queued_to, last, group):
+            self._draws.extend(self._draw_completions(c, min(group, last - c)))
         return len(self._draws)
 
     def _take_draws(self) -> _CompletionDraws:
@@ -356,7 +382,7 @@ class DecodeState:
             dr = self._draws.popleft()
             assert dr.blocks_before == self.blocks
             return dr
-        return self._draw_completion(self.blocks)
+        return self._draw_completions(self.blocks, 1)[0]
 
     # ------------------------------------------------------------------ block completion
     def _complete_block(self, accumulate: bool = True) -> None:
@@ -546,8 +572,8 @@ class DecodeState:
             n = hi - lo
             while self.exact and self.buf_len + n > self.cap:
                 self._grow_buffer()
-            self.buf_k[:, self.buf_len: self.buf_len + n, : self.d] = k[:, lo:hi].float()
-            self.buf_v[:, self.buf_len: self.buf_len + n, : self.dv] = v[:, lo:hi].float()
+            self.buf_k[:, self.buf_len: self.buf_len + n, : self.d] = k[:, lo:hi]
+            self.buf_v[:, self.buf_len: self.buf_len + n, : self.dv] = v[:, lo:hi]
             if self.score_f64:
                 self._put_k64(k64[:, lo:hi], self.buf_len, self.buf_len + n)
             self.buf_len += n
@@ -583,6 +609,8 @@ class DecodeState:
                 vp[:, koff: koff + hi - lo, : self.dv] = v[:, lo:hi]
             self._accumulate(kp, vp, hi - lo, kp.shape[1], self.state_num, self.state_den, row_off=koff)
             for b in range(nb):
+                if not self._draws:  # the draws of the next blocks, at most 64 ahead
+                    self.reserve_draws(min(nb - b, 64) * self.block)
                 to_buffer(lo + b * self.block, lo + (b + 1) * self.block)
                 self._complete_block(accumulate=False)
             i = hi

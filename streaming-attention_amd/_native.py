@@ -364,7 +364,8 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
 
 
 def stream_handle(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The device's current stream, without a Stream object (4 us of a small call's host time)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)
 
 
 _wave_tile_options: dict = {}
