@@ -575,16 +575,20 @@ int sta_decode_tail(const void* q, const void* k, const void* v, int dtype, int6
   hipStream_t s = static_cast<hipStream_t>(stream);
   const int kc = d <= 64 ? 1 : (d <= 128 ? 2 : 4);
   const int vc = dv <= 64 ? 1 : (dv <= 128 ? 2 : 4);
-  const dim3 blk(sta::DEC_THREADS);
-  if (kc == 1 && vc == 1) hipLaunchKernelGGL((sta::decode_tail_kernel<1, 1>), grid, blk, 0, s, a);
-  else if (kc == 1 && vc == 2) hipLaunchKernelGGL((sta::decode_tail_kernel<1, 2>), grid, blk, 0, s, a);
-  else if (kc == 1) hipLaunchKernelGGL((sta::decode_tail_kernel<1, 4>), grid, blk, 0, s, a);
-  else if (kc == 2 && vc == 1) hipLaunchKernelGGL((sta::decode_tail_kernel<2, 1>), grid, blk, 0, s, a);
-  else if (kc == 2 && vc == 2) hipLaunchKernelGGL((sta::decode_tail_kernel<2, 2>), grid, blk, 0, s, a);
-  else if (kc == 2) hipLaunchKernelGGL((sta::decode_tail_kernel<2, 4>), grid, blk, 0, s, a);
-  else if (vc == 1) hipLaunchKernelGGL((sta::decode_tail_kernel<4, 1>), grid, blk, 0, s, a);
-  else if (vc == 2) hipLaunchKernelGGL((sta::decode_tail_kernel<4, 2>), grid, blk, 0, s, a);
-  else hipLaunchKernelGGL((sta::decode_tail_kernel<4, 4>), grid, blk, 0, s, a);
+  // the wide workgroup for queries of few streams (at most one a compute unit)
+  const bool wide = (flags & sta::DEC_QUERY) && streams <= 256;
+#define STA_TAIL(KC, VC)                                                                                            \
+  if (kc == KC && vc == VC) {                                                                                       \
+    if (wide)                                                                                                       \
+      hipLaunchKernelGGL((sta::decode_tail_kernel<KC, VC, sta::DEC_TAIL_WIDE>), grid, dim3(sta::DEC_TAIL_WIDE), 0,  \
+                         s, a);                                                                                     \
+    else                                                                                                            \
+      hipLaunchKernelGGL((sta::decode_tail_kernel<KC, VC, sta::DEC_THREADS>), grid, dim3(sta::DEC_THREADS), 0, s, a); \
+  }
+  STA_TAIL(1, 1) STA_TAIL(1, 2) STA_TAIL(1, 4)
+  STA_TAIL(2, 1) STA_TAIL(2, 2) STA_TAIL(2, 4)
+  STA_TAIL(4, 1) STA_TAIL(4, 2) STA_TAIL(4, 4)
+#undef STA_TAIL
   return check_launch();
 }
 

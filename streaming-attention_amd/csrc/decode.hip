@@ -27,7 +27,11 @@
 namespace sta {
 
 constexpr int DEC_THREADS = 256;
-constexpr int DEC_GROUPS = DEC_THREADS / 16;  // items in flight per workgroup pass (16 lanes per item)
+// decode_tail_kernel's workgroup: 256 threads, or 512 where the streams are at most the compute units: the time
+// is then the chain of one stream's loads (items of the buffer and of each level one after the other, and the
+// moment partials), which one list of all items with twice as many in flight shortens (1 stream, d = dv = 64, 3
+// occupied levels of 64: 12.7 -> 5.6 us; 1024 threads have too few registers for 4 items each).
+constexpr int DEC_TAIL_WIDE = 512;
 constexpr int DEC_MAX_X = 260;                // staged query features x[0..d] (d <= 256) plus zeros
 
 enum DecFlags : int { DEC_APPEND = 1, DEC_CURRENT = 2, DEC_QUERY = 4 };
@@ -228,19 +232,22 @@ __device__ __forceinline__ float dec_exp(float z) { return __builtin_amdgcn_exp2
 // Items per 16-lane group in flight: NB rows are loaded before any of them is used.
 constexpr int DEC_NB = 4;
 
-template <int KC, int VC>
-__global__ __launch_bounds__(DEC_THREADS) void decode_tail_kernel(const DecTailArgs a) {
+template <int KC, int VC, int T>
+__global__ __launch_bounds__(T) void decode_tail_kernel(const DecTailArgs a) {
+  constexpr int DEC_GROUPS = T / 16;  // items in flight per workgroup pass (16 lanes per item)
+  constexpr bool WIDE = T > DEC_THREADS;
   __shared__ float xs[DEC_MAX_X];
   __shared__ float cur_k[DEC_MAX_X];
   __shared__ float cur_v[4 * 16 * VC];
   __shared__ float redv[DEC_GROUPS][4 * 16 * VC];
-  __shared__ float redd[DEC_GROUPS][2];
+  __shared__ float redd[DEC_GROUPS][WIDE ? 3 : 2];
+  __shared__ int occ[64];
   const int64_t s = blockIdx.x;
   const int tid = threadIdx.x;
   const int dk4 = a.dk >> 2, dv4 = a.ldv >> 2;
 
   if (a.flags & (DEC_APPEND | DEC_CURRENT)) {
-    for (int j = tid; j < a.dk + a.ldv; j += DEC_THREADS) {
+    for (int j = tid; j < a.dk + a.ldv; j += T) {
       if (j < a.dk) {
         const float x = j < a.d ? load_elem(a.k, s * a.d + j, a.dtype) : 0.f;
         cur_k[j] = x;
@@ -254,8 +261,11 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_tail_kernel(const DecTailA
     }
   }
   if (!(a.flags & DEC_QUERY)) return;
-  for (int j = tid; j < DEC_MAX_X; j += DEC_THREADS)
+  for (int j = tid; j < DEC_MAX_X; j += T)
     xs[j] = j < a.d ? a.scale * load_elem(a.q, s * a.d + j, a.dtype) : 0.f;
+  if constexpr (WIDE) {
+    if (tid < 64 && ((a.level_mask >> tid) & 1u)) occ[__popcll(a.level_mask & ((uint64_t(1) << tid) - 1))] = tid;
+  }
   __syncthreads();
 
   const int c = tid & 15, g = tid >> 4;
@@ -271,25 +281,103 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_tail_kernel(const DecTailA
   float den = 0.f, tay = 0.f;  // tay: Taylor part of the buffered tokens (reference low denominator)
 
   const DecTaylor tc = dec_taylor(a.degree);
-  // buffered tokens: exact exponential, weight 1 (DEC_NB items per group in flight)
+  float low = 0.f;  // WIDE: this group's share of the moment partials' denominators
+  int n_items = a.buf_len + ((a.flags & DEC_CURRENT) ? 1 : 0);
   const float* bk = a.buf_k + s * a.B * a.dk;
   const float* bv = a.buf_v + s * a.B * a.ldv;
-  for (int j0 = g; j0 < a.buf_len; j0 += DEC_NB * DEC_GROUPS) {
-    DecItem<KC, VC> it[DEC_NB];
+  if constexpr (WIDE) {
+    // moment partials: split j is one more row of group j % DEC_GROUPS, in flight with the items
+    for (int j = g; j < a.splits; j += DEC_GROUPS) {
+      const float* pn = a.part_num + (s * a.splits + j) * a.ldv;
+      low += a.part_den[s * a.splits + j];
 #pragma unroll
-    for (int b = 0; b < DEC_NB; ++b) {
-      const int jb = min(j0 + b * DEC_GROUPS, a.buf_len - 1);
-      dec_load_item<KC, VC>(it[b], bk + jb * a.dk, bv + jb * a.ldv, c, dk4, dv4);
+      for (int u = 0; u < VC; ++u)
+        if (c + 16 * u < dv4) acc[u] += *reinterpret_cast<const floatx4*>(pn + 4 * (c + 16 * u));
     }
+    // buffered tokens, then the occupied levels' items, as one list: occ[i] is the i-th occupied level
+    const int n_occ = __popcll(a.level_mask);
+    const int total = a.buf_len + n_occ * a.m;
+    n_items += n_occ * a.m;
+    for (int j0 = g; j0 < total; j0 += DEC_NB * DEC_GROUPS) {
+      DecItem<KC, VC> it[DEC_NB];
+      float w[DEC_NB];
 #pragma unroll
-    for (int b = 0; b < DEC_NB; ++b) {
-      const float z = dec_dot<KC>(x, it[b].k);
-      const bool on = j0 + b * DEC_GROUPS < a.buf_len;
-      const float p = on ? dec_exp(z) : 0.f;
-      den += p;
-      tay += on ? dec_tp(z, tc) : 0.f;
+      for (int b = 0; b < DEC_NB; ++b) {
+        const int jb = min(j0 + b * DEC_GROUPS, total - 1);
+        const float *kr, *vr, *wr = nullptr;
+        if (jb < a.buf_len) {
+          kr = bk + jb * a.dk;
+          vr = bv + jb * a.ldv;
+        } else {
+          const int o = (jb - a.buf_len) / a.m;
+          const int64_t row = (s * a.L + occ[o]) * a.m + (jb - a.buf_len - o * a.m);
+          kr = a.lev_k + row * a.dk;
+          vr = a.lev_v + row * a.ldv;
+          wr = a.lev_w + row;
+        }
+        dec_load_item<KC, VC>(it[b], kr, vr, c, dk4, dv4);
+        w[b] = wr ? *wr : 0.f;
+      }
 #pragma unroll
-      for (int j = 0; j < VC; ++j) acc[j] += p * it[b].v[j];
+      for (int b = 0; b < DEC_NB; ++b) {
+        const int jb = j0 + b * DEC_GROUPS;
+        const float z = dec_dot<KC>(x, it[b].k);
+        const float ex = dec_exp(z), tp = dec_tp(z, tc);
+        const bool buffered = jb < a.buf_len, on = jb < total;
+        const float p = !on ? 0.f : buffered ? ex : w[b] * (ex - tp);
+        den += p;
+        tay += on && buffered ? tp : 0.f;
+#pragma unroll
+        for (int j = 0; j < VC; ++j) acc[j] += p * it[b].v[j];
+      }
+    }
+  } else {
+    // buffered tokens: exact exponential, weight 1 (DEC_NB items per group in flight)
+    for (int j0 = g; j0 < a.buf_len; j0 += DEC_NB * DEC_GROUPS) {
+      DecItem<KC, VC> it[DEC_NB];
+#pragma unroll
+      for (int b = 0; b < DEC_NB; ++b) {
+        const int jb = min(j0 + b * DEC_GROUPS, a.buf_len - 1);
+        dec_load_item<KC, VC>(it[b], bk + jb * a.dk, bv + jb * a.ldv, c, dk4, dv4);
+      }
+#pragma unroll
+      for (int b = 0; b < DEC_NB; ++b) {
+        const float z = dec_dot<KC>(x, it[b].k);
+        const bool on = j0 + b * DEC_GROUPS < a.buf_len;
+        const float p = on ? dec_exp(z) : 0.f;
+        den += p;
+        tay += on ? dec_tp(z, tc) : 0.f;
+#pragma unroll
+        for (int j = 0; j < VC; ++j) acc[j] += p * it[b].v[j];
+      }
+    }
+    // level items: weighted exp_{>t} residual
+    for (int l = 0; l < a.L; ++l) {
+      if (!((a.level_mask >> l) & 1u)) continue;
+      n_items += a.m;
+      const int64_t base = (s * a.L + l) * a.m;
+      const float* lk = a.lev_k + base * a.dk;
+      const float* lv = a.lev_v + base * a.ldv;
+      const float* lw = a.lev_w + base;
+      for (int j0 = g; j0 < a.m; j0 += DEC_NB * DEC_GROUPS) {
+        DecItem<KC, VC> it[DEC_NB];
+        float w[DEC_NB];
+#pragma unroll
+        for (int b = 0; b < DEC_NB; ++b) {
+          const int jb = min(j0 + b * DEC_GROUPS, a.m - 1);
+          dec_load_item<KC, VC>(it[b], lk + jb * a.dk, lv + jb * a.ldv, c, dk4, dv4);
+          w[b] = lw[jb];
+        }
+#pragma unroll
+        for (int b = 0; b < DEC_NB; ++b) {
+          const float z = dec_dot<KC>(x, it[b].k);
+          const bool on = j0 + b * DEC_GROUPS < a.m;
+          const float r = on ? w[b] * (dec_exp(z) - dec_tp(z, tc)) : 0.f;
+          den += r;
+#pragma unroll
+          for (int j = 0; j < VC; ++j) acc[j] += r * it[b].v[j];
+        }
+      }
     }
   }
   // the current token of this launch (group 0)
@@ -303,42 +391,13 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_tail_kernel(const DecTailA
 #pragma unroll
     for (int j = 0; j < VC; ++j) acc[j] += p * it.v[j];
   }
-  // level items: weighted exp_{>t} residual
-  int n_items = a.buf_len + ((a.flags & DEC_CURRENT) ? 1 : 0);
-  for (int l = 0; l < a.L; ++l) {
-    if (!((a.level_mask >> l) & 1u)) continue;
-    n_items += a.m;
-    const int64_t base = (s * a.L + l) * a.m;
-    const float* lk = a.lev_k + base * a.dk;
-    const float* lv = a.lev_v + base * a.ldv;
-    const float* lw = a.lev_w + base;
-    for (int j0 = g; j0 < a.m; j0 += DEC_NB * DEC_GROUPS) {
-      DecItem<KC, VC> it[DEC_NB];
-      float w[DEC_NB];
-#pragma unroll
-      for (int b = 0; b < DEC_NB; ++b) {
-        const int jb = min(j0 + b * DEC_GROUPS, a.m - 1);
-        dec_load_item<KC, VC>(it[b], lk + jb * a.dk, lv + jb * a.ldv, c, dk4, dv4);
-        w[b] = lw[jb];
-      }
-#pragma unroll
-      for (int b = 0; b < DEC_NB; ++b) {
-        const float z = dec_dot<KC>(x, it[b].k);
-        const bool on = j0 + b * DEC_GROUPS < a.m;
-        const float r = on ? w[b] * (dec_exp(z) - dec_tp(z, tc)) : 0.f;
-        den += r;
-#pragma unroll
-        for (int j = 0; j < VC; ++j) acc[j] += r * it[b].v[j];
-      }
-    }
-  }
-
   // ---- fixed-order combination: groups, then moment partials ----
 #pragma unroll
   for (int j = 0; j < VC; ++j) *reinterpret_cast<floatx4*>(&redv[g][4 * (c + 16 * j)]) = acc[j];
   if (c == 0) {
     redd[g][0] = den;
     redd[g][1] = tay;
+    if constexpr (WIDE) redd[g][2] = low;
   }
   __syncthreads();
   float tail_den = 0.f, buf_tay = 0.f;
@@ -347,12 +406,17 @@ __global__ __launch_bounds__(DEC_THREADS) void decode_tail_kernel(const DecTailA
     buf_tay += redd[j][1];
   }
   float low_den = 0.f;
-  for (int j = 0; j < a.splits; ++j) low_den += a.part_den[s * a.splits + j];
+  if constexpr (WIDE) {
+    for (int j = 0; j < DEC_GROUPS; ++j) low_den += redd[j][2];
+  } else {
+    for (int j = 0; j < a.splits; ++j) low_den += a.part_den[s * a.splits + j];
+  }
   const float total = low_den + tail_den;
   const float safe = fmaxf(total, a.eps);
-  for (int col = tid; col < a.dv; col += DEC_THREADS) {
+  for (int col = tid; col < a.dv; col += T) {
     float num = 0.f;
-    for (int j = 0; j < a.splits; ++j) num += a.part_num[(s * a.splits + j) * a.ldv + col];
+    if constexpr (!WIDE)
+      for (int j = 0; j < a.splits; ++j) num += a.part_num[(s * a.splits + j) * a.ldv + col];
     for (int j = 0; j < DEC_GROUPS; ++j) num += redv[j][col];
     store_elem(a.out, s * a.dv + col, a.out_dtype, __fdiv_rn(num, safe));
   }

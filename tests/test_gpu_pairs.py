@@ -10,6 +10,7 @@ import torch
 import _engine
 import _native
 import fast_article_attention as faa
+import streaming_taylor_coreset_attention as stc
 import triton_article_attention as taa
 
 pytestmark = pytest.mark.gpu
@@ -121,3 +122,24 @@ def test_residual_kernel_inside_one_block(n, d, dv, dtype, products, semantics):
                           products=pr, residual_products=pr, out_dtype=dtype).out
     ref = exact(q, k, v, 0.2, 1e-12)
     assert rel(out, ref) < TOL[dtype] + (2e-6 if products == "fp32" else 1e-5)
+
+
+@pytest.mark.parametrize("d,dv,block,tokens", [(64, 64, 16, 39), (40, 200, 8, 64), (130, 72, 6, 25), (16, 16, 300, 290)])
+@pytest.mark.parametrize("fused", [True, False])
+def test_few_streams_tail_matches_many(d, dv, block, tokens, fused):
+    """The wide decode tail (up to 256 streams) against the same tokens among 257 streams: fp32 sums in another
+    order (a few 2^-23)."""
+    g = torch.Generator().manual_seed(d)
+    q, k, v = (torch.randn(tokens, 257, w, generator=g).mul_(0.3).to(DEV) for w in (d, d, dv))
+    outs = []
+    for s in (2, 257):
+        att = stc.ArticleStreamingAttention(d, dv, degree=2, block_size=block, streams=s)
+        rows = []
+        for t in range(tokens):
+            if fused:
+                rows.append(att.step(q[t, :s], k[t, :s], v[t, :s])[:2])
+            else:
+                att.update(k[t, :s], v[t, :s])
+                rows.append(att.query(q[t, :s])[:2])
+        outs.append(torch.stack(rows))
+    assert rel(outs[0], outs[1].cpu().double()) < 2e-6
