@@ -395,6 +395,20 @@ int sta_block_attention(const void* q, const void* k, const void* v, int dtype, 
                         float* out_den, void* stream);
 
 /*
+ * sta_block_attention with a tile's key and item batches dealt out to ksplit (1 .. 16) workgroups, for grids that
+ * leave compute units idle: their raw sums go to part_num [ksplit][BH][N][4 ceil(Dv / 4)] (16-byte aligned) and
+ * part_den [ksplit][BH][N], and a second launch adds and normalises them.  out_den must be NULL when ksplit > 1.
+ */
+int sta_block_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                              int dv, int ld_qk, int ld_v, int degree, float scale, float eps, int mode, int block,
+                              int chunk, int shift, int exp_clamp, int products, const float* low_num,
+                              const float* low_den, int fsplit, const int32_t* tile_ptr, const int32_t* tile_nodes,
+                              int n_tiles, const int32_t* node_meta, int n_nodes, int cap, const int32_t* node_src,
+                              const float* node_w, const float* rep_k, const float* rep_v, int ld_rep_k, int ld_rep_v,
+                              int64_t n_rep, void* out, int out_dtype, float* out_den, int ksplit, float* part_num,
+                              float* part_den, void* stream);
+
+/*
  * Exact causal softmax attention, FlashAttention-style (online row maximum, no N x N scores).
  * Replaces _flash_causal_kernel / triton_flash_causal_attention (triton_article_attention.py:372-435,
  * :580-637):  out_i = sum_{j<=i} exp(s q_i.k_j - m_i) v_j / max(sum_{j<=i} exp(s q_i.k_j - m_i), 1e-20).

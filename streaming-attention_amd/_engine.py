@@ -133,6 +133,22 @@ def pair_splits(bh: int, n: int, compute_units: int) -> int:
     return max(1, min(2 * compute_units // tiles, n // 256, 8))
 
 
+def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, compute_units: int) -> int:
+    """Workgroups that share a tile of the residual kernel (sta_block_attention_split), width = d + dv: two
+    workgroups a compute unit where the tiles alone are fewer (1 x 4096 fp32, d = dv = 64: kernel 116 -> 39 us with
+    8, 4 x 2048 bf16: 54 -> 33), two a tile up to three tiles for two units (16 x 3000 fp32, 384 tiles: 104 -> 93;
+    440 tiles: 74 -> 86 and left alone), none where the longest tile is so short that the second launch costs
+    the host more (1 x 1024, d = dv = 32: a pass 61 -> 65 us)."""
+    tiles = bh * plan.n_tiles
+    most = int(np.diff(plan.tile_ptr).max()) * plan.cap + min(block, plan.n)  # items and keys of the longest tile
+    if most * width < 40000:
+        return 1
+    want = 2 * compute_units // tiles
+    if want < 2:
+        want = 2 if 2 * tiles <= 3 * compute_units else 1
+    return max(1, min(want, most // 128, 8))
+
+
 # Offer the planner the 64-column moment workgroups (split products, 32 < dv <= 64).  Off: on 32 heads x
 # 65536 tokens (d = dv = 64) they take 9.6 ms against 8.4 ms for two 32-column workgroups per compute
 # unit; the feature work they save (17 % of the VALU) is less than one wave per SIMD loses in latency.
@@ -592,16 +608,22 @@ def prefill(
     else:
         k2_products = RESIDUAL_PRODUCTS
 
+    ksplit = 1 if raw else residual_splits(bh, plan, block, d + dv, _compute_units(dev))
+    part_num = part_den = None
+    if ksplit > 1:
+        part_num = torch.empty((ksplit, bh, n, -(-dv // 4) * 4), device=dev, dtype=torch.float32)
+        part_den = torch.empty((ksplit, bh, n), device=dev, dtype=torch.float32)
+
     def k24():
-        st = lib.sta_block_attention(
+        st = lib.sta_block_attention_split(
             mq.data_ptr(), mk.data_ptr(), mv.data_ptr(), dt, bh, n, d, dv, dm, mv.shape[-1], degree, float(scale),
             float(eps), mode, block, chunk, shift, 1 if exp_clamp else 0,
             k2_products, low_num.data_ptr(), low_den.data_ptr(),
             fsplit, tptr_d.data_ptr(), tnodes_d.data_ptr(), plan.n_tiles, meta_d.data_ptr(), n_nodes_arg, plan.cap,
             _native.ptr(node_src), _native.ptr(node_w), _native.ptr(rep_k), _native.ptr(rep_v),
             rep_k.shape[-1] if rep_k is not None else 0, rep_v.shape[-1] if rep_v is not None else 0, n_rep_arg,
-            out.data_ptr(), odt, _native.ptr(out_den), stream)
-        _native.check(st, "sta_block_attention")
+            out.data_ptr(), odt, _native.ptr(out_den), ksplit, _native.ptr(part_num), _native.ptr(part_den), stream)
+        _native.check(st, "sta_block_attention_split")
 
     _run(timer, "block_attention", k24)
     return PrefillResult(out, node_src, node_w, plan, count, fsplit, out_den,

@@ -777,13 +777,13 @@ int sta_segment_mean(const void* k, const void* v, int dtype, int64_t bh, int64_
   return check_launch();
 }
 
-int sta_block_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+int sta_block_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, int degree, float scale, float eps, int mode, int block, int chunk,
                         int shift, int exp_clamp, int products, const float* low_num, const float* low_den, int fsplit,
                         const int32_t* tile_ptr, const int32_t* tile_nodes, int n_tiles, const int32_t* node_meta,
                         int n_nodes, int cap, const int32_t* node_src, const float* node_w, const float* rep_k,
                         const float* rep_v, int ld_rep_k, int ld_rep_v, int64_t n_rep, void* out, int out_dtype,
-                        float* out_den, void* stream) {
+                        float* out_den, int ksplit, float* part_num, float* part_den, void* stream) {
   if (!q || !k || !v || !low_num || !low_den || !tile_ptr || !out) return STA_ERR_ARG;
   if (out_den && out_dtype != STA_F32) return STA_ERR_DTYPE;
   if (!dtype_ok(dtype) || !dtype_ok(out_dtype)) return STA_ERR_DTYPE;
@@ -805,7 +805,11 @@ int sta_block_attention(const void* q, const void* k, const void* v, int dtype, 
     if (((reinterpret_cast<uintptr_t>(rep_k) | reinterpret_cast<uintptr_t>(rep_v)) & 15u) != 0) return STA_ERR_ARG;
     if (dtype != STA_F32) return STA_ERR_DTYPE;
   }
+  if (ksplit < 1 || ksplit > sta::BA_MAX_SPLIT) return STA_ERR_SHAPE;
+  if (ksplit > 1 && (!part_num || !part_den || out_den || (reinterpret_cast<uintptr_t>(part_num) & 15u) != 0))
+    return STA_ERR_ARG;
   sta::BlockArgs a;
+  a.ksplit = ksplit; a.part_num = part_num; a.part_den = part_den; a.ldp = (dv + 3) / 4 * 4;
   a.q = q; a.k = k; a.v = v; a.dtype = dtype; a.n = n; a.d = d; a.dv = dv; a.degree = degree; a.scale = scale;
   a.eps = eps; a.mode = mode; a.block = block; a.chunk = chunk; a.shift = shift; a.exp_clamp = exp_clamp;
   a.low_num = low_num; a.low_den = low_den; a.fsplit = fsplit; a.tile_ptr = tile_ptr; a.tile_nodes = tile_nodes;
@@ -823,11 +827,30 @@ int sta_block_attention(const void* q, const void* k, const void* v, int dtype, 
   if (a.split && degree > 3) return STA_ERR_UNSUPPORTED;  // the split-product kernel's Taylor stops at 3
   hipStream_t s = static_cast<hipStream_t>(stream);
   const bool f32 = dtype == STA_F32;
-  if (d <= 16) return f32 ? dispatch_dvt<16, 4>(a, bh, s) : dispatch_dvt<16, 2>(a, bh, s);
-  if (d <= 32) return f32 ? dispatch_dvt<32, 4>(a, bh, s) : dispatch_dvt<32, 2>(a, bh, s);
-  if (d <= 64) return f32 ? dispatch_dvt<64, 4>(a, bh, s) : dispatch_dvt<64, 2>(a, bh, s);
-  if (d <= 128) return f32 ? dispatch_dvt<128, 4>(a, bh, s) : dispatch_dvt<128, 2>(a, bh, s);
-  return f32 ? dispatch_dvt<256, 4>(a, bh, s) : dispatch_dvt<256, 2>(a, bh, s);
+  int st;
+  if (d <= 16) st = f32 ? dispatch_dvt<16, 4>(a, bh, s) : dispatch_dvt<16, 2>(a, bh, s);
+  else if (d <= 32) st = f32 ? dispatch_dvt<32, 4>(a, bh, s) : dispatch_dvt<32, 2>(a, bh, s);
+  else if (d <= 64) st = f32 ? dispatch_dvt<64, 4>(a, bh, s) : dispatch_dvt<64, 2>(a, bh, s);
+  else if (d <= 128) st = f32 ? dispatch_dvt<128, 4>(a, bh, s) : dispatch_dvt<128, 2>(a, bh, s);
+  else st = f32 ? dispatch_dvt<256, 4>(a, bh, s) : dispatch_dvt<256, 2>(a, bh, s);
+  if (st != STA_OK || ksplit == 1) return st;
+  const int64_t blocks = (bh * n * (a.ldp / 4) + 255) / 256;
+  if (blocks > 0x7fffffff) return STA_ERR_SHAPE;
+  hipLaunchKernelGGL(sta::block_combine_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a, bh * n);
+  return check_launch();
+}
+
+int sta_block_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                        int dv, int ld_qk, int ld_v, int degree, float scale, float eps, int mode, int block, int chunk,
+                        int shift, int exp_clamp, int products, const float* low_num, const float* low_den, int fsplit,
+                        const int32_t* tile_ptr, const int32_t* tile_nodes, int n_tiles, const int32_t* node_meta,
+                        int n_nodes, int cap, const int32_t* node_src, const float* node_w, const float* rep_k,
+                        const float* rep_v, int ld_rep_k, int ld_rep_v, int64_t n_rep, void* out, int out_dtype,
+                        float* out_den, void* stream) {
+  return sta_block_attention_split(q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, degree, scale, eps, mode, block, chunk,
+                                   shift, exp_clamp, products, low_num, low_den, fsplit, tile_ptr, tile_nodes, n_tiles,
+                                   node_meta, n_nodes, cap, node_src, node_w, rep_k, rep_v, ld_rep_k, ld_rep_v, n_rep,
+                                   out, out_dtype, out_den, 1, nullptr, nullptr, stream);
 }
 
 int sta_selftest_mfma(const float* a, const float* b, float* d_out) {

@@ -67,6 +67,12 @@ struct BlockArgs {
   int out_dtype;
   float* out_den;  // optional [BH][n]: when set, out (fp32) receives num and out_den receives den, unnormalised
   int vec_out;     // dv a multiple of 4 and out aligned to 4 elements: whole-unit stores
+  // > 1: a tile's batches (and the moment partials) are dealt out to ksplit workgroups, whose raw sums
+  // block_combine_kernel adds up and normalises: part_num [ksplit][BH][n][ldp], part_den [ksplit][BH][n]
+  int ksplit;
+  float* part_num;
+  float* part_den;
+  int ldp;  // a multiple of 4
   int split;       // 1: split-bf16 matrix-core products (block_attn_kernel<..., true>)
 };
 
@@ -131,6 +137,10 @@ __device__ __forceinline__ float taylor2(float y, const TaylorCoef2& c) {
 }
 constexpr float LOG2E = 1.44269504f;
 
+// Few tiles (short sequences, few heads) leave compute units idle while a workgroup walks its batches, each a
+// chain of a load, two barriers and the products (about 3 us): BlockArgs::ksplit workgroups then share a tile
+// (1 x 4096 fp32 flat: 116 us with one, 39 us with eight).
+//
 // Work layout: one workgroup per (head, tile of 64*RS query rows); wave w owns RS strips of 16 rows.
 // Keys are staged in LDS 64 (or 32) at a time: K row-major, V transposed ([column][key]).  For a staged
 // batch each wave computes X = K Q^T for all its (strip, 16-key subtile) pairs with interleaved MFMA
@@ -146,6 +156,7 @@ constexpr float LOG2E = 1.44269504f;
 // Two waves per SIMD when the per-wave register arrays (queries, numerators, X and P tiles, prefetched
 // rows) leave room.
 constexpr int BA_LIST = 1024;
+constexpr int BA_MAX_SPLIT = 16;  // ksplit batches of 64 fit a list chunk
 __host__ __device__ constexpr int block_kb(int dp, int dvt) { return (dp + dvt * 16 > 192) ? 32 : 64; }
 __host__ __device__ constexpr int block_kpt(int dp, int dvt) { return (block_kb(dp, dvt) * dp / 4 + 255) / 256; }
 // value units: blocks of 4 keys x 4 columns
@@ -206,7 +217,8 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   __shared__ int Llo[BA_LIST], Lhi[BA_LIST];
   __shared__ float Lw[BA_LIST];
 
-  const int wg = xcd_remap(blockIdx.x, gridDim.x);
+  const int kw = xcd_remap(blockIdx.x, gridDim.x);
+  const int wg = kw / a.ksplit, ks = kw - wg * a.ksplit;
   const int64_t bh = wg / a.n_tiles;
   const int t = wg % a.n_tiles;
   const int tid = threadIdx.x;
@@ -463,7 +475,10 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   const int exp_from = max(chunk_start(row_hi, a.chunk, a.shift), residual_start(row_hi, a.mode, a.block));
   if (kstart < 0) kstart = 0;
   const int kend = row_hi + 1;
-  const int n_a = kend > kstart ? (kend - kstart + KB - 1) / KB : 0;
+  // this workgroup takes batches ks, ks + ksplit, ... of each phase (and of each list chunk)
+  const int n_own = kend > kstart ? (kend - kstart + KB - 1) / KB : 0;
+  const int n_a = (n_own - ks + a.ksplit - 1) / a.ksplit;
+  const int koff0 = ks * KB, kstep = a.ksplit * KB;
   const bool mat = a.rep_k != nullptr;  // segment-mean items index rep_k / rep_v (every node or none)
 
   // node item list, filled BA_LIST items at a time in tile-list order (uniform control flow)
@@ -642,11 +657,11 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     pden[rs] = a.low_den + bh * fs * pden_stride + a.low_off + i;
     pnum[rs] = a.low_num + (bh * fs * a.low_rows + a.low_off + i) * a.low_ld;
   }
-  const int n_pairs = RS * fs;
+  const int n_pairs = RS * ((fs - ks + a.ksplit - 1) / a.ksplit);  // the splits ks, ks + ksplit, ...
   float pair_d = 0.f;
   floatx4 pair_n[DVT];
   auto pair_load = [&](int p) {
-    const int f = p / RS, rs = p - f * RS;
+    const int fi = p / RS, rs = p - fi * RS, f = ks + fi * a.ksplit;
     const float* pd = pden[0];
     const float* pn = pnum[0];
 #pragma unroll
@@ -677,25 +692,25 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   };
 
   bool cur_node = n_a == 0;
-  int cur_off = cur_node ? 0 : kstart;
+  int cur_off = cur_node ? koff0 : kstart + koff0;
   // the first batch of the tile's own keys needs no list: its rows are in flight while the list's
   // chain of loads (tile list, node metadata, item indices) runs
   if (!cur_node) prefetch(false, cur_off);
   if (p_cur < p_end) fill();  // the first list chunk
   __syncthreads();
-  bool have = n_a > 0 || llen > 0;
+  bool have = n_a > 0 || koff0 < llen;  // (a list chunk with no batch for this workgroup is the last)
   if (have && cur_node) prefetch(true, cur_off);
   int pairs_done = 0;
   for (int b = 0; have; ++b) {
     __syncthreads();  // every wave is done with the staging buffers of the previous batch
     commit();
     bool nxt_node = true;
-    int nxt_off = cur_node ? cur_off + KB : 0;
+    int nxt_off = cur_node ? cur_off + kstep : koff0;
     if (!cur_node && b + 1 < n_a) {
       nxt_node = false;
-      nxt_off = cur_off + KB;
+      nxt_off = cur_off + kstep;
     } else if (nxt_off >= llen) {  // the list chunk is used up: refill it (uniform)
-      nxt_off = 0;
+      nxt_off = koff0;
       if (cur_node && p_cur < p_end)
         fill();
       else if (cur_node)
@@ -763,6 +778,16 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     dsum += __shfl_xor(dsum, 32);
     if (!rvalid[rs]) continue;
     const int64_t i = myrow[rs];
+    if (a.ksplit > 1) {
+      const int64_t row = (ks * static_cast<int64_t>(gridDim.x / (a.n_tiles * a.ksplit)) + bh) * a.n + i;
+      if (lg == 0) a.part_den[row] = dsum;
+#pragma unroll
+      for (int ct = 0; ct < DVT; ++ct) {
+        const int c0 = 16 * ct + 4 * lg;
+        if (c0 < a.ldp) *reinterpret_cast<floatx4*>(a.part_num + row * a.ldp + c0) = num[rs][ct];
+      }
+      continue;
+    }
     if (raw && lg == 0) a.out_den[bh * a.n + i] = dsum;
     const float dn = fmaxf(dsum, a.eps);
 #pragma unroll
@@ -796,6 +821,26 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
       }
     }
   }
+}
+
+// out = sum of the ksplit partial numerators / max(sum of the denominators, eps), four columns a thread.
+static __global__ __launch_bounds__(256) void block_combine_kernel(const BlockArgs a, int64_t rows) {
+  const int cu = a.ldp >> 2;
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t row = e / cu;
+  if (row >= rows) return;
+  const int c0 = static_cast<int>(e - row * cu) * 4;
+  floatx4 o = {0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+  for (int s = 0; s < a.ksplit; ++s) {
+    const int64_t r = s * rows + row;
+    o += *reinterpret_cast<const floatx4*>(a.part_num + r * a.ldp + c0);
+    den += a.part_den[r];
+  }
+  const float dn = fmaxf(den, a.eps);
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    if (c0 + m < a.dv) store_elem(a.out, row * a.dv + c0 + m, a.out_dtype, o[m] / dn);
 }
 
 }  // namespace sta

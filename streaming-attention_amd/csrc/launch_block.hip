@@ -15,7 +15,7 @@ namespace sta_api {
 
 template <int DP, int DVT, int ES>
 int launch_block(const sta::BlockArgs& a, int64_t bh, hipStream_t s) {
-  const int64_t grid = bh * a.n_tiles;
+  const int64_t grid = bh * a.n_tiles * a.ksplit;
   if (grid <= 0 || grid > 0x7fffffff) return STA_ERR_SHAPE;
   if (a.split && ES == 2 && a.dtype == sta::BF16 && a.rep_k == nullptr)  // key / value rows exact in bf16
     hipLaunchKernelGGL((sta::block_attn_kernel<DP, DVT, 2, ES, true, ES == 2>), dim3(static_cast<unsigned>(grid)),

@@ -143,3 +143,32 @@ def test_few_streams_tail_matches_many(d, dv, block, tokens, fused):
                 rows.append(att.query(q[t, :s])[:2])
         outs.append(torch.stack(rows))
     assert rel(outs[0], outs[1].cpu().double()) < 2e-6
+
+
+@pytest.mark.parametrize("semantics,bh,n,d,dv,degree,block,dtype,out_dtype", [
+    ("flat", 1, 1100, 64, 64, 2, 64, torch.float32, torch.float32), ("flat", 2, 4300, 16, 30, 2, 100, torch.bfloat16, None),
+    ("levels", 1, 3000, 40, 72, 2, 48, torch.float16, None), ("levels", 3, 200, 128, 200, 3, 128, torch.float32, None),
+    ("segment", 2, 900, 64, 64, 2, 128, torch.float16, torch.float32), ("flat", 1, 700, 200, 16, 2, 64, torch.float32, None),
+])
+@pytest.mark.parametrize("ksplit", [2, 3, 16])
+def test_residual_tiles_shared_by_workgroups(monkeypatch, semantics, bh, n, d, dv, degree, block, dtype, out_dtype, ksplit):
+    """ksplit workgroups a tile (more than its batches, and a remainder of its list chunks among them) against
+    one: the same terms in another order of fp32 sums (2e-6), rounded to 16 bits at most twice apart."""
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(bh, n, w, generator=g).mul_(0.4).to(dtype).to(DEV) for w in (d, d, dv))
+    kw = dict(degree=degree, block=block, scale=0.3, semantics=semantics, stride=2, out_dtype=out_dtype or dtype,
+              exp_clamp=semantics == "segment")
+    print(semantics, bh, n, d, dv, degree, block, dtype, ksplit, flush=True)
+    outs = []
+    for s in (1, ksplit):
+        monkeypatch.setattr(_engine, "residual_splits", lambda *a, s=s: s)
+        outs.append(_engine.prefill(q, k, v, **kw).out)
+    assert rel(outs[1], outs[0].cpu().double()) < 2e-6 + 2 * TOL[out_dtype or dtype]
+
+
+def test_residual_split_rule():
+    flat = lambda n, block: _engine._plan.flat_plan(n, block, "sorted_pair")
+    assert _engine.residual_splits(1, flat(1024, 128), 128, 64, 256) == 1
+    assert _engine.residual_splits(1, flat(4096, 256), 256, 128, 256) == 8
+    assert _engine.residual_splits(16, flat(3000, 128), 128, 128, 256) == 2
+    assert _engine.residual_splits(64, flat(3000, 128), 128, 128, 256) == 1
