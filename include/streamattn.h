@@ -430,6 +430,18 @@ int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, 
                         int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream);
 
 /*
+ * sta_flash_attention / sta_exact_attention with a tile's key batches dealt out to nsplit >= 1 workgroups, for
+ * grids that leave compute units idle: raw sums to part_num [nsplit][BH][N][4 ceil(Dv / 4)], denominators and row
+ * maxima to part_den [nsplit][BH][N][2] (both 16-byte aligned), added and normalised by a second launch.
+ */
+int sta_flash_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                              int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, int nsplit,
+                              float* part_num, float* part_den, void* stream);
+int sta_exact_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                              int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, int nsplit,
+                              float* part_num, float* part_den, void* stream);
+
+/*
  * The Taylor part over pairs, for short sequences: low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i,
  * c(i) = floor((i + shift) / chunk) chunk - shift, in sta_moments' partials layout with nsplit partials (a tile's
  * keys are dealt out to nsplit workgroups), for sta_block_attention with the same chunk and shift.

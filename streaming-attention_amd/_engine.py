@@ -140,13 +140,28 @@ def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, com
     440 tiles: 74 -> 86 and left alone), none where the longest tile is so short that the second launch costs
     the host more (1 x 1024, d = dv = 32: a pass 61 -> 65 us)."""
     tiles = bh * plan.n_tiles
-    most = int(np.diff(plan.tile_ptr).max()) * plan.cap + min(block, plan.n)  # items and keys of the longest tile
+    if 2 * tiles > 3 * compute_units:
+        return 1
+    most = plan.longest_tile * plan.cap + min(block, plan.n)  # items and keys of the longest tile
     if most * width < 40000:
         return 1
     want = 2 * compute_units // tiles
-    if want < 2:
-        want = 2 if 2 * tiles <= 3 * compute_units else 1
-    return max(1, min(want, most // 128, 8))
+    return max(1, min(max(want, 2), most // 128, 8))
+
+
+def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int) -> int:
+    """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split): where the tiles leave
+    compute units idle, and up to two tiles a unit where long tiles would meet (d = dv = 64; 1 x 8192 fp32 397 -> 70 us
+    with 8, 4 x 8192 bf16, 256 tiles, 178 -> 88 with 4, 8 x 8191 fp32, 512 tiles, 467 -> 387 with 3, 32 x 2048 113 -> 109
+    with 2).  Each takes at least 128 keys of the longest tile (1024 where no unit is idle: 64 x 1024 63 -> 73 with
+    2); beyond two tiles a unit (40 x 2048 bf16 58 -> 68 with 2) and for calls bound by their launches (1 x 500, d =
+    dv = 32, 14 -> 17) one."""
+    tiles = bh * -(-n // _plan.TILE_ROWS)
+    if n * (d + dv) < 48000 or tiles > 2 * compute_units:
+        return 1
+    want = min(4 * compute_units // tiles, n // 128, 8) if tiles <= compute_units else \
+        min(6 * compute_units // tiles, n // 1024)
+    return max(1, want)
 
 
 # Offer the planner the 64-column moment workgroups (split products, 32 < dv <= 64).  Off: on 32 heads x
@@ -648,22 +663,28 @@ def flash(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, *, scale: float,
 
 def _pairs(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, scale: float, eps: Optional[float],
            out_dtype: torch.dtype, timer: Optional[KernelTimer]) -> torch.Tensor:
-    """Launch of the pair kernel: sta_flash_attention (eps None), or sta_exact_attention with its smallest
-    denominator eps."""
+    """Launch of the pair kernel: sta_flash_attention_split (eps None), or sta_exact_attention_split with its
+    smallest denominator eps."""
     bh, n, d = q3.shape
     dv = v3.shape[-1]
     out = torch.empty((bh, n, dv), device=q3.device, dtype=out_dtype)
     dq, dvp = -(-d // 4) * 4, -(-dv // 4) * 4
     mq, mk, mv = _padded_rows(q3, dq), _padded_rows(k3, dq), _padded_rows(v3, dvp)
     lib = _native.lib()
+    nsplit = flash_splits(bh, n, d, dv, _compute_units(q3.device))
+    part_num = part_den = None
+    if nsplit > 1:
+        part_num = torch.empty((nsplit, bh, n, dvp), device=q3.device, dtype=torch.float32)
+        part_den = torch.empty((nsplit, bh, n, 2), device=q3.device, dtype=torch.float32)
     name = "flash" if eps is None else "exact_attention"
-    fn = lib.sta_flash_attention if eps is None else lib.sta_exact_attention
+    fn = lib.sta_flash_attention_split if eps is None else lib.sta_exact_attention_split
     args = (float(scale),) if eps is None else (float(scale), float(eps))
 
     def launch():
         st = fn(mq.data_ptr(), mk.data_ptr(), mv.data_ptr(), _native.DTYPE_CODES[q3.dtype], bh, n, d, dv, dq, dvp,
-                *args, out.data_ptr(), _native.DTYPE_CODES[out_dtype], _native.stream_handle(q3.device))
-        _native.check(st, "sta_" + ("flash_attention" if eps is None else name))
+                *args, out.data_ptr(), _native.DTYPE_CODES[out_dtype], nsplit, _native.ptr(part_num),
+                _native.ptr(part_den), _native.stream_handle(q3.device))
+        _native.check(st, "sta_flash_attention_split" if eps is None else "sta_exact_attention_split")
 
     _run(timer, name, launch)
     return out

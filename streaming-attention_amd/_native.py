@@ -105,6 +105,13 @@ _SIGNATURES = {
     "sta_exact_attention": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _c_p, _i32, _c_p],
     ),
+    "sta_flash_attention_split": (
+        _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _c_p, _i32, _i32, _c_p, _c_p, _c_p],
+    ),
+    "sta_exact_attention_split": (
+        _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _c_p, _i32, _i32, _c_p, _c_p,
+               _c_p],
+    ),
     "sta_pair_moments": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _i32, _f32, _i32, _i32, _i32, _c_p, _c_p,
                _c_p],  # q k v dtype bh n d dv ld_qk ld_v degree scale chunk shift nsplit num den stream

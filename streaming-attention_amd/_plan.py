@@ -16,6 +16,7 @@ The projection direction is normalised with the same torch ops as the reference
 from __future__ import annotations
 
 import heapq
+import functools
 import itertools
 import math
 import threading
@@ -960,6 +961,11 @@ class NodePlan:
     n_tiles: int
     call_sizes: List[int] = field(default_factory=list)  # n_in of each draw slot (call order)
     level_of: Optional[np.ndarray] = None  # level of each node (levels mode)
+
+    @functools.cached_property
+    def longest_tile(self) -> int:
+        """Nodes of the row tile with the most of them."""
+        return int(np.diff(self.tile_ptr).max()) if self.n_tiles > 0 else 0
 
 
 def _tile_lists(meta: np.ndarray, n: int, shift: int) -> Tuple[np.ndarray, np.ndarray, int]:

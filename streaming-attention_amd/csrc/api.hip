@@ -129,8 +129,13 @@ int flash_dispatch(const sta::FlashArgs& a, int weight, void* stream) {
 }
 
 int flash_launch(int weight, const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
-                 int dv, int ld_qk, int ld_v, float scale, float floor, void* out, int out_dtype, void* stream) {
+                 int dv, int ld_qk, int ld_v, float scale, float floor, void* out, int out_dtype, int nsplit,
+                 float* part_num, float* part_den, void* stream) {
   sta::FlashArgs a;
+  if (nsplit < 1) return STA_ERR_SHAPE;
+  if (nsplit > 1 && (!part_num || !part_den ||
+                     ((reinterpret_cast<uintptr_t>(part_num) | reinterpret_cast<uintptr_t>(part_den)) & 15u) != 0))
+    return STA_ERR_ARG;
   if (!out) return STA_ERR_ARG;
   if (!dtype_ok(out_dtype)) return STA_ERR_DTYPE;
   if (const int st = flash_args(a, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v); st != STA_OK) return st;
@@ -139,7 +144,14 @@ int flash_launch(int weight, const void* q, const void* k, const void* v, int dt
   a.floor = floor;
   a.out = out; a.out_dtype = out_dtype;
   a.vec_out = (out_dtype == STA_F32 && dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) ? 1 : 0;
-  return flash_dispatch(a, weight, stream);
+  a.nsplit = nsplit; a.low_num = part_num; a.low_den = part_den; a.low_ld = (dv + 3) / 4 * 4;
+  const int st = flash_dispatch(a, weight, stream);
+  if (st != STA_OK || nsplit == 1) return st;
+  const int64_t blocks = (bh * n * (a.low_ld / 4) + 255) / 256;
+  if (blocks > 0x7fffffff) return STA_ERR_SHAPE;
+  hipLaunchKernelGGL(sta::flash_combine_kernel, dim3(static_cast<unsigned>(blocks)), dim3(256), 0,
+                     static_cast<hipStream_t>(stream), a);
+  return check_launch();
 }
 
 // Exclusive scan over the segments of each (head, feature split, column group): seg_state[p] <- sum of
@@ -191,13 +203,28 @@ int sta_limits(int* max_d, int* max_dv, int* max_degree, int* max_compress_in) {
 
 int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, void* stream) {
+  return flash_launch(sta::FLASH_SOFTMAX, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, 1e-20f, out, out_dtype, 1,
+                      nullptr, nullptr, stream);
+}
+
+int sta_flash_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                              int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, int nsplit,
+                              float* part_num, float* part_den, void* stream) {
   return flash_launch(sta::FLASH_SOFTMAX, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, 1e-20f, out, out_dtype,
-                      stream);
+                      nsplit, part_num, part_den, stream);
 }
 
 int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream) {
-  return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, stream);
+  return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, 1, nullptr,
+                      nullptr, stream);
+}
+
+int sta_exact_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
+                              int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, int nsplit,
+                              float* part_num, float* part_den, void* stream) {
+  return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, nsplit,
+                      part_num, part_den, stream);
 }
 
 int sta_pair_moments(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d, int dv,

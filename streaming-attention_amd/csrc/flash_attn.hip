@@ -35,6 +35,7 @@
 // = 174 TF/s (fp32 matrix instructions, unbalanced tiles: 857 us); 2 x 16 x 8192 bf16: 479 us = 579 TF/s
 // (710 us with a rescale and 12 more VALU instructions a pair); FLASH_EXP 4 x 8 x 2048 fp32: 102 us (513 us as
 // moment scan + residual kernel in fp32 products);
+// with few tiles, FlashArgs::nsplit workgroups share one: 1 x 8192 fp32 397 -> 70 us, 8 x 8191 467 -> 387 us.
 // FLASH_TAYLOR 8 x 16 x 4096 bf16: 0.5 ms in the place of the moment scan's 1.06.
 #include <type_traits>
 
@@ -61,7 +62,9 @@ struct FlashArgs {
   void* out;     // [BH][n][dv], dense
   int out_dtype;
   int vec_out;  // fp32 output, dv % 4 == 0 and 16-byte aligned: 16-byte stores
-  // key batches of a tile are dealt out to nsplit workgroups, each with sums of its own (1 but for FLASH_TAYLOR)
+  // key batches of a tile are dealt out to nsplit workgroups, each with sums of its own.  FLASH_TAYLOR: partials
+  // (below).  The others, nsplit > 1: raw sums low_num [nsplit][BH][n][low_ld] and {denominator, row maximum}
+  // low_den [nsplit][BH][n][2], which flash_combine_kernel adds up and normalises
   int nsplit;
   // FLASH_TAYLOR: coefficients of x, x^2, x^3 (the logit, or q.k of 16-bit rows), the row chunk and its offset
   // (c(i) = floor((i + shift) / chunk) chunk - shift; row tiles start at -shift), the partials
@@ -441,10 +444,10 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
 
   const int row_hi = (r0 + FLASH_ROWS < n ? r0 + FLASH_ROWS : n) - 1;  // r0 < n: t < ceil(n / FLASH_ROWS)
   const int kend = limit(row_hi);
-  const int step = TAYLOR ? a.nsplit : 1;  // this workgroup's batches: split, split + step, ...
+  const int step = a.nsplit;  // this workgroup's batches: split, split + step, ...
   const int nb_all = (kend + KB - 1) / KB;
-  const int nb = TAYLOR ? (nb_all - split + step - 1) / step : nb_all;
-  auto offset = [&](int b) { return (TAYLOR ? split + b * step : b) * KB; };
+  const int nb = (nb_all - split + step - 1) / step;
+  auto offset = [&](int b) { return (split + b * step) * KB; };
 
   // Staging registers: this thread's 4-element units of the next batch's rows, raw: key rows unit by unit,
   // value rows as blocks of 4 keys x 4 columns (the transposed write is then 8 bytes).  Offsets inside
@@ -544,9 +547,9 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
         process(std::false_type{}, off, st, st + KP * KPL);
     }
   };
-  if (!TAYLOR || nb > 0) prefetch(offset(0));
+  if (nb > 0) prefetch(offset(0));
   if constexpr (NST == 2) {
-    if (!TAYLOR || nb > 0) commit(stage, stage + KP * KPL);
+    if (nb > 0) commit(stage, stage + KP * KPL);
     if (nb > 1) prefetch(offset(1));
     __syncthreads();
     for (int b = 0; b < nb; ++b) {
@@ -588,6 +591,16 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
       }
       continue;
     }
+    if (a.nsplit > 1) {
+      const int64_t row = (split * a.bh + bh) * a.n + myrow[rs];
+      if (lg == 0) *reinterpret_cast<floatx2*>(a.low_den + 2 * row) = floatx2{dsum, W == FLASH_SOFTMAX ? mrow[rs] : 0.f};
+#pragma unroll
+      for (int ct = 0; ct < DVT; ++ct) {
+        const int c0 = 16 * ct + 4 * lg;
+        if (c0 < a.low_ld) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
+      }
+      continue;
+    }
     const float dn = fmaxf(dsum, a.floor);
     const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
 #pragma unroll
@@ -606,6 +619,33 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
       }
     }
   }
+}
+
+// out = the nsplit raw sums relative to their largest maximum, added in order, over their denominator; four columns
+// a thread.
+static __global__ __launch_bounds__(256) void flash_combine_kernel(const FlashArgs a) {
+  const int cu = a.low_ld >> 2;
+  const int64_t rows = a.bh * a.n;
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int64_t row = e / cu;
+  if (row >= rows) return;
+  const int c0 = static_cast<int>(e - row * cu) * 4;
+  const floatx2* const dm = reinterpret_cast<const floatx2*>(a.low_den);
+  float top = dm[row][1];
+  for (int s = 1; s < a.nsplit; ++s) top = fmaxf(top, dm[s * rows + row][1]);
+  floatx4 o = {0.f, 0.f, 0.f, 0.f};
+  float den = 0.f;
+  for (int s = 0; s < a.nsplit; ++s) {
+    const int64_t r = s * rows + row;
+    const floatx2 d = dm[r];
+    const float f = __builtin_amdgcn_exp2f(d[1] - top);
+    o += f * *reinterpret_cast<const floatx4*>(a.low_num + r * a.low_ld + c0);
+    den = fmaf(f, d[0], den);
+  }
+  const float dn = fmaxf(den, a.floor);
+#pragma unroll
+  for (int m = 0; m < 4; ++m)
+    if (c0 + m < a.dv) store_elem(a.out, row * a.dv + c0 + m, a.out_dtype, o[m] / dn);
 }
 
 }  // namespace sta

@@ -172,3 +172,23 @@ def test_residual_split_rule():
     assert _engine.residual_splits(1, flat(4096, 256), 256, 128, 256) == 8
     assert _engine.residual_splits(16, flat(3000, 128), 128, 128, 256) == 2
     assert _engine.residual_splits(64, flat(3000, 128), 128, 128, 256) == 1
+
+
+@pytest.mark.parametrize("heads,n,d,dv,dtype", [(1, 300, 64, 64, torch.float32), (3, 1025, 40, 72, torch.bfloat16),
+                                                (2, 130, 128, 200, torch.float16), (8, 65, 16, 5, torch.float32)])
+@pytest.mark.parametrize("nsplit", [2, 5, 8])
+def test_exact_tiles_shared_by_workgroups(monkeypatch, heads, n, d, dv, dtype, nsplit):
+    """nsplit workgroups a tile, more than its key batches among them, against float64 (bounds as above)."""
+    monkeypatch.setattr(_engine, "flash_splits", lambda *a: nsplit)
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(1, heads, n, w, generator=g).to(dtype) for w in (d, d, dv))
+    out = taa.triton_flash_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=0.4)
+    assert rel(out, exact(q, k, v, 0.4)) < (4e-6 if dtype == torch.bfloat16 else 1e-6)
+    out = faa.fast_article_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=0.1, compressor="none")
+    assert rel(out, exact(q, k, v, 0.1, 1e-12)) < TOL[dtype] + 1e-6
+
+
+def test_exact_split_rule():
+    sp = lambda bh, n, w=64: _engine.flash_splits(bh, n, w, w, 256)
+    assert [sp(1, 8192), sp(4, 8192), sp(8, 8191), sp(32, 2048), sp(40, 2048), sp(64, 1024), sp(1, 500, 32)] == \
+        [8, 4, 3, 2, 1, 1, 1]
