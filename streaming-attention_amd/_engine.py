@@ -109,21 +109,24 @@ def ws_query_block(semantics: str, block: int) -> Optional[int]:
     return None  # raw Taylor sums: the residual kernel adds the polynomial over the query block's keys
 
 
-# Longest sequence whose Taylor part runs over the pairs (sta_pair_moments) instead of the moment scan: the
-# pairs take n^2 / 2 (d + dv) products of a head, the moments n F dv for F features, both with the widths the
-# kernels pad to (and the scan no less than that of 512 features x 64 columns: its cost per chunk), so the
-# crossing is at n = R F dv / (d + dv), R from the rates measured on both sides (64 heads, d = dv = 64, degree 2,
-# scan / pairs): fp32 4096: 564 / 427 us, 6144: 881 / 968; fp16 6144: 943 / 746, 8192: 1372 / 1339; bf16 (two products
-# a value less) 6144: 775 / 561, 8192: 1071 / 1001.  d = dv = 128 (32 heads), fp32 8192: 5459 / 2385, bf16 5739 / 1026;
-# d = 16, dv = 64, degree 3, fp32 2048: 169 / 95, 4096: 317 / 342; degree 1, d = 64, fp32 1024: 61 / 49, 2048: 111 / 141.
-PAIRS_RATIO = {torch.float32: 4.7, torch.bfloat16: 7.5, torch.float16: 6.5}
+# Longest sequence whose Taylor part runs over the pairs (sta_pair_moments) instead of the moment scan.  A pair's
+# time grows with the padded d + dv (32 dimensions at least) and a constant 24 columns' worth of weights, a token's
+# scan with F dv for F features (64 columns at a time, and no less than 200 features x 64 where the wave-specialised
+# scan applies, 512 x 64 with the chunked one), so the crossing is at n = R F dv / (d + dv + 24), R from the rates
+# measured on both sides (64 heads, d = dv = 64, degree 2, scan / pairs): fp32 4096: 564 / 427 us, 6144: 881 / 968; fp16
+# 6144: 943 / 746, 8192: 1372 / 1339; bf16 (two products a value less) 6144: 775 / 561, 8192: 1071 / 1001.  d = dv = 128
+# (32 heads), fp32 8192: 5459 / 2385, bf16 5739 / 1026; d = 16, dv = 64, degree 3, fp32 2048: 169 / 95, 4096: 317 / 342;
+# d = dv = 32, fp32 2048: 108 / 78, 4096: 186 / 266; d = dv = 16, bf16 levels, 64 x 3000: a pass 173 / 195.
+# One line for all types, fp32's: a bf16 call then takes the route of its fp32 values, and gives their sums bit for bit.
+PAIRS_RATIO = 5.6
 
 
-def use_pairs(n: int, d: int, dv: int, degree: int, dtype: torch.dtype) -> bool:
-    pad_d = max(16, 1 << (d - 1).bit_length())
+def use_pairs(n: int, d: int, dv: int, degree: int, block: int) -> bool:
+    pad_d = max(32, 1 << (d - 1).bit_length())
     pad_dv = max(16, 1 << (dv - 1).bit_length())
-    scan = max(_plan.num_features(d, degree) * 64 * -(-dv // 64), 512 * 64)
-    return n * (pad_d + pad_dv) <= PAIRS_RATIO[dtype] * scan
+    least = 200 if block % 32 == 0 and block >= 64 else 512
+    scan = max(_plan.num_features(d, degree) * 64 * -(-dv // 64), least * 64)
+    return n * (pad_d + pad_dv + 24) <= PAIRS_RATIO * scan
 
 
 def pair_splits(bh: int, n: int, compute_units: int) -> int:
@@ -387,7 +390,7 @@ def prefill(
 
     # short sequences: the Taylor part over the pairs (sta_pair_moments)
     pairs = (semantics in ("flat", "levels", "segment") and degree <= 3 and d <= FLASH_D and products is None and
-             (moment_kernel == "pairs" or (moment_kernel is None and use_pairs(n, d, dv, degree, pq.dtype))))
+             (moment_kernel == "pairs" or (moment_kernel is None and use_pairs(n, d, dv, degree, block))))
     qblock = None
     if pairs:
         chunk = block if block % chunk == 0 else chunk

@@ -159,11 +159,15 @@ constexpr int BA_LIST = 1024;
 constexpr int BA_MAX_SPLIT = 16;  // ksplit batches of 64 fit a list chunk
 __host__ __device__ constexpr int block_kb(int dp, int dvt) { return (dp + dvt * 16 > 192) ? 32 : 64; }
 __host__ __device__ constexpr int block_kpt(int dp, int dvt) { return (block_kb(dp, dvt) * dp / 4 + 255) / 256; }
-// value units: blocks of 4 keys x 4 columns
-__host__ __device__ constexpr int block_vpt(int dp, int dvt) { return (block_kb(dp, dvt) * dvt + 255) / 256; }
+// value units: blocks of 4 keys x 4 columns (2 keys for 16 columns, whose 64 blocks of 4 would leave three waves
+// without one: d = dv = 16, 64 heads x 3000 bf16 levels, a pass 178 us)
+__host__ __device__ constexpr int block_vk(int dvt) { return dvt == 1 ? 2 : 4; }
+__host__ __device__ constexpr int block_vpt(int dp, int dvt) {
+  return (block_kb(dp, dvt) / block_vk(dvt) * dvt * 4 + 255) / 256;
+}
 __host__ __device__ constexpr int block_occupancy(int dp, int dvt, int rs) {
   return (rs * dp / 4 + rs * dvt * 4 + 2 * rs * (block_kb(dp, dvt) / 16) * 4 +
-          4 * (block_kpt(dp, dvt) + 4 * block_vpt(dp, dvt))) <= 160
+          4 * (block_kpt(dp, dvt) + block_vk(dvt) * block_vpt(dp, dvt))) <= 160
              ? 2
              : 1;
 }
@@ -518,10 +522,11 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // when written to LDS, so no instruction waits on the loads before the next commit): key rows unit by unit,
   // value rows as blocks of 4 keys x 4 columns, so that the transposed write is one word per column and
   // plane.  Absent rows and columns load from beyond the buffer, which reads as zero.
-  constexpr int KU = DP / 4, VU = DV / 4, KG = KB / 4;
+  constexpr int VK = block_vk(DVT);
+  constexpr int KU = DP / 4, VU = DV / 4, KG = KB / VK;
   constexpr int KPT = block_kpt(DP, DVT), VPT = block_vpt(DP, DVT);
   static_assert(256 % KU == 0, "a thread's key units share one column");
-  uint4 pk[KPT], pv[VPT][4];
+  uint4 pk[KPT], pv[VPT][VK];
   int pj = -1, plo = 0, phi = -1;
   float pw = 0.f;
   const int ku = tid % KU, kr0 = tid / KU;
@@ -547,18 +552,25 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     for (int i = 0; i < VPT; ++i) {
       const int e = tid + 256 * i, g = e % KG, u = e / KG;  // key-fast: conflict-light transposed writes
       const bool in = (KG * VU % 256 == 0 || e < KG * VU) && 4 * u < ldv;
-      int4 src = int4{-1, -1, -1, -1};
+      int sv[VK];
+#pragma unroll
+      for (int c = 0; c < VK; ++c) sv[c] = -1;
       if (in) {
         if (node) {
-          src = *reinterpret_cast<const int4*>(Lj + off + 4 * g);
+          if constexpr (VK == 4) {
+            const int4 x = *reinterpret_cast<const int4*>(Lj + off + 4 * g);
+            sv[0] = x.x; sv[1] = x.y; sv[2] = x.z; sv[3] = x.w;
+          } else {
+            const int2 x = *reinterpret_cast<const int2*>(Lj + off + 2 * g);
+            sv[0] = x.x; sv[1] = x.y;
+          }
         } else {
-          const int j = off + 4 * g;
-          src = int4{j < kend ? j : -1, j + 1 < kend ? j + 1 : -1, j + 2 < kend ? j + 2 : -1, j + 3 < kend ? j + 3 : -1};
+#pragma unroll
+          for (int c = 0; c < VK; ++c) sv[c] = off + VK * g + c < kend ? off + VK * g + c : -1;
         }
       }
-      const int sv[4] = {src.x, src.y, src.z, src.w};
 #pragma unroll
-      for (int c = 0; c < 4; ++c)
+      for (int c = 0; c < VK; ++c)
         pv[i][c] = load_row_unit<ES>(vr, sv[c] >= 0 ? static_cast<uint32_t>(sv[c]) * vst + 4 * ES * u : BLOCK_ABSENT);
     }
     if (tid < KB) {
@@ -591,33 +603,39 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     for (int i = 0; i < VPT; ++i) {
       const int e = tid + 256 * i, g = e % KG, u = e / KG;
       if (KG * VU % 256 != 0 && e >= KG * VU) continue;
+      // one word a column and plane: VK keys in contraction order (split_key_pos) or in order (fp32)
+      auto put = [&](__bf16* dst, const uint32_t (&w)[VK / 2]) {
+        if constexpr (VK == 4)
+          *reinterpret_cast<uint2*>(dst) = uint2{w[0], w[1]};
+        else
+          *reinterpret_cast<uint32_t*>(dst) = w[0];
+      };
       if constexpr (KVX) {
-        // 16-bit 4 x 4 transpose: column m of the 4 keys
-        __bf16* const dst = Vh + 4 * u * LDVB + split_key_pos(4 * g);
+        // 16-bit transpose: column m of the VK keys
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
           const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
-          const uint32_t k0 = m < 2 ? pv[i][0].x : pv[i][0].y, k1 = m < 2 ? pv[i][1].x : pv[i][1].y;
-          const uint32_t k2 = m < 2 ? pv[i][2].x : pv[i][2].y, k3 = m < 2 ? pv[i][3].x : pv[i][3].y;
-          *reinterpret_cast<uint2*>(dst + m * LDVB) =
-              uint2{__builtin_amdgcn_perm(k1, k0, sel), __builtin_amdgcn_perm(k3, k2, sel)};
+          uint32_t w[VK / 2];
+#pragma unroll
+          for (int c = 0; c < VK; c += 2)
+            w[c / 2] = __builtin_amdgcn_perm(m < 2 ? pv[i][c + 1].x : pv[i][c + 1].y, m < 2 ? pv[i][c].x : pv[i][c].y, sel);
+          put(Vh + (4 * u + m) * LDVB + split_key_pos(VK * g), w);
         }
       } else {
-        floatx4 f[4];
+        floatx4 f[VK];
 #pragma unroll
-        for (int c = 0; c < 4; ++c) f[c] = unit_to_f4<ES>(pv[i][c], a.dtype, 1.f);
+        for (int c = 0; c < VK; ++c) f[c] = unit_to_f4<ES>(pv[i][c], a.dtype, 1.f);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
           if constexpr (SPLIT) {
-            // each subtile pair's keys in contraction order (split_key_pos)
-            const int dst = (4 * u + m) * LDVB + split_key_pos(4 * g);
-            uint32_t h0, h1, l0, l1;
-            split_pair(f[0][m], f[1][m], h0, l0);
-            split_pair(f[2][m], f[3][m], h1, l1);
-            *reinterpret_cast<uint2*>(Vh + dst) = uint2{h0, h1};
-            *reinterpret_cast<uint2*>(Vl + dst) = uint2{l0, l1};
+            uint32_t h[VK / 2], l[VK / 2];
+#pragma unroll
+            for (int c = 0; c < VK; c += 2) split_pair(f[c][m], f[c + 1][m], h[c / 2], l[c / 2]);
+            put(Vh + (4 * u + m) * LDVB + split_key_pos(VK * g), h);
+            put(Vl + (4 * u + m) * LDVB + split_key_pos(VK * g), l);
           } else {
-            *reinterpret_cast<floatx4*>(Vt + (4 * u + m) * LDVT + 4 * g) = floatx4{f[0][m], f[1][m], f[2][m], f[3][m]};
+#pragma unroll
+            for (int c = 0; c < VK; ++c) Vt[(4 * u + m) * LDVT + VK * g + c] = f[c][m];
           }
         }
       }

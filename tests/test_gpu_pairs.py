@@ -100,8 +100,10 @@ def test_taylor_pairs_match_the_moment_scan(bh, n, d, dv, degree, block, dtype, 
 
 
 def test_pair_rule_and_splits():
-    assert _engine.use_pairs(1024, 32, 32, 2, torch.float32)
-    assert not _engine.use_pairs(65536, 64, 64, 2, torch.bfloat16)
+    assert _engine.use_pairs(1024, 32, 32, 2, 128)
+    assert _engine.use_pairs(4096, 64, 64, 2, 256)
+    assert not _engine.use_pairs(65536, 64, 64, 2, 256)
+    assert not _engine.use_pairs(3000, 16, 16, 2, 128)
     assert _engine.pair_splits(1, 200, 256) == 1 and _engine.pair_splits(1, 4096, 256) == 8
     assert _engine.pair_splits(64, 4096, 256) == 1
 
