@@ -570,54 +570,173 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   }
 
   // ---- epilogue: row sums (over the four lane groups), normalise, store ----
+  float dsum[RS];
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
-    float dsum;
     if constexpr (DENM) {
-      dsum = dacc[rs][0];  // every element of the column is the row's sum
+      dsum[rs] = dacc[rs][0];  // every element of the column is the row's sum
     } else {
-      dsum = den[rs];
-      dsum += __shfl_xor(dsum, 16);
-      dsum += __shfl_xor(dsum, 32);
+      dsum[rs] = den[rs];
+      dsum[rs] += __shfl_xor(dsum[rs], 16);
+      dsum[rs] += __shfl_xor(dsum[rs], 32);
     }
-    if (!rvalid[rs]) continue;
+  }
+  auto put_den = [&](int row, float ds, float mr) {
+    if (lg != 0) return;
+    if constexpr (TAYLOR)
+      a.low_den[(bh * a.nsplit + split) * a.low_rows + a.low_off + row] = ds;
+    else if (a.nsplit > 1)
+      *reinterpret_cast<floatx2*>(a.low_den + 2 * ((split * a.bh + bh) * a.n + row)) =
+          floatx2{ds, W == FLASH_SOFTMAX ? mr : 0.f};
+  };
+  auto put = [&](int row, int c0, float ds, const floatx4& x) {  // columns c0 .. c0 + 3
     if constexpr (TAYLOR) {
-      const int64_t row = (bh * a.nsplit + split) * a.low_rows + a.low_off + myrow[rs];
-      if (lg == 0) a.low_den[row] = dsum;
-#pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) {
-        const int c0 = 16 * ct + 4 * lg;  // low_ld is whole 32-column groups
-        if (c0 < a.dv) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
-      }
-      continue;
+      const int64_t lrow = (bh * a.nsplit + split) * a.low_rows + a.low_off + row;
+      if (c0 < a.dv)  // low_ld is whole 32-column groups
+        *reinterpret_cast<floatx4*>(a.low_num + lrow * a.low_ld + c0) = x;
+      return;
     }
     if (a.nsplit > 1) {
-      const int64_t row = (split * a.bh + bh) * a.n + myrow[rs];
-      if (lg == 0) *reinterpret_cast<floatx2*>(a.low_den + 2 * row) = floatx2{dsum, W == FLASH_SOFTMAX ? mrow[rs] : 0.f};
-#pragma unroll
-      for (int ct = 0; ct < DVT; ++ct) {
-        const int c0 = 16 * ct + 4 * lg;
-        if (c0 < a.low_ld) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
-      }
-      continue;
+      if (c0 < a.low_ld)
+        *reinterpret_cast<floatx4*>(a.low_num + ((split * a.bh + bh) * a.n + row) * a.low_ld + c0) = x;
+      return;
     }
-    const float dn = fmaxf(dsum, a.floor);
-    const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
+    if (c0 >= a.dv) return;
+    const float dn = fmaxf(ds, a.floor);
+    const int64_t o0 = (bh * a.n + row) * a.dv + c0;
+    floatx4 o;
 #pragma unroll
-    for (int ct = 0; ct < DVT; ++ct) {
-      const int c0 = 16 * ct + 4 * lg;
-      if (c0 >= a.dv) continue;
-      floatx4 o;
+    for (int r = 0; r < 4; ++r) o[r] = x[r] / dn;
+    if (a.vec_out) {
+      *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + o0) = o;
+    } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = num[rs][ct][r] / dn;
-      if (a.vec_out) {
-        *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + obase + c0) = o;
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (c0 + r < a.dv) store_elem(a.out, obase + c0 + r, a.out_dtype, o[r]);
-      }
+      for (int r = 0; r < 4; ++r)
+        if (c0 + r < a.dv) store_elem(a.out, o0 + r, a.out_dtype, o[r]);
     }
+  };
+
+  // Planes hold neither infinities nor fp32 values that round to one (above 3.396e38, the type's lowest among
+  // them: a key switched off by a dimension of -inf or the lowest value), and lose the last bits of values whose
+  // lower planes are subnormal.  Either shows in the sums: the first as an infinity or a NaN (inf - inf in the
+  // second plane), the second as values below 2^-95.  A wave with such a row takes its rows again in fp32 matrix
+  // instructions, a strip at a time, the next 16 keys' operands in flight from memory (no barrier: the other
+  // waves are not needed).  Few registers, so that the products above keep theirs: wide values repeat the logits
+  // for each 64 columns.
+  if constexpr (!TAYLOR) {
+    bool again = false;
+    if constexpr (IN == F32 || W == FLASH_EXP) {
+      bool bad = false;
+#pragma unroll
+      for (int rs = 0; rs < RS; ++rs) {
+        float sum[2] = {0.f, 0.f};
+#pragma unroll
+        for (int ct = 0; ct < DVT; ++ct)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) sum[r & 1] += fabsf(num[rs][ct][r]);
+        const float all = sum[0] + sum[1];
+        const bool b = !(all + fabsf(dsum[rs]) < __builtin_huge_valf()) ||
+                       (IN == F32 && all < dsum[rs] * 0x1p-95f && all > 0.f);
+        bad = bad || (b && rvalid[rs]);
+      }
+      again = again || __any(bad);
+    }
+    if (again) {
+      constexpr int CT = DVT < 4 ? DVT : 4, DU = DP / 16;
+#pragma unroll 1
+      for (int job = 0; job < RS * (DVT / CT); ++job) {
+        const int ct0 = job / RS * CT, rbase = r0 + (wave * RS + job % RS) * 16, row = rbase + li;
+        const int lrow = limit(row), jend = min(kend, limit(rbase + 15));
+        // 4 dimensions a lane group and step: columns 16 m + 4 lg of a row
+        auto row_units = [&](floatx4 (&f)[DU], const void* p, int64_t at, bool on, float scale) {
+#pragma unroll
+          for (int m = 0; m < DU; ++m) {
+            const int col = 16 * m + 4 * lg;
+            f[m] = unit_to_f4<ES>(unit_clip<ES>(load_unit<ES>(p, at + min(col, a.ldqk - 4)), on ? a.d - col : 0), IN, scale);
+          }
+        };
+        floatx4 qf[DU], kf[DU], acc[CT];
+        float vf[4][CT], ds = 0.f, top = -1e30f;
+        // keys j0 + li and values of keys j0 + 4 lg + s; those behind jend are zero
+        auto load_keys = [&](int j0) {
+          row_units(kf, a.k, qkbase + static_cast<int64_t>(min(j0 + li, jend - 1)) * a.ldqk, j0 + li < jend, 1.f);
+        };
+        auto load_values = [&](int j0) {
+#pragma unroll
+          for (int s = 0; s < 4; ++s) {
+            const int j = j0 + 4 * lg + s;
+            const int64_t vrow = vbase + static_cast<int64_t>(min(j, jend - 1)) * a.ldv;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+              const int col = 16 * (ct0 + c) + li;
+              const float x = load_elem(a.v, vrow + min(col, a.dv - 1), IN);
+              vf[s][c] = j < jend && col < a.dv ? x : 0.f;
+            }
+          }
+        };
+        row_units(qf, a.q, qkbase + static_cast<int64_t>(row < n ? row : 0) * a.ldqk, row < n, a.scale2);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
+        int b = 0, j0 = offset(0);
+        if (nb > 0 && j0 < jend) {
+          load_keys(j0);
+          load_values(j0);
+        }
+#pragma unroll 1
+        while (b < nb && j0 < jend) {
+          int next = j0 + 16;  // the batch's next 16 keys, or the next batch
+          if (next >= offset(b) + KB) next = offset(++b);
+          const int j = j0;
+          j0 = next;
+          floatx4 x = {0.f, 0.f, 0.f, 0.f};  // keys j + 4 lg + r of the row
+#pragma unroll
+          for (int m = 0; m < DU; ++m)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x = mfma4(kf[m][e], qf[m][e], x);
+          const bool more = b < nb && j0 < jend;
+          if (more) load_keys(j0);
+          float m0 = 0.f;
+          if constexpr (W == FLASH_SOFTMAX) {
+            m0 = top;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (j + 4 * lg + r < lrow) m0 = fmaxf(m0, x[r]);
+            m0 = fmaxf(m0, __shfl_xor(m0, 16));
+            m0 = fmaxf(m0, __shfl_xor(m0, 32));
+            const float alpha = __builtin_amdgcn_exp2f(top - m0);
+            top = m0;
+            ds *= alpha;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[c] *= alpha;
+          }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            x[r] = j + 4 * lg + r < lrow ? __builtin_amdgcn_exp2f(x[r] - m0) : 0.f;
+            ds += x[r];
+          }
+#pragma unroll
+          for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int c = 0; c < CT; ++c) acc[c] = mfma4(vf[s][c], x[s], acc[c]);
+          if (more) load_values(j0);
+        }
+        ds += __shfl_xor(ds, 16);
+        ds += __shfl_xor(ds, 32);
+        if (row < n) {
+          if (ct0 == 0) put_den(row, ds, top);
+#pragma unroll
+          for (int c = 0; c < CT; ++c) put(row, 16 * (ct0 + c) + 4 * lg, ds, acc[c]);
+        }
+      }
+      return;
+    }
+  }
+#pragma unroll
+  for (int rs = 0; rs < RS; ++rs) {
+    if (!rvalid[rs]) continue;
+    put_den(myrow[rs], dsum[rs], mrow[rs]);
+#pragma unroll
+    for (int ct = 0; ct < DVT; ++ct) put(myrow[rs], 16 * ct + 4 * lg, dsum[rs], num[rs][ct]);
   }
 }
 

@@ -190,6 +190,70 @@ def test_exact_tiles_shared_by_workgroups(monkeypatch, heads, n, d, dv, dtype, n
     assert rel(out, exact(q, k, v, 0.1, 1e-12)) < TOL[dtype] + 1e-6
 
 
+MASKS = {"lowest": torch.finfo(torch.float32).min, "-inf": float("-inf")}
+
+
+@pytest.mark.parametrize("heads,n,d,dv,nsplit", [(2, 40, 16, 16, 1), (1, 300, 33, 72, 1), (3, 1025, 64, 64, 5),
+                                                 (1, 130, 128, 200, 2)])
+@pytest.mark.parametrize("mask", sorted(MASKS))
+def test_keys_switched_off_by_a_dimension(monkeypatch, heads, n, d, dv, nsplit, mask):
+    """A key dimension of the type's lowest value or -inf against queries of 1 there: weight 0 for those keys, also
+    for rows that have seen no other key, whose sums are then 0.  fp32 products (1e-6)."""
+    monkeypatch.setattr(_engine, "flash_splits", lambda *a: nsplit)
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(1, heads, n, w, generator=g) for w in (d, d, dv))
+    q[..., 0], k[..., 0] = 1.0, 0.0
+    k[:, :, 5::7, 0] = MASKS[mask]
+    k[:, :, :2, 0] = MASKS[mask]
+    print(heads, n, d, dv, nsplit, mask, flush=True)
+    out = taa.triton_flash_causal_attention(q.to(DEV), k.to(DEV), v.to(DEV), scale=0.4)
+    assert (out[:, :, :2] == 0).all()
+    assert rel(out[:, :, 2:], exact(q, k, v, 0.4)[:, :, 2:]) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("n,d,dv,nsplit", [(300, 64, 64, 1), (700, 16, 40, 3)])
+def test_infinite_and_largest_values(monkeypatch, dtype, n, d, dv, nsplit):
+    """An infinite value makes its column infinite from its row on and leaves the columns beside it, and rows at
+    least a key batch before it, as they are; the largest finite value stays finite under softmax weights."""
+    monkeypatch.setattr(_engine, "flash_splits", lambda *a: nsplit)
+    g = torch.Generator().manual_seed(n)
+    q, k, v = (torch.randn(1, 2, n, w, generator=g).to(dtype) for w in (d, d, dv))
+    at = n // 2 // 64 * 64 + 3
+    vi = v.clone()
+    vi[:, :, at, 3] = float("inf")
+    if dtype != torch.float32:  # the two-plane 16-bit weights of the softmax make inf or NaN of it
+        fns = [(lambda x: faa.fast_article_causal_attention(*x, scale=0.1, compressor="none"), 0.1, 1e-12)]
+    else:
+        fns = [(lambda x: faa.fast_article_causal_attention(*x, scale=0.1, compressor="none"), 0.1, 1e-12),
+               (lambda x: taa.triton_flash_causal_attention(*x, scale=0.1), 0.1, None)]
+    print(n, d, dv, nsplit, dtype, flush=True)
+    for fn, scale, eps in fns:
+        out = fn([x.to(DEV) for x in (q, k, vi)]).cpu()
+        ref = exact(q, k, v, scale, eps)
+        assert (out[:, :, at:, 3] == float("inf")).all()
+        keep = torch.ones(n, dv, dtype=torch.bool)
+        keep[at - 63:, 3] = False
+        assert rel(out[:, :, keep], ref[:, :, keep]) < TOL[dtype] + 1e-6
+    vm = v.clone()
+    vm[:, :, at, 3] = torch.finfo(dtype).max
+    out = taa.triton_flash_causal_attention(*(x.to(DEV) for x in (q, k, vm)), scale=0.1).cpu()
+    ref = exact(q, k, vm, 0.1)
+    rest = torch.arange(dv) != 3
+    tol = 4e-6 if dtype == torch.bfloat16 else 1e-6
+    assert rel(out[:, :, at:, 3] * 2.0 ** -100, ref[:, :, at:, 3] * 2.0 ** -100) < tol
+    assert rel(out[..., rest], ref[..., rest]) < tol
+
+
+@pytest.mark.parametrize("power", [-100, -118])
+def test_tiny_values_keep_their_bits(power):
+    """Values whose lower planes would be subnormal: linear in the values, so 1e-6 as at ordinary sizes."""
+    g = torch.Generator().manual_seed(8)
+    q, k, v = (torch.randn(1, 2, 200, 32, generator=g) for _ in range(3))
+    out = taa.triton_flash_causal_attention(q.to(DEV), k.to(DEV), (v * 2.0 ** power).to(DEV), scale=0.3)
+    assert rel(out.cpu().double() * 2.0 ** -power, exact(q, k, v, 0.3)) < 1e-6
+
+
 def test_exact_split_rule():
     sp = lambda bh, n, w=64: _engine.flash_splits(bh, n, w, w, 256)
     assert [sp(1, 8192), sp(4, 8192), sp(8, 8191), sp(32, 2048), sp(40, 2048), sp(64, 1024), sp(1, 500, 32)] == \
