@@ -417,7 +417,7 @@ int sta_block_attention_split(const void* q, const void* k, const void* v, int d
  *   d <= 128, dv <= 256.  fp32 accumulation; 16-bit inputs' products are exact, fp32 operands are carried
  *   as three bf16 planes (each product within 2^-23 of its exact value for operands of 2^-110 .. 3.39e38 in magnitude).
  *   Rows whose sums come out infinite, NaN or below 2^-95 (infinities, the type's lowest value as a mask, tiny
- *   values) are taken again in fp32 products.
+ *   values) are taken again in fp32 products, as are all rows where ld_qk or ld_v times 64 rows exceeds 1 GiB.
  */
 int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                         int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, void* stream);

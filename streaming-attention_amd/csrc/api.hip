@@ -115,6 +115,9 @@ int flash_args(sta::FlashArgs& a, const void* q, const void* k, const void* v, i
   a = sta::FlashArgs{};
   a.q = q; a.k = k; a.v = v; a.dtype = dtype; a.n = n; a.d = d; a.dv = dv; a.ldqk = ld_qk; a.ldv = ld_v;
   a.bh = bh; a.nsplit = 1;
+  // the staged rows' offsets inside a batch of up to 64 keys stay inside flash_rsrc's 1 GiB
+  const int64_t esize = dtype == STA_F32 ? 4 : 2;
+  a.direct = 64 * esize * std::max<int64_t>(ld_qk, ld_v) > (int64_t(1) << 30) ? 1 : 0;
   return STA_OK;
 }
 
@@ -233,7 +236,7 @@ int sta_pair_moments(const void* q, const void* k, const void* v, int dtype, int
   sta::FlashArgs a;
   if (!low_num || !low_den) return STA_ERR_ARG;
   if (const int st = flash_args(a, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v); st != STA_OK) return st;
-  if (degree < 0 || degree > 3) return STA_ERR_UNSUPPORTED;
+  if (degree < 0 || degree > 3 || a.direct) return STA_ERR_UNSUPPORTED;
   if (chunk <= 0 || shift < 0 || shift >= chunk || (reinterpret_cast<uintptr_t>(low_num) & 15u) != 0) return STA_ERR_ARG;
   if (nsplit <= 0) return STA_ERR_SHAPE;
   a.scale2 = scale;

@@ -74,6 +74,8 @@ struct FlashArgs {
   float* low_den;  // [BH][nsplit][low_rows]
   int64_t low_rows;
   int low_ld, low_off;
+  // 1: row strides so long that a batch's offsets leave the 1 GiB buffers: every row takes the fp32 products
+  int direct;
 };
 
 constexpr int FLASH_ROWS = 128;  // query rows of a workgroup: 4 waves x 2 strips of 16
@@ -446,7 +448,8 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   const int kend = limit(row_hi);
   const int step = a.nsplit;  // this workgroup's batches: split, split + step, ...
   const int nb_all = (kend + KB - 1) / KB;
-  const int nb = (nb_all - split + step - 1) / step;
+  const int nb_own = (nb_all - split + step - 1) / step;
+  const int nb = a.direct ? 0 : nb_own;
   auto offset = [&](int b) { return (split + b * step) * KB; };
 
   // Staging registers: this thread's 4-element units of the next batch's rows, raw: key rows unit by unit,
@@ -624,7 +627,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   // waves are not needed).  Few registers, so that the products above keep theirs: wide values repeat the logits
   // for each 64 columns.
   if constexpr (!TAYLOR) {
-    bool again = false;
+    bool again = a.direct != 0;
     if constexpr (IN == F32 || W == FLASH_EXP) {
       bool bad = false;
 #pragma unroll
@@ -678,12 +681,12 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[c] = floatx4{0.f, 0.f, 0.f, 0.f};
         int b = 0, j0 = offset(0);
-        if (nb > 0 && j0 < jend) {
+        if (nb_own > 0 && j0 < jend) {
           load_keys(j0);
           load_values(j0);
         }
 #pragma unroll 1
-        while (b < nb && j0 < jend) {
+        while (b < nb_own && j0 < jend) {
           int next = j0 + 16;  // the batch's next 16 keys, or the next batch
           if (next >= offset(b) + KB) next = offset(++b);
           const int j = j0;
@@ -693,7 +696,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
           for (int m = 0; m < DU; ++m)
 #pragma unroll
             for (int e = 0; e < 4; ++e) x = mfma4(kf[m][e], qf[m][e], x);
-          const bool more = b < nb && j0 < jend;
+          const bool more = b < nb_own && j0 < jend;
           if (more) load_keys(j0);
           float m0 = 0.f;
           if constexpr (W == FLASH_SOFTMAX) {

@@ -254,6 +254,25 @@ def test_tiny_values_keep_their_bits(power):
     assert rel(out.cpu().double() * 2.0 ** -power, exact(q, k, v, 0.3)) < 1e-6
 
 
+@pytest.mark.parametrize("dtype,ld", [(torch.float32, 1 << 27), (torch.bfloat16, 1 << 28)])
+def test_row_strides_beyond_a_batch_buffer(dtype, ld):
+    """Rows 512 MiB apart (q, k and v side by side in one allocation): the batch offsets leave the 1 GiB buffers."""
+    n, d, dv = 3, 16, 8
+    big = torch.empty(n, ld, device=DEV, dtype=dtype)
+    g = torch.Generator().manual_seed(9)
+    q, k, v = (torch.randn(1, 1, n, w, generator=g).to(dtype) for w in (d, d, dv))
+    for i, x in enumerate((q, k, v)):
+        big[:, 16 * i: 16 * i + x.shape[-1]] = x[0, 0].to(DEV)
+    out = torch.empty(n, dv, device=DEV)
+    lib, es = _native.lib(), big.element_size()
+    print(dtype, ld, flush=True)
+    _native.check(lib.sta_flash_attention(big.data_ptr(), big.data_ptr() + 16 * es, big.data_ptr() + 32 * es,
+                                          _native.DTYPE_CODES[dtype], 1, n, d, dv, ld, ld, 0.3, out.data_ptr(),
+                                          _native.DTYPE_CODES[torch.float32],
+                                          _native.stream_handle(torch.device(DEV))), "sta_flash_attention")
+    assert rel(out, exact(q, k, v, 0.3)[0, 0]) < 1e-6
+
+
 def test_exact_split_rule():
     sp = lambda bh, n, w=64: _engine.flash_splits(bh, n, w, w, 256)
     assert [sp(1, 8192), sp(4, 8192), sp(8, 8191), sp(32, 2048), sp(40, 2048), sp(64, 1024), sp(1, 500, 32)] == \
