@@ -153,23 +153,26 @@ constexpr float LOG2E = 1.44269504f;
 // item) filled up to BA_LIST items at a time, so a batch may span two nodes.  The rows of batch b+1 are
 // loaded into registers while batch b computes (one batch of software pipelining), so the global
 // latency of the gathers is hidden behind the matrix-core work.
-// Two waves per SIMD when the per-wave register arrays (queries, numerators, X and P tiles, prefetched
-// rows) leave room.
 constexpr int BA_LIST = 1024;
 constexpr int BA_MAX_SPLIT = 16;  // ksplit batches of 64 fit a list chunk
 __host__ __device__ constexpr int block_kb(int dp, int dvt) { return (dp + dvt * 16 > 192) ? 32 : 64; }
 __host__ __device__ constexpr int block_kpt(int dp, int dvt) { return (block_kb(dp, dvt) * dp / 4 + 255) / 256; }
-// value units: blocks of 4 keys x 4 columns (2 keys for 16 columns, whose 64 blocks of 4 would leave three waves
-// without one: d = dv = 16, 64 heads x 3000 bf16 levels, a pass 178 us)
-__host__ __device__ constexpr int block_vk(int dvt) { return dvt == 1 ? 2 : 4; }
-__host__ __device__ constexpr int block_vpt(int dp, int dvt) {
-  return (block_kb(dp, dvt) / block_vk(dvt) * dvt * 4 + 255) / 256;
+// value units: blocks of VK keys x 4 columns, VK = 4 where each of the 256 threads has such a block, less where
+// waves would have none (kernel, 64 heads x 3000, d = dv = 32, levels: 70 us with VK = 4, 56 with 2; d = dv = 16
+// fp32: 51.6 with 2, 49.5 with 1)
+__host__ __device__ constexpr int block_vk(int dp, int dvt) {
+  return block_kb(dp, dvt) * dvt >= 256 ? 4 : (block_kb(dp, dvt) * dvt >= 128 ? 2 : 1);
 }
+__host__ __device__ constexpr int block_vpt(int dp, int dvt) {
+  return (block_kb(dp, dvt) / block_vk(dp, dvt) * dvt * 4 + 255) / 256;
+}
+// waves per SIMD by the per-wave register arrays: three where they are small, which the compiler does not keep to
+// by itself (64 heads x 1500, d = dv = 16 flat: 768 tiles are one round of three workgroups a compute unit, 57 us, or
+// two rounds of two, 80 us)
 __host__ __device__ constexpr int block_occupancy(int dp, int dvt, int rs) {
-  return (rs * dp / 4 + rs * dvt * 4 + 2 * rs * (block_kb(dp, dvt) / 16) * 4 +
-          4 * (block_kpt(dp, dvt) + block_vk(dvt) * block_vpt(dp, dvt))) <= 160
-             ? 2
-             : 1;
+  const int regs = rs * dp / 4 + rs * dvt * 4 + 2 * rs * (block_kb(dp, dvt) / 16) * 4 +
+                   4 * (block_kpt(dp, dvt) + block_vk(dp, dvt) * block_vpt(dp, dvt));
+  return regs <= 120 ? 3 : (regs <= 160 ? 2 : 1);
 }
 
 // SPLIT: split-bf16 matrix-core products (the fp32 operands as bf16 hi + lo, three 16x16x32 bf16 products
@@ -522,7 +525,7 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // when written to LDS, so no instruction waits on the loads before the next commit): key rows unit by unit,
   // value rows as blocks of 4 keys x 4 columns, so that the transposed write is one word per column and
   // plane.  Absent rows and columns load from beyond the buffer, which reads as zero.
-  constexpr int VK = block_vk(DVT);
+  constexpr int VK = block_vk(DP, DVT);
   constexpr int KU = DP / 4, VU = DV / 4, KG = KB / VK;
   constexpr int KPT = block_kpt(DP, DVT), VPT = block_vpt(DP, DVT);
   static_assert(256 % KU == 0, "a thread's key units share one column");
@@ -560,6 +563,8 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
           if constexpr (VK == 4) {
             const int4 x = *reinterpret_cast<const int4*>(Lj + off + 4 * g);
             sv[0] = x.x; sv[1] = x.y; sv[2] = x.z; sv[3] = x.w;
+          } else if constexpr (VK == 1) {
+            sv[0] = Lj[off + g];
           } else {
             const int2 x = *reinterpret_cast<const int2*>(Lj + off + 2 * g);
             sv[0] = x.x; sv[1] = x.y;
@@ -603,19 +608,38 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     for (int i = 0; i < VPT; ++i) {
       const int e = tid + 256 * i, g = e % KG, u = e / KG;
       if (KG * VU % 256 != 0 && e >= KG * VU) continue;
+      if constexpr (SPLIT && VK == 1) {  // a key's 4 columns as pairs, one half a column
+        uint32_t h[2], l[2];
+        if constexpr (KVX) {
+          h[0] = pv[i][0].x;
+          h[1] = pv[i][0].y;
+        } else {
+          const floatx4 f = unit_to_f4<ES>(pv[i][0], a.dtype, 1.f);
+          split_pair(f[0], f[1], h[0], l[0]);
+          split_pair(f[2], f[3], h[1], l[1]);
+        }
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+          const int at = (4 * u + m) * LDVB + split_key_pos(g), sh = (m & 1) * 16;
+          Vh[at] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(h[m >> 1] >> sh));
+          if constexpr (!KVX) Vl[at] = __builtin_bit_cast(__bf16, static_cast<uint16_t>(l[m >> 1] >> sh));
+        }
+        continue;
+      }
       // one word a column and plane: VK keys in contraction order (split_key_pos) or in order (fp32)
-      auto put = [&](__bf16* dst, const uint32_t (&w)[VK / 2]) {
+      constexpr int VW = VK < 2 ? 1 : VK / 2;
+      auto put = [&](__bf16* dst, const uint32_t (&w)[VW]) {
         if constexpr (VK == 4)
           *reinterpret_cast<uint2*>(dst) = uint2{w[0], w[1]};
         else
           *reinterpret_cast<uint32_t*>(dst) = w[0];
       };
-      if constexpr (KVX) {
+      if constexpr (KVX && VK > 1) {
         // 16-bit transpose: column m of the VK keys
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
           const uint32_t sel = (m & 1) ? 0x07060302u : 0x05040100u;
-          uint32_t w[VK / 2];
+          uint32_t w[VW];
 #pragma unroll
           for (int c = 0; c < VK; c += 2)
             w[c / 2] = __builtin_amdgcn_perm(m < 2 ? pv[i][c + 1].x : pv[i][c + 1].y, m < 2 ? pv[i][c].x : pv[i][c].y, sel);
@@ -627,8 +651,8 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
         for (int c = 0; c < VK; ++c) f[c] = unit_to_f4<ES>(pv[i][c], a.dtype, 1.f);
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-          if constexpr (SPLIT) {
-            uint32_t h[VK / 2], l[VK / 2];
+          if constexpr (SPLIT && VK > 1) {
+            uint32_t h[VW], l[VW];
 #pragma unroll
             for (int c = 0; c < VK; c += 2) split_pair(f[c][m], f[c + 1][m], h[c / 2], l[c / 2]);
             put(Vh + (4 * u + m) * LDVB + split_key_pos(VK * g), h);

@@ -168,6 +168,20 @@ def test_residual_tiles_shared_by_workgroups(monkeypatch, semantics, bh, n, d, d
     assert rel(outs[1], outs[0].cpu().double()) < 2e-6 + 2 * TOL[out_dtype or dtype]
 
 
+@pytest.mark.parametrize("d,dv", [(16, 16), (8, 5), (32, 16), (128, 16), (256, 12), (24, 24), (64, 32), (256, 32), (256, 64)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_narrow_values_of_the_residual_kernel(d, dv, dtype):
+    """Values staged one, two and four keys a thread, own keys and coreset items: split products (2^-16 each) against
+    fp32 products, plus the rounding of 16-bit outputs."""
+    g = torch.Generator().manual_seed(d + dv)
+    q, k, v = (torch.randn(2, 700, w, generator=g).mul_(0.5 if w == d else 1.0).to(dtype).to(DEV) for w in (d, d, dv))
+    kw = dict(degree=2, block=48, scale=0.2, semantics="flat", out_dtype=dtype)
+    print(d, dv, dtype, flush=True)
+    outs = [_engine.prefill(q, k, v, residual_products=pr, **kw).out
+            for pr in (_native.PRODUCTS_SPLIT_BF16, _native.PRODUCTS_FP32)]
+    assert rel(outs[0], outs[1].cpu().double()) < 2 * TOL[dtype] + 1e-5
+
+
 def test_residual_split_rule():
     flat = lambda n, block: _engine._plan.flat_plan(n, block, "sorted_pair")
     assert _engine.residual_splits(1, flat(1024, 128), 128, 64, 256) == 1
