@@ -382,9 +382,10 @@ def prefill(
 
     # no coreset item takes part (compressor "none", or a sequence inside its first block): the Taylor part
     # and the residual add up to exp, summed over the pairs in one launch.  Keys wider than the pair
-    # kernel's rows, and callers that choose a moment kernel or its products, keep the moment scan.
+    # kernel's rows, clamped logits, and callers that choose a moment kernel or its products keep the moment scan.
     no_items = semantics == "exact" or (semantics == "flat" and n <= block) or (semantics == "levels" and n < block)
-    if no_items and d <= FLASH_D and products is None and residual_products is None and moment_kernel is None:
+    if no_items and d <= FLASH_D and not exp_clamp and products is None and residual_products is None and \
+            moment_kernel is None:
         return PrefillResult(_pairs(q3, k3, v3, scale, eps, out_dtype, timer), None, None, plan,
                              _plan.num_features(d, degree), 0)
 

@@ -61,6 +61,21 @@ def test_sequence_inside_its_first_block(n, block):
     assert rel(out[:, :, :block], ref[:, :, :block]) < (1e-6 if n <= block else 2e-5)  # 2-plane products beyond
 
 
+@pytest.mark.parametrize("semantics,n,block", [("flat", 100, 128), ("exact", 150, 1)])
+def test_clamped_logits_without_items(semantics, n, block):
+    """exp_clamp holds where no coreset item takes part: logits up to 120 weigh exp(80), and a logit of 80
+    rounds to 2^-17, its weight to 8e-6 of itself."""
+    g = torch.Generator().manual_seed(12)
+    q, k = (torch.nn.functional.normalize(torch.randn(2, n, 16, generator=g), dim=-1) for _ in range(2))
+    k[:, ::9] = q[:, ::9]
+    v = torch.randn(2, n, 16, generator=g)
+    out = _engine.prefill(q.to(DEV), k.to(DEV), v.to(DEV), degree=2, block=block, scale=120.0, semantics=semantics,
+                          exp_clamp=True).out
+    x = (q.double() @ k.double().transpose(-1, -2).contiguous() * 120.0).clamp(max=80.0)
+    w = torch.exp(x) * torch.ones(n, n, dtype=torch.float64).tril()
+    assert rel(out, w @ v.double() / w.sum(-1, keepdim=True)) < 3e-5
+
+
 def test_pair_weights_and_the_smallest_denominator():
     """Raw weights far below 1 meet the smallest denominator as in num / max(den, eps); scale 0 is the mean."""
     g = torch.Generator().manual_seed(6)
