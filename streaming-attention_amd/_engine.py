@@ -137,34 +137,57 @@ def pair_splits(bh: int, n: int, compute_units: int) -> int:
 
 
 def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, compute_units: int) -> int:
-    """Workgroups that share a tile of the residual kernel (sta_block_attention_split), width = d + dv: two
-    workgroups a compute unit where the tiles alone are fewer (1 x 4096 fp32, d = dv = 64: kernel 116 -> 39 us with
-    8, 4 x 2048 bf16: 54 -> 33), two a tile up to three tiles for two units (16 x 3000 fp32, 384 tiles: 104 -> 93;
-    440 tiles: 74 -> 86 and left alone), none where the longest tile is so short that the second launch costs
-    the host more (1 x 1024, d = dv = 32: a pass 61 -> 65 us)."""
+    """Workgroups that share a tile of the residual kernel (sta_block_attention_split), width = d + dv, up to three
+    tiles for two compute units (440 tiles on 256: 74 -> 86 us and left alone), by the least estimated time in us.
+    The longest tile by itself takes `alone`; shared, it falls towards the time in which all tiles fill the
+    chip, but the second launch costs the host 6 us, which a pass with less than 27 us here does not win back (1 x 1024,
+    d = dv = 64 bf16, 26 us: a pass 53 -> 60; 4 x 2048, 49 us: 81 -> 61), and the partials are written and read back.
+    Kernel, 1 x 4096 fp32: 116 -> 39 with 8; 4 x 2048 bf16: 54 -> 33.  Passes with 1 | 2 | 4 workgroups, d = dv = 64
+    bf16 unless said, 256 tiles: 8 x 4000 153 | 129 | 135; 32 x 1000 60 | 62 | 74; 64 x 450, d = dv = 128 69 | 85 | 109;
+    16 x 2000, d = dv = 24 93 | 85 (2); 384 tiles: 16 x 3000 fp32 226 | 215 | 226; 48 x 1000 79 | 90 | 104; levels,
+    16 x 3000 161 | 176 | 189."""
     tiles = bh * plan.n_tiles
-    if 2 * tiles > 3 * compute_units:
-        return 1
     most = plan.longest_tile * plan.cap + min(block, plan.n)  # items and keys of the longest tile
-    if most * width < 40000:
+    alone = 2.35e-4 * most * (width + 64)
+    if 2 * tiles > 3 * compute_units or alone < 27:
         return 1
-    want = 2 * compute_units // tiles
-    return max(1, min(max(want, 2), most // 128, 8))
+    part = bh * plan.n * width * 4 / 7e6  # a partial sum, written and read
+    fill = 0.42 * tiles / compute_units
+
+    def estimate(s: int) -> float:
+        if s == 1:
+            return alone
+        if tiles > compute_units:
+            return 0.55 * alone + part * s + 14
+        return alone * max(fill + (1 - fill) / (s * s), 1 / s) + part * s + 8
+
+    return min(range(1, max(1, min(max(2 * compute_units // tiles, 2), most // 128, 8)) + 1), key=estimate)
 
 
-def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int) -> int:
-    """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split): where the tiles leave
-    compute units idle, and up to two tiles a unit where long tiles would meet (d = dv = 64; 1 x 8192 fp32 397 -> 70 us
-    with 8, 4 x 8192 bf16, 256 tiles, 178 -> 88 with 4, 8 x 8191 fp32, 512 tiles, 467 -> 387 with 3, 32 x 2048 113 -> 109
-    with 2).  Each takes at least 128 keys of the longest tile (1024 where no unit is idle: 64 x 1024 63 -> 73 with
-    2); beyond two tiles a unit (40 x 2048 bf16 58 -> 68 with 2) and for calls bound by their launches (1 x 500, d =
-    dv = 32, 14 -> 17) one."""
+def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, element_size: int = 4) -> int:
+    """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split), by the least estimated time
+    in us.  The longest tile by itself takes `alone`; shared by s workgroups it falls towards the time in which all
+    tiles fill the chip, but the s partial sums are written and read back and a second launch adds them (no
+    such call takes less than 23 us, others 17).  Measured passes, d = dv = 64 unless said, with 1 | 2 | 4 | 8
+    workgroups: 1 x 500 fp32 29 | 23 | 23 | 24, bf16 17 | 23 | 23 | 23; 4 x 1000 bf16 28 | 23.5 | 24 | 23; 16 x 1500 fp32
+    78 | 52 | 45 | 53; 32 x 1000 (256 tiles, 256 units) fp32 54 | 41 | 45 | 58, bf16 30 | 32 | 35 | 44; 64 x 512, d = dv = 128
+    fp32 56 | 62 | 84 | 122; 8 x 4000 fp32 196 | 114 | 103 | 112.
+    Between one and two tiles a unit, where long tiles would meet, about three workgroups a unit for tiles of
+    1024 keys each (fp32; 1500 for 16-bit rows: 8 x 8191 fp32 467 -> 387 with 3, 20 x 3000, d = dv = 32 bf16 57 -> 50 with
+    2, 32 x 2048 bf16 55 -> 57 and left alone)."""
     tiles = bh * -(-n // _plan.TILE_ROWS)
-    if n * (d + dv) < 48000 or tiles > 2 * compute_units:
+    if tiles > 2 * compute_units:
         return 1
-    want = min(4 * compute_units // tiles, n // 128, 8) if tiles <= compute_units else \
-        min(6 * compute_units // tiles, n // 1024)
-    return max(1, want)
+    if tiles > compute_units:
+        return max(1, min(6 * compute_units // tiles, n // (1024 if element_size == 4 else 1500)))
+    alone = n * (70 + d + dv) * 2.6e-4 + 4 if element_size == 4 else n * (139 + d + dv) * 8.8e-5 + 5
+    part = bh * n * dv * 8 / 4.5e6  # a partial sum, written and read
+    fill = tiles / (2 * compute_units) * (0.84 if d + dv <= 160 else 1.0)
+
+    def estimate(s: int) -> float:
+        return alone if s == 1 else max(23.3, alone * max(fill + (1 - fill) / (s * s), 1 / s) + part * s + 8)
+
+    return min(range(1, max(1, min(4 * compute_units // tiles, n // 128, 8)) + 1), key=estimate)
 
 
 # Offer the planner the 64-column moment workgroups (split products, 32 < dv <= 64).  Off: on 32 heads x
@@ -675,7 +698,7 @@ def _pairs(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, scale: float, e
     dq, dvp = -(-d // 4) * 4, -(-dv // 4) * 4
     mq, mk, mv = _padded_rows(q3, dq), _padded_rows(k3, dq), _padded_rows(v3, dvp)
     lib = _native.lib()
-    nsplit = flash_splits(bh, n, d, dv, _compute_units(q3.device))
+    nsplit = flash_splits(bh, n, d, dv, _compute_units(q3.device), q3.element_size())
     part_num = part_den = None
     if nsplit > 1:
         part_num = torch.empty((nsplit, bh, n, dvp), device=q3.device, dtype=torch.float32)

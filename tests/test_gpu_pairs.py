@@ -306,3 +306,16 @@ def test_exact_split_rule():
     sp = lambda bh, n, w=64: _engine.flash_splits(bh, n, w, w, 256)
     assert [sp(1, 8192), sp(4, 8192), sp(8, 8191), sp(32, 2048), sp(40, 2048), sp(64, 1024), sp(1, 500, 32)] == \
         [8, 4, 3, 2, 1, 1, 1]
+
+
+def test_splits_that_would_cost_more_than_they_give():
+    """The second launch and the partial sums' traffic: short 16-bit tiles, wide rows in many tiles."""
+    sp = lambda bh, n, w, es: _engine.flash_splits(bh, n, w, w, 256, es)
+    assert [sp(4, 500, 64, 2), sp(32, 700, 64, 2), sp(64, 512, 128, 2), sp(64, 512, 128, 4), sp(32, 2048, 64, 2)] == [1] * 5
+    assert sp(4, 500, 64, 4) > 1 and sp(1, 1500, 16, 4) > 1 and sp(4, 8192, 64, 2) > 1
+    flat = lambda n, block: _engine._plan.flat_plan(n, block, "sorted_pair")
+    levels = lambda n, block: _engine._plan.levels_plan(n, block, "sorted_pair")
+    assert _engine.residual_splits(64, flat(450, 128), 128, 256, 256) == 1
+    assert _engine.residual_splits(48, flat(1000, 128), 128, 128, 256) == 1
+    assert _engine.residual_splits(16, levels(3000, 128), 128, 128, 256) == 1
+    assert _engine.residual_splits(1, levels(4096, 256), 256, 128, 256) > 1
