@@ -357,11 +357,18 @@ class DecodeState:
         views = [flat[o: o + n].view(t).view(shape) for (o, n, shape), t in
                  zip(spans, ([torch.int32, real, real] + ([torch.int32] if perm else [])) * count)]
         out, per = [], 4 if perm else 3
+        if not perm:  # one table of zeros for all of them
+            none = torch.zeros(self.S * max(len(ms) for ms in methods) * max_in, device=self.device, dtype=torch.int32)
         for i, ms in enumerate(methods):
             v = views[per * i: per * i + per]
-            pm = v[3] if perm else torch.zeros((self.S, len(ms), max_in), device=self.device, dtype=torch.int32)
+            pm = v[3] if perm else none[: self.S * len(ms) * max_in].view(self.S, len(ms), max_in)
             out.append(_CompletionDraws(first + i, len(ms), v[0], v[1], v[2], pm))
         return out
+
+    def _draw_group(self) -> int:
+        """Completions whose tables (two calls each in the mean) take about 64 MiB on the device, at least one."""
+        per = self.S * (2 * self.d + 3 * self.block) * 4 * (2 if self.score_f64 else 1)
+        return max(1, (64 << 20) // per)
 
     def reserve_draws(self, tokens: int) -> int:
         """Draw ahead, on the host, the compress calls of every block completion within the next
@@ -370,9 +377,7 @@ class DecodeState:
             return 0
         queued_to = self.blocks + len(self._draws)
         last = (self.length + tokens) // self.block
-        # about 64 MiB of tables at a time
-        per = self.S * (2 * self.d + 3 * self.block) * 4 * (2 if self.score_f64 else 1)
-        group = max(1, (64 << 20) // per)
+        group = self._draw_group()  # an upload each; all of them stay on the device until their blocks complete
         for c in range(queued_to, last, group):
             self._draws.extend(self._draw_completions(c, min(group, last - c)))
         return len(self._draws)
@@ -609,8 +614,8 @@ class DecodeState:
                 vp[:, koff: koff + hi - lo, : self.dv] = v[:, lo:hi]
             self._accumulate(kp, vp, hi - lo, kp.shape[1], self.state_num, self.state_den, row_off=koff)
             for b in range(nb):
-                if not self._draws:  # the draws of the next blocks, at most 64 ahead
-                    self.reserve_draws(min(nb - b, 64) * self.block)
+                if not self._draws:  # one upload's worth of the next blocks' draws, at most 64 ahead
+                    self.reserve_draws(min(nb - b, 64, self._draw_group()) * self.block)
                 to_buffer(lo + b * self.block, lo + (b + 1) * self.block)
                 self._complete_block(accumulate=False)
             i = hi

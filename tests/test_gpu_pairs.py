@@ -162,6 +162,33 @@ def test_few_streams_tail_matches_many(d, dv, block, tokens, fused):
     assert rel(outs[0], outs[1].cpu().double()) < 2e-6
 
 
+@pytest.mark.parametrize("compressor", ["sorted_pair", "random"])
+def test_bulk_draws_ahead_are_bounded(compressor):
+    """extend() keeps one upload of draws (64 MiB by its estimate of two calls a completion, half as much again for
+    the calls of a run of completions), however many blocks it takes, and draws what single blocks draw."""
+    kw = dict(degree=1, block_size=128, streams=2048, compressor=compressor)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    k, v = (torch.randn(2048, 40 * 128, 8, device=DEV, generator=g) for _ in range(2))
+    a, b = (stc.ArticleStreamingAttention(8, 8, **kw) for _ in range(2))
+    sizes, draw = [], a._st._draw_completions
+
+    def counted(first, count):
+        out = draw(first, count)
+        held = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes()
+                for dr in list(a._st._draws) + out for t in (dr.methods, dr.dirs, dr.unif, dr.perms)}
+        sizes.append(sum(held.values()))
+        return out
+
+    a._st._draw_completions = counted
+    a.extend(k, v)
+    assert len(sizes) > 1 and max(sizes) <= 96 << 20
+    for i in range(40):
+        b.extend(k[:, 128 * i: 128 * i + 128].contiguous(), v[:, 128 * i: 128 * i + 128].contiguous())
+    for x, y in zip(a._st.level_items(), b._st.level_items()):
+        assert (x is None) == (y is None)
+        assert x is None or all(torch.equal(s, t) for s, t in zip(x, y))
+
+
 @pytest.mark.parametrize("semantics,bh,n,d,dv,degree,block,dtype,out_dtype", [
     ("flat", 1, 1100, 64, 64, 2, 64, torch.float32, torch.float32), ("flat", 2, 4300, 16, 30, 2, 100, torch.bfloat16, None),
     ("levels", 1, 3000, 40, 72, 2, 48, torch.float16, None), ("levels", 3, 200, 128, 200, 3, 128, torch.float32, None),
