@@ -98,6 +98,29 @@ def make_inputs(batch, heads, n, d, dv, seed, radius=1.0, ball=True):
     return q / qn * rq, k / kn * rk, v
 
 
+def moments_roofline(kernel: str, bh: int, n: int, d: int, dv: int, degree: int, block: int, shift: int, dtype: str):
+    """What the launch timed as "moments" does, by the kernel that ran: its name, algorithmic flops and the peak of
+    the products it takes.  The scan updates and queries F features a token; over the pairs (short sequences) a row
+    takes the keys before its block."""
+    import _engine
+    import _plan
+
+    if kernel == "flash_attn_kernel":
+        keys = sum(max(0, (i + shift) // block * block - shift) for i in range(n))
+        qk, pv = 2.0 * d, 2.0 * (dv + 1)
+        x, p = {"fp32": (3, 5), "bf16": (1, 3), "fp16": (1, 5)}[dtype]  # bf16 products of a product
+        return {"kernel": "flash_attn_kernel (Taylor part over the pairs)", "flops": (qk + pv) * keys * bh,
+                "peak": MFMA_BF16_PEAK_TFLOPS * (qk + pv) / (x * qk + p * pv), "products": f"split-bf16 {x} + {p}",
+                "peak_basis": f"bf16 dense peak over {x} bf16 matrix-core products for QK^T and {p} for PV, by their flops"}
+    f = _plan.num_features(d, degree)
+    split = _engine.MOMENT_PRODUCTS == _engine._native.PRODUCTS_SPLIT_BF16
+    return {"kernel": f"{kernel} (K1, exact Taylor moment scan)",
+            "flops": 4.0 * f * (dv + 1) * bh * n,  # update + query, 2*F*(dv+1) each per head-token
+            "peak": SPLIT_BF16_PEAK_TFLOPS if split else MFMA_FP32_PEAK_TFLOPS, "products": "split-bf16" if split else "fp32",
+            "peak_basis": ("fp32-equivalent flops of split-bf16 products: bf16 dense peak / 3 (three bf16 "
+                           "matrix-core products per fp32 product)" if split else "fp32 matrix-core peak")}
+
+
 def measured_traffic(workload: str, kernel: str):
     """HBM bytes per launch of `kernel` from the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of
     this workload (calibrated against a copy of known size), or None when there is none."""
@@ -401,13 +424,11 @@ def main() -> int:
     _plan.draws_for(plan, _plan.sequence_seeds(w["seed"] + 7919 * 5, bh), d, w["compressor"])
     draws_ms = (time.perf_counter() - t0) * 1e3
 
-    f = _plan.num_features(d, w["degree"])
-    mom_flops = 4.0 * f * (dv + 1) * bh * n  # algorithmic: update + query, 2*F*(dv+1) each per head-token
+    roof = moments_roofline(res.moment_kernel, bh, n, d, dv, w["degree"], w["block"], plan.shift, w["dtype"])
+    mom_flops, peak = roof["flops"], roof["peak"]
     mom_ms = mom_tot / mom_launches
     achieved = mom_flops / (mom_ms * 1e-3) / 1e12
     value = bh * n / (ms_step * 1e-3)
-    split = _engine.MOMENT_PRODUCTS == _engine._native.PRODUCTS_SPLIT_BF16
-    peak = SPLIT_BF16_PEAK_TFLOPS if split else MFMA_FP32_PEAK_TFLOPS
 
     line = {
         "metric": "head-tokens/sec, N=64K d=64 deg-2; % of HBM/MFMA roofline",
@@ -426,15 +447,14 @@ def main() -> int:
         "data": "synthetic",
         "config": w,
         "roofline": {
-            "kernel": f"{res.moment_kernel} (K1, exact Taylor moment scan)",
+            "kernel": roof["kernel"],
             "bound": "mfma",
             "achieved": achieved,
             "peak": peak,
             "unit": "TFLOP/s",
             "frac": achieved / peak,
-            "products": "split-bf16" if split else "fp32",
-            "peak_basis": ("fp32-equivalent flops of split-bf16 products: bf16 dense peak / 3 (three bf16 "
-                           "matrix-core products per fp32 product)" if split else "fp32 matrix-core peak"),
+            "products": roof["products"],
+            "peak_basis": roof["peak_basis"],
             "traffic": measured_traffic(w["workload"], res.moment_kernel),
             # the same fp32-equivalent rate against the bound fp32 matrix-core products would have
             "achieved_vs_fp32_mfma_peak": achieved / MFMA_FP32_PEAK_TFLOPS,

@@ -19,6 +19,18 @@ def test_measured_traffic_reads_the_committed_profiles():
     assert bench.measured_traffic("no_such_workload", "moments_ws_kernel") is None
 
 
+def test_moments_roofline_is_of_the_kernel_that_ran():
+    scan = bench.moments_roofline("moments_ws_kernel", 32, 65536, 64, 64, 2, 256, 1, "fp32")
+    assert "moment scan" in scan["kernel"] and scan["flops"] == 4.0 * 2145 * 65 * 32 * 65536
+    assert abs(scan["peak"] - bench.MFMA_BF16_PEAK_TFLOPS / 3) < 1e-9
+    pairs = bench.moments_roofline("flash_attn_kernel", 128, 4096, 64, 64, 2, 256, 0, "bf16")
+    keys = 256 * 256 * (16 * 15 // 2)  # 256 rows a block, 256 b keys before block b
+    assert "pairs" in pairs["kernel"] and pairs["flops"] == (2 * 64 + 2 * 65) * keys * 128
+    assert bench.MFMA_BF16_PEAK_TFLOPS / 3 < pairs["peak"] < bench.MFMA_BF16_PEAK_TFLOPS
+    levels = bench.moments_roofline("flash_attn_kernel", 1, 4, 16, 16, 2, 2, 1, "fp32")
+    assert levels["flops"] == (2 * 16 + 2 * 17) * (0 + 1 + 1 + 3)
+
+
 def test_host_cpus_describes_the_host():
     info, usable = bench.host_cpus()
     assert usable >= 1 and info["os_cpu_count"] >= 1 and info["cpus_allowed"] >= usable
