@@ -372,7 +372,8 @@ int sta_segment_mean(const void* k, const void* v, int dtype, int64_t bh, int64_
  *     rep_k/rep_v instead of k/v).
  *   low_num / low_den: sta_moments' (or sta_moments_ws') partial outputs (sta_moment_partials_layout),
  *     fsplit splits; chunk: their chunk (sta_moment_chunk) or query block, a multiple of the moment
- *     chunk that divides or is a multiple of the tile rows.
+ *     chunk that divides or is a multiple of the tile rows; or sta_pair_moments' partials, any chunk.
+ *     A head's rows span at most 4 GiB (STA_ERR_UNSUPPORTED beyond), as in sta_moments.
  *   ld_qk / ld_v: row strides (elements) of q, k and of v, multiples of 4 (rows are read in units of
  *     4 elements; pad them with zero columns), bases 16-byte aligned.
  *   rep_k / rep_v (fp32, row strides ld_rep_k / ld_rep_v, multiples of 4): materialized items
@@ -423,22 +424,20 @@ int sta_flash_attention(const void* q, const void* k, const void* v, int dtype, 
                         int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, void* stream);
 
 /*
- * Exact causal attention with the article's unnormalised weights (compressor "none",
- * fast_article_attention.py:437-464, :596-598: the Taylor part and the residual over every earlier key add up
- * to exp):  out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum_{j<=i} exp(s q_i.k_j), eps).
- * Arguments as sta_flash_attention; the weights keep fp32 accuracy for every input type.
- */
-int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
-                        int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream);
-
-/*
- * sta_flash_attention / sta_exact_attention with a tile's key batches dealt out to nsplit >= 1 workgroups, for
- * grids that leave compute units idle: raw sums to part_num [nsplit][BH][N][4 ceil(Dv / 4)], denominators and row
- * maxima to part_den [nsplit][BH][N][2] (both 16-byte aligned), added and normalised by a second launch.
+ * sta_flash_attention with a tile's key batches dealt out to nsplit >= 1 workgroups, for grids that leave compute
+ * units idle: raw sums to part_num [nsplit][BH][N][4 ceil(Dv / 4)], denominators and row maxima to part_den
+ * [nsplit][BH][N][2] (both 16-byte aligned, NULL with nsplit 1), added and normalised by a second launch.
  */
 int sta_flash_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                               int dv, int ld_qk, int ld_v, float scale, void* out, int out_dtype, int nsplit,
                               float* part_num, float* part_den, void* stream);
+
+/*
+ * Exact causal attention with the article's unnormalised weights (compressor "none",
+ * fast_article_attention.py:437-464, :596-598: the Taylor part and the residual over every earlier key add up
+ * to exp):  out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum_{j<=i} exp(s q_i.k_j), eps).
+ * Arguments as sta_flash_attention_split; the weights keep fp32 accuracy for every input type.
+ */
 int sta_exact_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                               int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, int nsplit,
                               float* part_num, float* part_den, void* stream);

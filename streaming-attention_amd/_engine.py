@@ -235,7 +235,7 @@ def _unit_width(width: int, element_size: int) -> int:
     return -(-width // per_unit) * per_unit
 
 
-FLASH_D = 128  # key dimensions of the pair kernel (sta_flash_attention, sta_exact_attention)
+FLASH_D = 128  # key dimensions of the pair kernel (sta_flash_attention_split, sta_exact_attention_split)
 STAGED_D = 128  # key dimensions the moment kernels stage whole; wider keys go through dimension windows
 MAX_D_HIGH_DEGREE = 64  # degree 5 .. 8
 

@@ -102,9 +102,6 @@ _SIGNATURES = {
     "sta_flash_attention": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _c_p, _i32, _c_p],
     ),
-    "sta_exact_attention": (
-        _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _f32, _c_p, _i32, _c_p],
-    ),
     "sta_flash_attention_split": (
         _i32, [_c_p, _c_p, _c_p, _i32, _i64, _i64, _i32, _i32, _i32, _i32, _f32, _c_p, _i32, _i32, _c_p, _c_p, _c_p],
     ),

@@ -217,12 +217,6 @@ int sta_flash_attention_split(const void* q, const void* k, const void* v, int d
                       nsplit, part_num, part_den, stream);
 }
 
-int sta_exact_attention(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
-                        int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, void* stream) {
-  return flash_launch(sta::FLASH_EXP, q, k, v, dtype, bh, n, d, dv, ld_qk, ld_v, scale, eps, out, out_dtype, 1, nullptr,
-                      nullptr, stream);
-}
-
 int sta_exact_attention_split(const void* q, const void* k, const void* v, int dtype, int64_t bh, int64_t n, int d,
                               int dv, int ld_qk, int ld_v, float scale, float eps, void* out, int out_dtype, int nsplit,
                               float* part_num, float* part_den, void* stream) {

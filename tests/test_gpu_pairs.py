@@ -1,5 +1,5 @@
-"""The pair kernel (sta_flash_attention, sta_exact_attention) at the edges of its tiles, key batches and tile
-orders, against float64 attention.  fp32 operands as three bf16 planes keep each product within 2^-23 of its
+"""The pair kernel (sta_flash_attention_split, sta_exact_attention_split, sta_pair_moments) at the edges of its
+tiles, key batches and tile orders, against float64 attention.  fp32 operands as three bf16 planes keep each product within 2^-23 of its
 value and the sums are fp32: a few 2^-23 in the 2-norm (1e-6).  bf16 weights as hi + lo planes of 8 bits are
 within 2^-16 each, uniform and of random sign (4e-6 at most in the 2-norm).  16-bit outputs add their rounding:
 half a unit in the last of 8 (bf16) or 11 (fp16) bits at most, uniform, so 2^-8 / sqrt(3) or 2^-11 / sqrt(3)."""
