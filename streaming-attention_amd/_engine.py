@@ -164,28 +164,36 @@ def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, com
     return min(range(1, max(1, min(max(2 * compute_units // tiles, 2), most // 128, 8)) + 1), key=estimate)
 
 
-def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, element_size: int = 4) -> int:
-    """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split), by the least estimated time
-    in us.  The longest tile by itself takes `alone`; shared by s workgroups it falls towards the time in which all
-    tiles fill the chip, but the s partial sums are written and read back and a second launch adds them (no
-    such call takes less than 23 us, others 17).  Measured passes, d = dv = 64 unless said, with 1 | 2 | 4 | 8
-    workgroups: 1 x 500 fp32 29 | 23 | 23 | 24, bf16 17 | 23 | 23 | 23; 4 x 1000 bf16 28 | 23.5 | 24 | 23; 16 x 1500 fp32
-    78 | 52 | 45 | 53; 32 x 1000 (256 tiles, 256 units) fp32 54 | 41 | 45 | 58, bf16 30 | 32 | 35 | 44; 64 x 512, d = dv = 128
-    fp32 56 | 62 | 84 | 122; 8 x 4000 fp32 196 | 114 | 103 | 112.
+def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, dtype: torch.dtype = torch.float32,
+                 softmax: bool = True) -> int:
+    """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split; softmax False:
+    sta_exact_attention_split), by the least estimated time in us.  The longest tile by itself takes `alone`; shared by
+    s workgroups it falls towards the time in which all tiles fill the chip, but the s partial sums are written and
+    read back and a second launch adds them: no softmax call with one takes less than 23 us (17 without), no call of
+    the fast path less than 33 (26).  Measured passes, d = dv = 64 unless said, with 1 | 2 | 4 | 8 workgroups: softmax 1 x
+    500 fp32 29 | 23 | 23 | 24, bf16 17 | 23 | 23 | 23; 4 x 1000 bf16 28 | 23.5 | 24 | 23; 16 x 1500 fp32 78 | 52 | 45 | 53; 32 x
+    1000 (256 tiles, 256 units) fp32 54 | 41 | 45 | 58, bf16 30 | 32 | 35 | 44; 64 x 512, d = dv = 128 fp32 56 | 62 | 84 | 122;
+    8 x 4000 fp32 196 | 114 | 103 | 112; exp 4 x 500 fp32 29 | 32 | 32 | 32; 32 x 1000 fp16 40 | 34 | 36 | 44.
     Between one and two tiles a unit, where long tiles would meet, about three workgroups a unit for tiles of
-    1024 keys each (fp32; 1500 for 16-bit rows: 8 x 8191 fp32 467 -> 387 with 3, 20 x 3000, d = dv = 32 bf16 57 -> 50 with
-    2, 32 x 2048 bf16 55 -> 57 and left alone)."""
+    1024 keys each (1500 for the 16-bit softmax: 20 x 3000, d = dv = 32 bf16 57 -> 50 with 2, 32 x 2048 bf16 55 -> 57 and
+    left alone; exp 64 -> 59)."""
     tiles = bh * -(-n // _plan.TILE_ROWS)
     if tiles > 2 * compute_units:
         return 1
+    f32 = dtype == torch.float32
     if tiles > compute_units:
-        return max(1, min(6 * compute_units // tiles, n // (1024 if element_size == 4 else 1500)))
-    alone = n * (70 + d + dv) * 2.6e-4 + 4 if element_size == 4 else n * (139 + d + dv) * 8.8e-5 + 5
+        return max(1, min(6 * compute_units // tiles, n // (1024 if f32 or not softmax else 1500)))
+    alone = n * (70 + d + dv) * 2.6e-4 + 4 if f32 else n * (135 + d + dv) * 8.5e-5 + 5 + 0.016 * (d + dv)
+    if not (f32 or softmax):  # three weight planes against one value plane, two for fp16
+        alone += n * dv * (1.45e-4 if dtype == torch.float16 else 8.5e-5)
+    if dv > 128:  # one workgroup a unit
+        alone *= 1.5
     part = bh * n * dv * 8 / 4.5e6  # a partial sum, written and read
     fill = tiles / (2 * compute_units) * (0.84 if d + dv <= 160 else 1.0)
+    least = 23.3 if softmax else 33.0
 
     def estimate(s: int) -> float:
-        return alone if s == 1 else max(23.3, alone * max(fill + (1 - fill) / (s * s), 1 / s) + part * s + 8)
+        return alone if s == 1 else max(least, alone * max(fill + (1 - fill) / (s * s), 1 / s) + part * s + 8)
 
     return min(range(1, max(1, min(4 * compute_units // tiles, n // 128, 8)) + 1), key=estimate)
 
@@ -698,7 +706,7 @@ def _pairs(q3: torch.Tensor, k3: torch.Tensor, v3: torch.Tensor, scale: float, e
     dq, dvp = -(-d // 4) * 4, -(-dv // 4) * 4
     mq, mk, mv = _padded_rows(q3, dq), _padded_rows(k3, dq), _padded_rows(v3, dvp)
     lib = _native.lib()
-    nsplit = flash_splits(bh, n, d, dv, _compute_units(q3.device), q3.element_size())
+    nsplit = flash_splits(bh, n, d, dv, _compute_units(q3.device), q3.dtype, eps is None)
     part_num = part_den = None
     if nsplit > 1:
         part_num = torch.empty((nsplit, bh, n, dvp), device=q3.device, dtype=torch.float32)

@@ -337,9 +337,12 @@ def test_exact_split_rule():
 
 def test_splits_that_would_cost_more_than_they_give():
     """The second launch and the partial sums' traffic: short 16-bit tiles, wide rows in many tiles."""
-    sp = lambda bh, n, w, es: _engine.flash_splits(bh, n, w, w, 256, es)
-    assert [sp(4, 500, 64, 2), sp(32, 700, 64, 2), sp(64, 512, 128, 2), sp(64, 512, 128, 4), sp(32, 2048, 64, 2)] == [1] * 5
-    assert sp(4, 500, 64, 4) > 1 and sp(1, 1500, 16, 4) > 1 and sp(4, 8192, 64, 2) > 1
+    b16, f16, f32 = torch.bfloat16, torch.float16, torch.float32
+    sp = lambda bh, n, w, dt, softmax=True: _engine.flash_splits(bh, n, w, w, 256, dt, softmax)
+    assert [sp(4, 500, 64, b16), sp(32, 700, 64, f16), sp(64, 512, 128, b16), sp(64, 512, 128, f32), sp(32, 2048, 64, b16),
+            sp(4, 500, 64, f32, False), sp(4, 500, 64, b16, False), sp(32, 700, 64, f16, False)] == [1] * 8
+    assert sp(4, 500, 64, f32) > 1 and sp(1, 1500, 16, f32) > 1 and sp(4, 8192, 64, b16) > 1
+    assert sp(32, 1000, 64, f16, False) > 1 and sp(4, 1500, 64, b16, False) > 1 and sp(32, 2048, 64, b16, False) > 1
     flat = lambda n, block: _engine._plan.flat_plan(n, block, "sorted_pair")
     levels = lambda n, block: _engine._plan.levels_plan(n, block, "sorted_pair")
     assert _engine.residual_splits(64, flat(450, 128), 128, 256, 256) == 1
