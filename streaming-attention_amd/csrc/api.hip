@@ -148,6 +148,10 @@ int flash_launch(int weight, const void* q, const void* k, const void* v, int dt
   a.out = out; a.out_dtype = out_dtype;
   a.vec_out = (out_dtype == STA_F32 && dv % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) ? 1 : 0;
   a.nsplit = nsplit; a.low_num = part_num; a.low_den = part_den; a.low_ld = (dv + 3) / 4 * 4;
+  if (a.direct && weight == sta::FLASH_SOFTMAX && dtype != STA_F32) {
+    weight = sta::FLASH_EXP;
+    a.direct = 2;
+  }
   const int st = flash_dispatch(a, weight, stream);
   if (st != STA_OK || nsplit == 1) return st;
   const int64_t blocks = (bh * n * (a.low_ld / 4) + 255) / 256;

@@ -74,7 +74,8 @@ struct FlashArgs {
   float* low_den;  // [BH][nsplit][low_rows]
   int64_t low_rows;
   int low_ld, low_off;
-  // 1: row strides so long that a batch's offsets leave the 1 GiB buffers: every row takes the fp32 products
+  // 1: row strides so long that a batch's offsets leave the 1 GiB buffers: every row takes the fp32 products; 2: the
+  // softmax of 16-bit rows so, which FLASH_EXP's kernel takes (the 16-bit softmax has no fp32 products of its own)
   int direct;
 };
 
@@ -111,7 +112,7 @@ __host__ __device__ constexpr int flash_occupancy(int dp, int dvt, int in, int w
   const int unit = in == F32 ? 4 : 2;
   const int regs = flash_kp(in, w) * 2 * flash_dps(dp) / 8 + 2 * dvt * 4 + 2 * (kb / 16) * 4 +
                    unit * ((kb * dp / 4 + 255) / 256 + 4 * ((kb / 4 * dvt * 4 + 255) / 256));
-  return regs <= 100 && in != F32 ? 3 : (regs <= 176 ? 2 : 1);
+  return regs <= (in == F32 && w == FLASH_EXP ? 112 : 100) ? 3 : (regs <= 176 ? 2 : 1);
 }
 
 __host__ __device__ constexpr int flash_key_pos(int r) {
@@ -449,7 +450,8 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   const int step = a.nsplit;  // this workgroup's batches: split, split + step, ...
   const int nb_all = (kend + KB - 1) / KB;
   const int nb_own = (nb_all - split + step - 1) / step;
-  const int nb = a.direct ? 0 : nb_own;
+  constexpr bool FP32_ROWS = !TAYLOR && (IN == F32 || W == FLASH_EXP);  // has fp32 products of its own (below)
+  const int nb = FP32_ROWS && a.direct ? 0 : nb_own;
   auto offset = [&](int b) { return (split + b * step) * KB; };
 
   // Staging registers: this thread's 4-element units of the next batch's rows, raw: key rows unit by unit,
@@ -572,53 +574,6 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
     }
   }
 
-  // ---- epilogue: row sums (over the four lane groups), normalise, store ----
-  float dsum[RS];
-#pragma unroll
-  for (int rs = 0; rs < RS; ++rs) {
-    if constexpr (DENM) {
-      dsum[rs] = dacc[rs][0];  // every element of the column is the row's sum
-    } else {
-      dsum[rs] = den[rs];
-      dsum[rs] += __shfl_xor(dsum[rs], 16);
-      dsum[rs] += __shfl_xor(dsum[rs], 32);
-    }
-  }
-  auto put_den = [&](int row, float ds, float mr) {
-    if (lg != 0) return;
-    if constexpr (TAYLOR)
-      a.low_den[(bh * a.nsplit + split) * a.low_rows + a.low_off + row] = ds;
-    else if (a.nsplit > 1)
-      *reinterpret_cast<floatx2*>(a.low_den + 2 * ((split * a.bh + bh) * a.n + row)) =
-          floatx2{ds, W == FLASH_SOFTMAX ? mr : 0.f};
-  };
-  auto put = [&](int row, int c0, float ds, const floatx4& x) {  // columns c0 .. c0 + 3
-    if constexpr (TAYLOR) {
-      const int64_t lrow = (bh * a.nsplit + split) * a.low_rows + a.low_off + row;
-      if (c0 < a.dv)  // low_ld is whole 32-column groups
-        *reinterpret_cast<floatx4*>(a.low_num + lrow * a.low_ld + c0) = x;
-      return;
-    }
-    if (a.nsplit > 1) {
-      if (c0 < a.low_ld)
-        *reinterpret_cast<floatx4*>(a.low_num + ((split * a.bh + bh) * a.n + row) * a.low_ld + c0) = x;
-      return;
-    }
-    if (c0 >= a.dv) return;
-    const float dn = fmaxf(ds, a.floor);
-    const int64_t o0 = (bh * a.n + row) * a.dv + c0;
-    floatx4 o;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = x[r] / dn;
-    if (a.vec_out) {
-      *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + o0) = o;
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (c0 + r < a.dv) store_elem(a.out, o0 + r, a.out_dtype, o[r]);
-    }
-  };
-
   // Planes hold neither infinities nor fp32 values that round to one (above 3.396e38, the type's lowest among
   // them: a key switched off by a dimension of -inf or the lowest value), and lose the last bits of values whose
   // lower planes are subnormal.  Either shows in the sums: the first as an infinity or a NaN (inf - inf in the
@@ -626,26 +581,27 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
   // instructions, a strip at a time, the next 16 keys' operands in flight from memory (no barrier: the other
   // waves are not needed).  Few registers, so that the products above keep theirs: wide values repeat the logits
   // for each 64 columns.
-  if constexpr (!TAYLOR) {
-    bool again = a.direct != 0;
-    if constexpr (IN == F32 || W == FLASH_EXP) {
-      bool bad = false;
+  if constexpr (FP32_ROWS) {
+    bool bad = false;
 #pragma unroll
-      for (int rs = 0; rs < RS; ++rs) {
-        float sum[2] = {0.f, 0.f};
+    for (int rs = 0; rs < RS; ++rs) {
+      float sum[2] = {0.f, 0.f};
 #pragma unroll
-        for (int ct = 0; ct < DVT; ++ct)
+      for (int ct = 0; ct < DVT; ++ct)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) sum[r & 1] += fabsf(num[rs][ct][r]);
-        const float all = sum[0] + sum[1];
-        const bool b = !(all + fabsf(dsum[rs]) < __builtin_huge_valf()) ||
-                       (IN == F32 && all < dsum[rs] * 0x1p-95f && all > 0.f);
-        bad = bad || (b && rvalid[rs]);
+        for (int r = 0; r < 4; ++r) sum[r & 1] += fabsf(num[rs][ct][r]);
+      float ds = DENM ? dacc[rs][0] : den[rs];
+      if constexpr (!DENM) {
+        ds += __shfl_xor(ds, 16);
+        ds += __shfl_xor(ds, 32);
       }
-      again = again || __any(bad);
+      const float all = sum[0] + sum[1];
+      const bool b = !(all + fabsf(ds) < __builtin_huge_valf()) || (IN == F32 && all < ds * 0x1p-95f && all > 0.f);
+      bad = bad || (b && rvalid[rs]);
     }
-    if (again) {
+    if (__builtin_expect(a.direct != 0 || __any(bad), false)) {
       constexpr int CT = DVT < 4 ? DVT : 4, DU = DP / 16;
+      const bool softmax = W == FLASH_SOFTMAX || (IN != F32 && a.direct == 2);
 #pragma unroll 1
       for (int job = 0; job < RS * (DVT / CT); ++job) {
         const int ct0 = job / RS * CT, rbase = r0 + (wave * RS + job % RS) * 16, row = rbase + li;
@@ -699,7 +655,7 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
           const bool more = b < nb_own && j0 < jend;
           if (more) load_keys(j0);
           float m0 = 0.f;
-          if constexpr (W == FLASH_SOFTMAX) {
+          if (softmax) {
             m0 = top;
 #pragma unroll
             for (int r = 0; r < 4; ++r)
@@ -725,21 +681,75 @@ __global__ __launch_bounds__(256, flash_occupancy(DP, DVT, IN, W)) void flash_at
         }
         ds += __shfl_xor(ds, 16);
         ds += __shfl_xor(ds, 32);
-        if (row < n) {
-          if (ct0 == 0) put_den(row, ds, top);
+        if (row >= n) continue;
+        const int64_t part = (split * a.bh + bh) * a.n + row, obase = (bh * a.n + row) * a.dv;
+        if (a.nsplit > 1 && lg == 0 && ct0 == 0)
+          *reinterpret_cast<floatx2*>(a.low_den + 2 * part) = floatx2{ds, softmax ? top : 0.f};
+        const float dn = fmaxf(ds, a.floor);
 #pragma unroll
-          for (int c = 0; c < CT; ++c) put(row, 16 * (ct0 + c) + 4 * lg, ds, acc[c]);
+        for (int c = 0; c < CT; ++c) {
+          const int c0 = 16 * (ct0 + c) + 4 * lg;
+          if (a.nsplit > 1) {
+            if (c0 < a.low_ld) *reinterpret_cast<floatx4*>(a.low_num + part * a.low_ld + c0) = acc[c];
+          } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              if (c0 + r < a.dv) store_elem(a.out, obase + c0 + r, a.out_dtype, acc[c][r] / dn);
+          }
         }
       }
       return;
     }
   }
+  // ---- epilogue: row sums (over the four lane groups), normalise, store ----
 #pragma unroll
   for (int rs = 0; rs < RS; ++rs) {
+    float dsum;
+    if constexpr (DENM) {
+      dsum = dacc[rs][0];  // every element of the column is the row's sum
+    } else {
+      dsum = den[rs];
+      dsum += __shfl_xor(dsum, 16);
+      dsum += __shfl_xor(dsum, 32);
+    }
     if (!rvalid[rs]) continue;
-    put_den(myrow[rs], dsum[rs], mrow[rs]);
+    if constexpr (TAYLOR) {
+      const int64_t row = (bh * a.nsplit + split) * a.low_rows + a.low_off + myrow[rs];
+      if (lg == 0) a.low_den[row] = dsum;
 #pragma unroll
-    for (int ct = 0; ct < DVT; ++ct) put(myrow[rs], 16 * ct + 4 * lg, dsum[rs], num[rs][ct]);
+      for (int ct = 0; ct < DVT; ++ct) {
+        const int c0 = 16 * ct + 4 * lg;  // low_ld is whole 32-column groups
+        if (c0 < a.dv) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
+      }
+      continue;
+    }
+    if (a.nsplit > 1) {
+      const int64_t row = (split * a.bh + bh) * a.n + myrow[rs];
+      if (lg == 0) *reinterpret_cast<floatx2*>(a.low_den + 2 * row) = floatx2{dsum, W == FLASH_SOFTMAX ? mrow[rs] : 0.f};
+#pragma unroll
+      for (int ct = 0; ct < DVT; ++ct) {
+        const int c0 = 16 * ct + 4 * lg;
+        if (c0 < a.low_ld) *reinterpret_cast<floatx4*>(a.low_num + row * a.low_ld + c0) = num[rs][ct];
+      }
+      continue;
+    }
+    const float dn = fmaxf(dsum, a.floor);
+    const int64_t obase = (bh * a.n + myrow[rs]) * a.dv;
+#pragma unroll
+    for (int ct = 0; ct < DVT; ++ct) {
+      const int c0 = 16 * ct + 4 * lg;
+      if (c0 >= a.dv) continue;
+      floatx4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = num[rs][ct][r] / dn;
+      if (a.vec_out) {
+        *reinterpret_cast<floatx4*>(static_cast<float*>(a.out) + obase + c0) = o;
+      } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (c0 + r < a.dv) store_elem(a.out, obase + c0 + r, a.out_dtype, o[r]);
+      }
+    }
   }
 }
 
