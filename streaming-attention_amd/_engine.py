@@ -9,6 +9,7 @@ allocated here (the C ABI never allocates); plan arrays and draw tables are cach
 
 from __future__ import annotations
 
+import functools
 import os
 import threading
 from dataclasses import dataclass
@@ -121,6 +122,11 @@ def ws_query_block(semantics: str, block: int) -> Optional[int]:
 PAIRS_RATIO = 5.6
 
 
+def _padded_width(d: int, dv: int) -> int:
+    """d + dv as the pair and residual kernels run them: powers of two from 16."""
+    return max(16, 1 << (d - 1).bit_length()) + max(16, 1 << (dv - 1).bit_length())
+
+
 def use_pairs(n: int, d: int, dv: int, degree: int, block: int) -> bool:
     pad_d = max(32, 1 << (d - 1).bit_length())
     pad_dv = max(16, 1 << (dv - 1).bit_length())
@@ -136,9 +142,11 @@ def pair_splits(bh: int, n: int, compute_units: int) -> int:
     return max(1, min(2 * compute_units // tiles, n // 256, 8))
 
 
-def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, compute_units: int) -> int:
-    """Workgroups that share a tile of the residual kernel (sta_block_attention_split), width = d + dv, up to three
-    tiles for two compute units (440 tiles on 256: 74 -> 86 us and left alone), by the least estimated time in us.
+def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, compute_units: int,
+                    padded: Optional[int] = None) -> int:
+    """Workgroups that share a tile of the residual kernel (sta_block_attention_split), width = d + dv and what the
+    kernel pads it to, up to three tiles for two compute units (440 tiles on 256: 74 -> 86 us and left alone), by
+    the least estimated time in us.
     The longest tile by itself takes `alone`; shared, it falls towards the time in which all tiles fill the
     chip, but the second launch costs the host 6 us, which a pass with less than 27 us here does not win back (1 x 1024,
     d = dv = 64 bf16, 26 us: a pass 53 -> 60; 4 x 2048, 49 us: 81 -> 61), and the partials are written and read back.
@@ -148,7 +156,7 @@ def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, com
     16 x 3000 161 | 176 | 189."""
     tiles = bh * plan.n_tiles
     most = plan.longest_tile * plan.cap + min(block, plan.n)  # items and keys of the longest tile
-    alone = 2.35e-4 * most * (width + 64)
+    alone = 2.35e-4 * most * ((width if padded is None else padded) + 64)
     if 2 * tiles > 3 * compute_units or alone < 27:
         return 1
     part = bh * plan.n * width * 4 / 7e6  # a partial sum, written and read
@@ -164,6 +172,7 @@ def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, com
     return min(range(1, max(1, min(max(2 * compute_units // tiles, 2), most // 128, 8)) + 1), key=estimate)
 
 
+@functools.lru_cache(maxsize=512)
 def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, dtype: torch.dtype = torch.float32,
                  softmax: bool = True) -> int:
     """Workgroups that share a row tile of the exact kernels (sta_flash_attention_split; softmax False:
@@ -183,14 +192,17 @@ def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, dtype: to
     f32 = dtype == torch.float32
     if tiles > compute_units:
         return max(1, min(6 * compute_units // tiles, n // (1024 if f32 or not softmax else 1500)))
-    alone = n * (70 + d + dv) * 2.6e-4 + 4 if f32 else n * (135 + d + dv) * 8.5e-5 + 5 + 0.016 * (d + dv)
+    width = _padded_width(d, dv)
+    alone = n * (70 + width) * 2.6e-4 + 4 if f32 else n * (135 + width) * 8.5e-5 + 5 + 0.016 * width
     if not (f32 or softmax):  # three weight planes against one value plane, two for fp16
         alone += n * dv * (1.45e-4 if dtype == torch.float16 else 8.5e-5)
     if dv > 128:  # one workgroup a unit
         alone *= 1.5
-    part = bh * n * dv * 8 / 4.5e6  # a partial sum, written and read
-    fill = tiles / (2 * compute_units) * (0.84 if d + dv <= 160 else 1.0)
     least = 23.3 if softmax else 33.0
+    if alone <= least:
+        return 1
+    part = bh * n * dv * 8 / 4.5e6  # a partial sum, written and read
+    fill = tiles / (2 * compute_units) * (0.84 if width <= 160 else 1.0)
 
     def estimate(s: int) -> float:
         return alone if s == 1 else max(least, alone * max(fill + (1 - fill) / (s * s), 1 / s) + part * s + 8)
@@ -658,7 +670,7 @@ def prefill(
     else:
         k2_products = RESIDUAL_PRODUCTS
 
-    ksplit = 1 if raw else residual_splits(bh, plan, block, d + dv, _compute_units(dev))
+    ksplit = 1 if raw else residual_splits(bh, plan, block, d + dv, _compute_units(dev), _padded_width(d, dv))
     part_num = part_den = None
     if ksplit > 1:
         part_num = torch.empty((ksplit, bh, n, -(-dv // 4) * 4), device=dev, dtype=torch.float32)
