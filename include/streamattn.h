@@ -443,7 +443,7 @@ int sta_exact_attention_split(const void* q, const void* k, const void* v, int d
                               float* part_num, float* part_den, void* stream);
 
 /*
- * The Taylor part over pairs, for short sequences: low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i,
+ * The Taylor part over pairs: low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i,
  * c(i) = floor((i + shift) / chunk) chunk - shift, in sta_moments' partials layout with nsplit partials (a tile's
  * keys are dealt out to nsplit workgroups), for sta_block_attention with the same chunk and shift.
  * degree <= 3, 0 <= shift < chunk, low_num 16-byte aligned; the other arguments as sta_flash_attention.  fp32

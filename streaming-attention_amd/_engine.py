@@ -1,7 +1,13 @@
 """Launch sequence of the prefill path on one ROCm device:
 
-    K1 moments (sta_moments)  ->  K3 compress, one launch per tree level (sta_compress_nodes)
-                              ->  K2+K4 block attention with the normalisation (sta_block_attention)
+    K1 Taylor part: over the pairs (sta_pair_moments, where use_pairs says so), the wave-specialised moment scan
+       (sta_moments_ws_seg) or the chunked one (sta_moments)
+    K3 compress: level 0 and the merge levels (sta_compress_nodes, sta_compress_merges), or the segment means
+       (sta_segment_mean)
+    K2+K4 block attention with the normalisation (sta_block_attention_split)
+
+Where no coreset item takes part, one launch instead: exact attention over the pairs
+(sta_exact_attention_split); the exact softmax baseline is sta_flash_attention_split.
 
 All launches go to torch's current stream of the input device.  Device buffers are torch tensors
 allocated here (the C ABI never allocates); plan arrays and draw tables are cached per device.
@@ -117,7 +123,9 @@ def ws_query_block(semantics: str, block: int) -> Optional[int]:
 # measured on both sides (64 heads, d = dv = 64, degree 2, scan / pairs): fp32 4096: 564 / 427 us, 6144: 881 / 968; fp16
 # 6144: 943 / 746, 8192: 1372 / 1339; bf16 (two products a value less) 6144: 775 / 561, 8192: 1071 / 1001.  d = dv = 128
 # (32 heads), fp32 8192: 5459 / 2385, bf16 5739 / 1026; d = 16, dv = 64, degree 3, fp32 2048: 169 / 95, 4096: 317 / 342;
-# d = dv = 32, fp32 2048: 108 / 78, 4096: 186 / 266; d = dv = 16, bf16 levels, 64 x 3000: a pass 173 / 195.
+# d = dv = 32, fp32 2048: 108 / 78, 4096: 186 / 266; d = dv = 16, bf16 levels, 64 x 3000: a pass 173 / 195.  Long crossings,
+# whole passes: d = dv = 128, degree 2, 32 heads x 16384 fp32 18658 / 16077, x 21000 (the line: 21465) 25900 / 26275, 8 heads
+# 7054 / 7021, 1 head 1292 / 1178; degree 3, d = dv = 64, 8 x 32768 19684 / 6441, 1 x 111000 (112954) 14321 / 11784.
 # One line for all types, fp32's: a bf16 call then takes the route of its fp32 values, and gives their sums bit for bit.
 PAIRS_RATIO = 5.6
 
@@ -184,8 +192,8 @@ def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, dtype: to
     1000 (256 tiles, 256 units) fp32 54 | 41 | 45 | 58, bf16 30 | 32 | 35 | 44; 64 x 512, d = dv = 128 fp32 56 | 62 | 84 | 122;
     8 x 4000 fp32 196 | 114 | 103 | 112; exp 4 x 500 fp32 29 | 32 | 32 | 32; 32 x 1000 fp16 40 | 34 | 36 | 44.
     Between one and two tiles a unit, where long tiles would meet, about three workgroups a unit for tiles of
-    1024 keys each (1500 for the 16-bit softmax: 20 x 3000, d = dv = 32 bf16 57 -> 50 with 2, 32 x 2048 bf16 55 -> 57 and
-    left alone; exp 64 -> 59)."""
+    1024 keys each (8 x 8191 fp32 413 -> 351 with 3; 1500 for the 16-bit softmax: 20 x 3000, d = dv = 32 bf16 57 -> 50 with
+    2, 32 x 2048 bf16 55 -> 57 and left alone; exp 64 -> 59)."""
     tiles = bh * -(-n // _plan.TILE_ROWS)
     if tiles > 2 * compute_units:
         return 1
@@ -216,8 +224,8 @@ def flash_splits(bh: int, n: int, d: int, dv: int, compute_units: int, dtype: to
 MOMENT_WIDE = False
 
 # The same choice for the residual / combine kernel (sta_block_attention): logits and weighted value sums,
-# when coreset items take part.  Without them (compressor "none", the raw Taylor sums, or sequences no
-# longer than a block) the result is exact attention and keeps fp32 products: the reference holds those
+# when coreset items take part.  Without them (the raw Taylor sums; exact attention on keys wider than the
+# pair kernel's) it keeps fp32 products: the reference holds those
 # cases to 2e-6 / 3e-6 of softmax attention (test_fast_article_attention.py:10-29,
 # test_streaming_attention.py:10-21), which split products in this kernel exceed (about 5e-6).
 RESIDUAL_PRODUCTS = _native.PRODUCTS_SPLIT_BF16
@@ -432,7 +440,7 @@ def prefill(
         return PrefillResult(_pairs(q3, k3, v3, scale, eps, out_dtype, timer), None, None, plan,
                              _plan.num_features(d, degree), 0)
 
-    # short sequences: the Taylor part over the pairs (sta_pair_moments)
+    # the Taylor part over the pairs (sta_pair_moments) up to the length where the scan is the cheaper way
     pairs = (semantics in ("flat", "levels", "segment") and degree <= 3 and d <= FLASH_D and products is None and
              (moment_kernel == "pairs" or (moment_kernel is None and use_pairs(n, d, dv, degree, block))))
     qblock = None

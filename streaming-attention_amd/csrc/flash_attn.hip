@@ -7,10 +7,11 @@
 //                  m_i a running row maximum (online softmax)
 //   FLASH_EXP      compressor "none" (fast_article_attention.py:437-464, :596-598), where the Taylor part and the
 //                  residual add up to exp itself: out_i = sum_{j<=i} exp(s q_i.k_j) v_j / max(sum, eps)
-//   FLASH_TAYLOR   the Taylor part of a short sequence (degree <= 3; fast_article_attention.py:184-285): the partial sums
+//   FLASH_TAYLOR   the Taylor part (degree <= 3; fast_article_attention.py:184-285): the partial sums
 //                  low_num_i = sum_{j < c(i)} exp_{<=t}(s q_i.k_j) v_j and low_den_i in sta_moments' layout, c(i) the
 //                  start of the row's chunk, for sta_block_attention.  A pair costs 2 d + 2 (dv + 1) flop and a
-//                  token's moments 4 F (dv + 1), so the pairs are the cheaper way up to a few thousand tokens.
+//                  token's moments 4 F (dv + 1) for F features, so the pairs are the cheaper way up to a length that
+//                  grows with F: about 5000 tokens at d = dv = 64, degree 2, 20000 at 128, 100000 at 64, degree 3.
 //                  A tile's key batches can be dealt out to several workgroups (FlashArgs::nsplit).
 // fp32 accumulation, no N x N score matrix.
 //
@@ -28,15 +29,18 @@
 // instructions, 4.4e-7 against 5.1e-7 at 8191 keys).  2500 / 6 = 417 TF/s against their 157 TF/s.
 // 16-bit inputs are taken as they are (exact products, fp32 sums); their fp32 weights are carried as
 // 16-bit planes: hi + lo for the softmax (within 2^-16 P for bf16, 2^-20 P for fp16), three bf16 planes for
-// FLASH_EXP, whose fp16 values are two bf16 planes (exact: 11 bits).
+// FLASH_EXP, whose fp16 values are two bf16 planes (exact: 11 bits).  Rows that three planes cannot hold
+// (infinities, values above 3.396e38, values whose lower planes are subnormal) go through fp32 matrix instructions
+// after all, found by their sums: 8 x 8191 fp32 with every seventh key switched off by a dimension of finfo.min
+// 1.61 ms (0.92 ms in fp32 instructions alone), the check itself 0 to 0.7 us a call.
 //
 // What bounds it: fp32 rows the six products (two thirds of the time at d = dv = 64), 16-bit rows the VALU
-// work of a pair (exponential, maximum, planes: 6 instructions).  1 x 8 heads x 8191 fp32, d = dv = 64: 397 us
-// = 174 TF/s (fp32 matrix instructions, unbalanced tiles: 857 us); 2 x 16 x 8192 bf16: 479 us = 579 TF/s
-// (710 us with a rescale and 12 more VALU instructions a pair); FLASH_EXP 4 x 8 x 2048 fp32: 102 us (513 us as
-// moment scan + residual kernel in fp32 products);
-// with few tiles, FlashArgs::nsplit workgroups share one: 1 x 8192 fp32 397 -> 70 us, 8 x 8191 467 -> 387 us.
-// FLASH_TAYLOR 8 x 16 x 4096 bf16: 0.5 ms in the place of the moment scan's 1.06.
+// work of a pair (exponential, maximum, planes: 6 instructions).  8 heads x 8191 fp32, d = dv = 64: 413 us,
+// 351 us = 196 TF/s with three workgroups a tile (fp32 matrix instructions, unbalanced tiles: 858 us); 32 x 65536 fp32:
+// 83.4 ms = 211 TF/s, matrix cores 58 % busy; 2 x 16 x 8192 bf16: 467 us = 589 TF/s (710 us with a rescale and 12
+// more VALU instructions a pair); FLASH_EXP 4 x 8 x 2048 fp32: 102 us (515 us as moment scan + residual kernel in
+// fp32 products); with few tiles, FlashArgs::nsplit workgroups share one: 1 x 8192 fp32 394 -> 73 us, 4 x 8192 bf16
+// 180 -> 88.  FLASH_TAYLOR 8 x 16 x 4096 bf16: 0.51 ms (matrix cores 54 % busy) in the place of the moment scan's 1.1.
 #include <type_traits>
 
 #include "common.hpp"

@@ -2,8 +2,8 @@
 triton_flash_causal_attention, triton_article_attention.py:580-637) against the oracle: float64 causal
 softmax attention on the same (upcast) inputs, and the oracle's blocked online-softmax recursion.
 
-The kernel's products are exact fp32 products of the inputs and its sums fp32, so every input dtype is
-held to rel-L2 <= 2e-5 against float64 (the reference holds its tf32 Triton kernel to 2e-2,
+The kernel's products are within 2^-23 (fp32 inputs as three bf16 planes) or exact (16-bit) and its sums fp32, so every
+input dtype is held to rel-L2 <= 2e-5 against float64 (the reference holds its tf32 Triton kernel to 2e-2,
 test_triton_article_attention.py:69); 16-bit outputs to their rounding."""
 
 import pytest
