@@ -688,7 +688,13 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // 16 ct + 4 lg + r), so no exchange is needed.  Rows outside the sequence read a clamped row and are
   // never stored.  The fp32-product kernels (no register room for the in-flight pair: they would spill)
   // add every pair in the epilogue.
+  // The Taylor weight of a row is about its index, so from row 16384 on only the last batch takes a pair and the
+  // rest follow it: a residual weight of 1e-4 added to a sum of 32768 (unit in the last place 4e-3) is rounded away,
+  // every one in the same direction (65536 keys, d = 16, degree 3: 3.7e-5 of 64 bits, now 3.9e-6; d = dv = 64 by
+  // pairs, values of mean 1: 1.9e-5, now 6e-7; a pass takes 1 % longer at most).  Up to there this costs 1e-6 to 2e-6
+  // and the later order up to 3 % of a pass (1 x 8192, d = dv = 64, flat: 139.8 -> 143.3 us).
   constexpr bool PAIR_OVERLAP = SPLIT;
+  const bool early_pairs = row_lo < 16384;
   const int fs = a.fsplit;
   const int64_t pden_stride = a.low_rows, pnum_stride = a.low_rows * a.low_ld;
   const float* pden[RS];
@@ -762,7 +768,7 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
     // staged batch and list visible; whether every staged item is active on all rows of the tile
     const bool full = __syncthreads_and(item_full ? 1 : 0) != 0;
     if (nxt_have) prefetch(nxt_node, nxt_off);
-    const bool pair = PAIR_OVERLAP && pairs_done < n_pairs;
+    const bool pair = PAIR_OVERLAP && pairs_done < n_pairs && (early_pairs || !nxt_have);
     if (pair) pair_load(pairs_done);
     if (cur_node && full && fast)
       process(node_batch_full_fast{}, cur_off);

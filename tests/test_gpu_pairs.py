@@ -114,6 +114,39 @@ def test_taylor_pairs_match_the_moment_scan(bh, n, d, dv, degree, block, dtype, 
     assert rel(outs[0].out, outs[1].out.cpu().double()) < 5e-6
 
 
+def _long_pass(dtype, mean):
+    """Degree 3 over 65536 keys: the prefill by its kernels, and the last block's rows in 64 bits."""
+    n, d, dv, block = 65536, 16, 32, 256
+    g = torch.Generator().manual_seed(4)
+    q, k = (torch.nn.functional.normalize(torch.randn(1, n, d, generator=g), dim=-1).to(dtype) for _ in range(2))
+    v = (torch.randn(1, n, dv, generator=g) + mean).to(dtype)
+    run = lambda kernel, products: _engine.prefill(
+        q.to(DEV), k.to(DEV), v.to(DEV), degree=3, block=block, scale=1.0, semantics="flat", moment_kernel=kernel,
+        residual_products=products, out_dtype=torch.float32)
+    res = run("ws", _native.PRODUCTS_FP32)
+    poly = lambda x: 1 + x * (1 + x / 2 * (1 + x / 3))
+    lo, (q64, k64, v64) = n - block, (x[0].double() for x in (q, k, v))
+    x = q64[lo:] @ k64.T.contiguous()
+    w = poly(x)
+    w[:, lo:] = torch.exp(x[:, lo:]).tril_()
+    src = res.node_src[0, :lo // block].flatten().cpu().long()
+    xi = q64[lo:] @ k64[src].T.contiguous()
+    r = (torch.exp(xi) - poly(xi)) * res.node_w[0, :lo // block].flatten().cpu().double()
+    ref = (w @ v64 + r @ v64[src]) / (w.sum(-1) + r.sum(-1))[:, None]
+    return lambda kernel, products: (lambda o: (rel(o.out[0, lo:], ref), o.fsplit))(run(kernel, products))
+
+
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_residuals_beside_long_taylor_sums(dtype, mean):
+    """The residual kernel's split products drop less than 2^-16 of the residual, a few percent of the weight: with
+    either kernel's partial sums they end where the fp32 products end (within half; added to the partials one by one
+    the small weights are rounded away, all in one direction: 8 to 20 times the error)."""
+    error = _long_pass(dtype, mean)
+    for kernel in ("ws", "pairs"):
+        assert error(kernel, _native.PRODUCTS_SPLIT_BF16)[0] < 1.5 * error(kernel, _native.PRODUCTS_FP32)[0]
+
+
 def test_pair_rule_and_splits():
     assert _engine.use_pairs(1024, 32, 32, 2, 128)
     assert _engine.use_pairs(4096, 64, 64, 2, 256)
