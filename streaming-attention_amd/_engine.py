@@ -145,9 +145,12 @@ def use_pairs(n: int, d: int, dv: int, degree: int, block: int) -> bool:
 
 def pair_splits(bh: int, n: int, compute_units: int) -> int:
     """Workgroups that share a tile's keys in sta_pair_moments: two workgroups a compute unit where the tiles
-    alone are fewer, at most one per 256 keys of the longest tile and 8 (each adds a partial sum to read)."""
+    alone are fewer, at most one per 256 keys of the longest tile and 8 (each adds a partial sum to read), and
+    enough that none adds more than 21000 keys into one sum: the roundings of longer ones exceed the scan's, which
+    sums by features (65536 keys, degree 3, last rows against 64 bits, one sum / four / scan: d = dv = 64 4.8e-6 /
+    3.0e-6 / 3.4e-6, d = 16 5.1e-6 / 3.3e-6 / 3.9e-6; 1 x 65536, d = dv = 64: 4.73 -> 4.20 ms with four)."""
     tiles = bh * -(-n // _plan.TILE_ROWS)
-    return max(1, min(2 * compute_units // tiles, n // 256, 8))
+    return max(1, min(2 * compute_units // tiles, n // 256, 8), min(-(-n // 21000), 32))
 
 
 def residual_splits(bh: int, plan: "_plan.NodePlan", block: int, width: int, compute_units: int,

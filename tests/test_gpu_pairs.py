@@ -147,6 +147,17 @@ def test_residuals_beside_long_taylor_sums(dtype, mean):
         assert error(kernel, _native.PRODUCTS_SPLIT_BF16)[0] < 1.5 * error(kernel, _native.PRODUCTS_FP32)[0]
 
 
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_long_taylor_sums_over_pairs(dtype, mean):
+    """65536 keys in partial sums of at most 21000 are no further from 64 bits than the scan's sums by features (in
+    one sum they are, by a quarter and more)."""
+    error = _long_pass(dtype, mean)
+    pairs, nsplit = error("pairs", _native.PRODUCTS_FP32)
+    assert nsplit == 4
+    assert pairs <= error("ws", _native.PRODUCTS_FP32)[0]
+
+
 def test_pair_rule_and_splits():
     assert _engine.use_pairs(1024, 32, 32, 2, 128)
     assert _engine.use_pairs(4096, 64, 64, 2, 256)
