@@ -688,13 +688,15 @@ __global__ __launch_bounds__(256, block_occupancy(DP, DVT, RS)) void block_attn_
   // 16 ct + 4 lg + r), so no exchange is needed.  Rows outside the sequence read a clamped row and are
   // never stored.  The fp32-product kernels (no register room for the in-flight pair: they would spill)
   // add every pair in the epilogue.
-  // The Taylor weight of a row is about its index, so from row 16384 on only the last batch takes a pair and the
-  // rest follow it: a residual weight of 1e-4 added to a sum of 32768 (unit in the last place 4e-3) is rounded away,
-  // every one in the same direction (65536 keys, d = 16, degree 3: 3.7e-5 of 64 bits, now 3.9e-6; d = dv = 64 by
-  // pairs, values of mean 1: 1.9e-5, now 6e-7; a pass takes 1 % longer at most).  Up to there this costs 1e-6 to 2e-6
-  // and the later order up to 3 % of a pass (1 x 8192, d = dv = 64, flat: 139.8 -> 143.3 us).
+  // The Taylor weight of a row is about its index, so with a node a block, from row 16384 on, only the last batch
+  // takes a pair and the rest follow it: a residual weight of 1e-4 added to a sum of 32768 (unit in the last place
+  // 4e-3) is rounded away, every one in the same direction (65536 keys, d = 16, degree 3: 3.7e-5 of 64 bits, now
+  // 3.9e-6; d = dv = 64 by pairs, values of mean 1: 1.9e-5, now 6e-7; a pass takes about 1 % longer).  Up to there
+  // this costs 1e-6 to 2e-6 and the later order up to 3 % of a pass (1 x 8192, d = dv = 64: 139.8 -> 143.3 us).
+  // Items by level are few and weigh more the more tokens they stand for: none is lost beside the sum, and
+  // the early order stays (32 x 65536, d = dv = 64: 7.67 against 7.79 ms, the same error).
   constexpr bool PAIR_OVERLAP = SPLIT;
-  const bool early_pairs = row_lo < 16384;
+  const bool early_pairs = a.mode != MODE_FLAT || row_lo < 16384;
   const int fs = a.fsplit;
   const int64_t pden_stride = a.low_rows, pnum_stride = a.low_rows * a.low_ld;
   const float* pden[RS];
